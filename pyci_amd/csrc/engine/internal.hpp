@@ -153,6 +153,7 @@ struct pyci_ctx {
     hipStream_t stream2 = nullptr;
     pe::DevBuf<unsigned char> mf_ws2;
     std::unique_ptr<pe::DavBufs> dav[2];  // solver working memory per sector stream
+    pe::HostBuf<double> rdm_out;      // page-locked result of the full-space density matrices (at most 16 MB)
     double *noalloc_ws = nullptr;     // the fixed workspace of the allocation-free product on this device
 };
 
@@ -411,6 +412,8 @@ void fill_all_dets_device(pyci_ctx *ctx, int kind, i64 nb, i64 nup, i64 ndn, u64
 // HCI / RDMs
 i64 add_hci_device(pyci_ham *ham, pyci_wfn *wfn, const double *coeffs_host, double eps);
 void rdms_device(pyci_wfn *wfn, const double *coeffs_host, double *rdm1, double *rdm2);
+// full FullCI spaces (rdm_full.hip); false: not one that it serves
+bool rdms_full_space(pyci_wfn *wfn, const double *coeffs_host, double *rdm1, double *rdm2);
 void trdms_device(pyci_wfn *w1, pyci_wfn *w2, const double *c1_host, const double *c2_host, double *rdm1,
                   double *rdm2);
 // ENPT2 correction sum_a (sum_i H_ai c_i)^2 / (e - H_aa), e = energy - ecore (hci.hip)

@@ -1,7 +1,7 @@
 // One- and two-particle reduced density matrices on the GPU.
 //
 // Reference: compute_rdms for DOCIWfn (rdm.cpp:20-65) and FullCIWfn
-// (rdm.cpp:269-530): a loop over determinants I that visits every excitation
+// (rdm.cpp:269-530; full FullCI spaces are contracted in rdm_full.hip): a loop over determinants I that visits every excitation
 // J of I present in the wave function with J > I and scatters c_I c_J times the
 // phase into the symmetric index permutations, plus the diagonal c_I^2 terms.
 // GenCIWfn is computed from the operator algebra (every ordered pair I, J); the
@@ -497,6 +497,7 @@ void trdms_device(pyci_wfn *w1, pyci_wfn *w2, const double *c1_host, const doubl
 }
 
 void rdms_device(pyci_wfn *wfn, const double *coeffs_host, double *rdm1, double *rdm2) {
+    if (rdms_full_space(wfn, coeffs_host, rdm1, rdm2)) return;
     hipStream_t s = wfn->ctx->stream;
     const i64 n = wfn->nbasis, n2 = n * n, n4 = n2 * n2;
     i64 s1, s2;
