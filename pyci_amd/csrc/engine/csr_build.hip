@@ -8,13 +8,13 @@
 // column < ncol. Matrix elements use the reference's formulas and summation
 // order, so values are bit-identical to the serial code.
 //
-// Pass 1 counts entries per row (all stored entries, and those with col <= row
-// for the lower-triangle export) and keeps each chunk's hit ballot, an exclusive
-// scan turns counts into row pointers, pass 2 writes entries (wave-level ballot
-// compaction, probing only the hits) and the diagonal, and each row is sorted by
-// column (bitonic in LDS up to 4,096 entries, a segmented radix sort beyond).
-// The full FullCI space in colex order skips the count pass and the sort: its
-// rows are written in column order from per-string tables (SortedRows).
+// Three ways to the rows. The full FullCI space in colex order is written in column
+// order from per-string tables in one pass (SortedRows). Other sets are built by testing
+// pairs of determinants (k_pair_rows) up to a size that pairs_pay states. Beyond that, pass
+// 1 counts each row's excitations that are in the set and keeps each chunk's hit ballot, an
+// exclusive scan turns counts into row pointers, pass 2 writes entries (wave-level ballot
+// compaction, probing only the hits) and the diagonal, and each row is sorted by column
+// (bitonic in LDS up to 4,096 entries, a segmented radix sort beyond).
 #include <hipcub/hipcub.hpp>
 
 #include "internal.hpp"
@@ -58,6 +58,87 @@ struct SortedRows {
     int La, LbF, LbS;
 };
 
+// Off-diagonal element of a row's determinant (up, dn) for an excitation of class cls:
+// 0 alpha single ii -> jj, 1 alpha single and beta single kk -> ll, 2 alpha double
+// ii, kk -> jj, ll (ii < kk, jj < ll), 3 and 4 the same of beta; DOCI pair hop ii -> jj.
+template <int KIND>
+__device__ inline double row_element(const HamView &H, u64 up, u64 dn, int cls, int ii, int jj, int kk, int ll) {
+    const int n = H.n;
+    const double *one = H.one, *two = H.two;
+    if (KIND == PYCI_WFN_DOCI) return two[GIX(ii, ii, jj, jj)];  // v[k,l] = <kk|ll>
+    if (cls == 0) {
+        double v = one[ii * n + jj];
+        for (u64 x = up; x; x &= x - 1) {
+            int q = __builtin_ctzll(x);
+            v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
+        }
+        if (KIND == PYCI_WFN_FULLCI)
+            for (u64 x = dn; x; x &= x - 1) {
+                int q = __builtin_ctzll(x);
+                v += two[GIX(ii, q, jj, q)];
+            }
+        return (double)phase1(up, ii, jj) * v;
+    }
+    if (cls == 1) return (double)(phase1(up, ii, jj) * phase1(dn, kk, ll)) * two[GIX(ii, kk, jj, ll)];
+    if (cls == 2) return (double)phase2(up, ii, kk, jj, ll) * (two[GIX(ii, kk, jj, ll)] - two[GIX(ii, kk, ll, jj)]);
+    if (cls == 3) {
+        double v = one[ii * n + jj];
+        for (u64 x = up; x; x &= x - 1) {
+            int q = __builtin_ctzll(x);
+            v += two[GIX(ii, q, jj, q)];
+        }
+        for (u64 x = dn; x; x &= x - 1) {
+            int q = __builtin_ctzll(x);
+            v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
+        }
+        return (double)phase1(dn, ii, jj) * v;
+    }
+    return (double)phase2(dn, ii, kk, jj, ll) * (two[GIX(ii, kk, jj, ll)] - two[GIX(ii, kk, ll, jj)]);
+}
+
+template <int KIND>
+__device__ inline double row_diagonal(const HamView &H, u64 up, u64 dn) {
+    const int n = H.n;
+    const double *one = H.one, *two = H.two;
+    if (KIND == PYCI_WFN_DOCI) {
+        double v1 = 0.0, v2 = 0.0;
+        for (u64 x = up; x; x &= x - 1) {
+            int kk = __builtin_ctzll(x);
+            v1 += two[GIX(kk, kk, kk, kk)];
+            v2 += one[kk * (n + 1)];
+            for (u64 y = x & (x - 1); y; y &= y - 1) {
+                int ll = __builtin_ctzll(y);
+                v2 += two[GIX(kk, ll, kk, ll)] * 2 - two[GIX(kk, ll, ll, kk)];
+            }
+        }
+        return v1 + v2 * 2;
+    }
+    double v2 = 0.0;
+    for (u64 x = up; x; x &= x - 1) {
+        int ii = __builtin_ctzll(x);
+        v2 += one[(n + 1) * ii];
+        for (u64 y = x & (x - 1); y; y &= y - 1) {
+            int kk = __builtin_ctzll(y);
+            v2 += two[GIX(ii, kk, ii, kk)] - two[GIX(ii, kk, kk, ii)];
+        }
+        if (KIND == PYCI_WFN_FULLCI)
+            for (u64 y = dn; y; y &= y - 1) {
+                int kk = __builtin_ctzll(y);
+                v2 += two[GIX(ii, kk, ii, kk)];
+            }
+    }
+    if (KIND == PYCI_WFN_FULLCI)
+        for (u64 x = dn; x; x &= x - 1) {
+            int ii = __builtin_ctzll(x);
+            v2 += one[(n + 1) * ii];
+            for (u64 y = x & (x - 1); y; y &= y - 1) {
+                int kk = __builtin_ctzll(y);
+                v2 += two[GIX(ii, kk, ii, kk)] - two[GIX(ii, kk, kk, ii)];
+            }
+        }
+    return v2;
+}
+
 // Hit bitmap (bm, nchunk words per row, or null): the count pass stores each
 // chunk's ballot of candidates found in the set, and the fill pass then looks up
 // only those lanes and skips chunks without any (the candidates are enumerated in
@@ -73,7 +154,6 @@ __global__ void __launch_bounds__(256) k_rows(WfnView w, HamView H, i64 row0, i6
     const i64 row = row0 + (i64)blockIdx.x * ROWS_PER_BLOCK + (threadIdx.x >> 6);
     if (row >= row1) return;  // uniform per wavefront; no block barriers below
     const int n = H.n;
-    const double *one = H.one, *two = H.two;
     const u64 m = full_mask(n);
     const u64 up = w.dets[(i64)w.nkey * row];
     const u64 dn = (KIND == PYCI_WFN_FULLCI) ? w.dets[2 * row + 1] : 0ULL;
@@ -141,40 +221,7 @@ __global__ void __launch_bounds__(256) k_rows(WfnView w, HamView H, i64 row0, i6
                 col = wfn_lookup(w, nu, nd);
             }
             if (col >= ncol) col = -1;
-            if (FILL && col >= 0) {
-                if (KIND == PYCI_WFN_DOCI) {
-                    val = two[GIX(ii, ii, jj, jj)];  // v[k,l] = <kk|ll>
-                } else if (cls == 0) {
-                    double v = one[ii * n + jj];
-                    for (u64 x = up; x; x &= x - 1) {
-                        int q = __builtin_ctzll(x);
-                        v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                    }
-                    if (KIND == PYCI_WFN_FULLCI)
-                        for (u64 x = dn; x; x &= x - 1) {
-                            int q = __builtin_ctzll(x);
-                            v += two[GIX(ii, q, jj, q)];
-                        }
-                    val = (double)phase1(up, ii, jj) * v;
-                } else if (cls == 1) {
-                    val = (double)(phase1(up, ii, jj) * phase1(dn, kk, ll)) * two[GIX(ii, kk, jj, ll)];
-                } else if (cls == 2) {
-                    val = (double)phase2(up, ii, kk, jj, ll) * (two[GIX(ii, kk, jj, ll)] - two[GIX(ii, kk, ll, jj)]);
-                } else if (cls == 3) {
-                    double v = one[ii * n + jj];
-                    for (u64 x = up; x; x &= x - 1) {
-                        int q = __builtin_ctzll(x);
-                        v += two[GIX(ii, q, jj, q)];
-                    }
-                    for (u64 x = dn; x; x &= x - 1) {
-                        int q = __builtin_ctzll(x);
-                        v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                    }
-                    val = (double)phase1(dn, ii, jj) * v;
-                } else {
-                    val = (double)phase2(dn, ii, kk, jj, ll) * (two[GIX(ii, kk, jj, ll)] - two[GIX(ii, kk, ll, jj)]);
-                }
-            }
+            if (FILL && col >= 0) val = row_element<KIND>(H, up, dn, cls, ii, jj, kk, ll);
         }
         if constexpr (SORTED) {
             if (col >= 0) {
@@ -372,45 +419,7 @@ __global__ void __launch_bounds__(256) k_rows(WfnView w, HamView H, i64 row0, i6
     if (lane == 0) {
         const bool has_diag = row < ncol;
         if (FILL) {
-            double d;
-            if (KIND == PYCI_WFN_DOCI) {
-                double v1 = 0.0, v2 = 0.0;
-                for (u64 x = up; x; x &= x - 1) {
-                    int kk = __builtin_ctzll(x);
-                    v1 += two[GIX(kk, kk, kk, kk)];
-                    v2 += one[kk * (n + 1)];
-                    for (u64 y = x & (x - 1); y; y &= y - 1) {
-                        int ll = __builtin_ctzll(y);
-                        v2 += two[GIX(kk, ll, kk, ll)] * 2 - two[GIX(kk, ll, ll, kk)];
-                    }
-                }
-                d = v1 + v2 * 2;
-            } else {
-                double v2 = 0.0;
-                for (u64 x = up; x; x &= x - 1) {
-                    int ii = __builtin_ctzll(x);
-                    v2 += one[(n + 1) * ii];
-                    for (u64 y = x & (x - 1); y; y &= y - 1) {
-                        int kk = __builtin_ctzll(y);
-                        v2 += two[GIX(ii, kk, ii, kk)] - two[GIX(ii, kk, kk, ii)];
-                    }
-                    if (KIND == PYCI_WFN_FULLCI)
-                        for (u64 y = dn; y; y &= y - 1) {
-                            int kk = __builtin_ctzll(y);
-                            v2 += two[GIX(ii, kk, ii, kk)];
-                        }
-                }
-                if (KIND == PYCI_WFN_FULLCI)
-                    for (u64 x = dn; x; x &= x - 1) {
-                        int ii = __builtin_ctzll(x);
-                        v2 += one[(n + 1) * ii];
-                        for (u64 y = x & (x - 1); y; y &= y - 1) {
-                            int kk = __builtin_ctzll(y);
-                            v2 += two[GIX(ii, kk, ii, kk)] - two[GIX(ii, kk, kk, ii)];
-                        }
-                    }
-                d = v2;
-            }
+            const double d = row_diagonal<KIND>(H, up, dn);
             diag[row - row0] = d;
             if (has_diag) {
                 const int pos = SORTED ? T.seg[ra * T.La] + T.pf[rb * T.LbF] : written;
@@ -729,40 +738,52 @@ __global__ void k_sorted_meta(i64 row0, i64 nr, i64 rowlen, i64 nsd, SortedRows 
     }
 }
 
-// lo[0] = min, lo[1] = max over the determinants of the occupied orbitals below h
-__global__ void k_low_range(const u64 *dets, i64 nd, int nkey, int h, int *lo) {
-    int mn = 64, mx = 0;
-    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < nd; i += (i64)gridDim.x * blockDim.x) {
-        const int c = __popcll(dets[i * nkey] & full_mask(h));
+// lo[0] = min, lo[1] = max over the determinants of the occupied orbitals below h;
+// lo[2] is set where a determinant has other electron counts than nu and nd
+__global__ void k_low_range(const u64 *dets, i64 ndet, int nkey, int h, int nu, int nd, int *lo) {
+    int mn = 64, mx = 0, bad = 0;
+    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < ndet; i += (i64)gridDim.x * blockDim.x) {
+        const u64 d = dets[i * nkey];
+        const int c = __popcll(d & full_mask(h));
         mn = min(mn, c);
         mx = max(mx, c);
+        bad |= __popcll(d) != nu || (nkey == 2 && __popcll(dets[i * 2 + 1]) != nd);
     }
     for (int o = 32; o > 0; o >>= 1) {
         mn = min(mn, __shfl_xor(mn, o));
         mx = max(mx, __shfl_xor(mx, o));
+        bad |= __shfl_xor(bad, o);
     }
     if ((threadIdx.x & 63) == 0) {
         atomicMin(lo, mn);
         atomicMax(lo + 1, mx);
+        if (bad) atomicMax(lo + 2, 1);
     }
 }
 
-// GenCI: nbasis / 2 if every determinant of the set has the same number of occupied
-// spin orbitals in the lower half (a set of one Sz in the alpha-then-beta ordering),
-// else 0. An excitation that changes that number then cannot find a column.
-static int genci_split(const pyci_wfn *wfn, hipStream_t s) {
+// What the row kernels may take for granted of a set. szh: GenCI, nbasis / 2 if every
+// determinant has the same number of occupied spin orbitals in the lower half (a set of one
+// Sz in the alpha-then-beta ordering), else 0: an excitation that changes that number then
+// cannot find a column. occ: every determinant has the wave function's electron counts.
+struct SetTraits {
+    int szh;
+    bool occ;
+};
+
+static SetTraits set_traits(const pyci_wfn *wfn, hipStream_t s) {
     const int n = (int)wfn->nbasis;
-    if (wfn->kind != PYCI_WFN_GENCI || n < 2 || n % 2 != 0 || wfn->ndet < 1) return 0;
-    DevBuf<int> lo(2);
-    const int init[2] = {64, 0};
+    if (wfn->ndet < 1) return {0, true};
+    DevBuf<int> lo(3);
+    const int init[3] = {64, 0, 0};
     PE_HIP(hipMemcpyAsync(lo.p, init, sizeof(init), hipMemcpyHostToDevice, s));
-    k_low_range<<<(unsigned)std::min<i64>(1024, (wfn->ndet + 255) / 256), 256, 0, s>>>(wfn->dets.p, wfn->ndet,
-                                                                                     (int)wfn->nkey, n / 2, lo.p);
+    k_low_range<<<(unsigned)std::min<i64>(1024, (wfn->ndet + 255) / 256), 256, 0, s>>>(
+        wfn->dets.p, wfn->ndet, (int)wfn->nkey, n / 2, (int)wfn->nup, (int)wfn->ndn, lo.p);
     PE_LAUNCH_CHECK();
-    int h[2] = {0, 1};
+    int h[3] = {0, 1, 1};
     PE_HIP(hipMemcpyAsync(h, lo.p, sizeof(h), hipMemcpyDeviceToHost, s));
     PE_HIP(hipStreamSynchronize(s));
-    return h[0] == h[1] ? n / 2 : 0;
+    const bool half = wfn->kind == PYCI_WFN_GENCI && n >= 2 && n % 2 == 0 && h[0] == h[1];
+    return {half ? n / 2 : 0, h[2] == 0};
 }
 
 template <int KIND>
@@ -863,6 +884,229 @@ static bool build_rows_sorted(pyci_op *op, const pyci_wfn *wfn, const WfnView &w
     return true;
 }
 
+// ---------------------------------------------------------------------------
+// Rows of a set by testing every pair of determinants: column j belongs to row i where
+// at most two electrons differ, popcount(det_i ^ det_j) <= 4. A test is 5 (GenCI) or 9
+// (FullCI) vector instructions for 64 columns and reads the columns in order, where the
+// enumeration of k_rows hashes and probes for every excitation of the row, almost all of
+// which are outside a selected set; the columns come out sorted, so no row sort follows.
+//
+// A wave takes 8 rows (their determinants in scalar registers) and 4,096 columns at a
+// time, one column per lane: the count pass adds up the ballots; the fill pass keeps the
+// ballot of chunk c in lane c, ranks the lanes' hits by a wave scan, and lets every lane
+// pop its hits into a queue in LDS that is emptied 64 entries at a time, so that the
+// elements are evaluated with all lanes at work whatever the density of the set. Columns
+// are split over blockIdx.y where the rows alone would not fill the chip; cnt holds one
+// count per row and split, and its scan is the place of each.
+// ---------------------------------------------------------------------------
+constexpr int PAIR_ROWS = 8;
+constexpr int PAIR_COLS = 4096;
+
+template <int KIND, bool FILL>
+__global__ void __launch_bounds__(256) k_pair_rows(WfnView w, HamView H, i64 row0, i64 row1, i64 ncol, i64 seglen,
+                                                   i64 *cnt, unsigned long long *low, const double *diag,
+                                                   int32_t *cols, double *vals) {
+    constexpr int NW = KIND == PYCI_WFN_FULLCI ? 2 : 1;
+    __shared__ u64 hits[FILL ? 4 : 1][FILL ? PAIR_ROWS : 1][64];
+    __shared__ int qcol[FILL ? 4 : 1][128];
+    __shared__ unsigned qpos[FILL ? 4 : 1][128];  // row of the wave << 28 | place in the row's split
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const i64 rbase = row0 + ((i64)blockIdx.x * 4 + wave) * PAIR_ROWS;
+    if (rbase >= row1) return;  // uniform per wavefront; no block barriers below
+    const int nrows = (int)min((i64)PAIR_ROWS, row1 - rbase), nseg = (int)gridDim.y;
+    const i64 cbeg = (i64)blockIdx.y * seglen, cend = min(ncol, cbeg + seglen);
+    u64 ra[PAIR_ROWS], rb[PAIR_ROWS];
+#pragma unroll
+    for (int r = 0; r < PAIR_ROWS; ++r) {
+        const i64 row = min(rbase + r, row1 - 1);
+        ra[r] = w.dets[NW * row];
+        rb[r] = NW == 2 ? w.dets[NW * row + NW - 1] : 0ULL;
+    }
+    int total[PAIR_ROWS] = {};
+    int wr = 0, lw = 0, qn = 0;  // lane r: entries and lower entries of row r so far; queue length
+    // entry `at` of the queue: evaluate the element and write it
+    auto emit = [&](int at, bool valid) {
+        if (!valid) return;
+        const int col = qcol[wave][at];
+        const unsigned qp = qpos[wave][at];
+        const i64 row = rbase + (qp >> 28);
+        const u64 up = w.dets[NW * row], dn = NW == 2 ? w.dets[NW * row + NW - 1] : 0ULL;
+        const u64 cu = w.dets[NW * (i64)col], cd = NW == 2 ? w.dets[NW * (i64)col + NW - 1] : 0ULL;
+        const u64 hu = up & ~cu, pu = cu & ~up, hd = dn & ~cd, pd = cd & ~dn;
+        const int nu = __popcll(hu), nd = __popcll(hd);
+        double val;
+        if (nu + nd == 0) {
+            val = diag[row - row0];
+        } else {
+            // the alpha excitation's orbitals, then beta's; a double of one spin takes both of its own
+            const u64 h1 = nu ? hu : hd, p1 = nu ? pu : pd;
+            const u64 h2 = nu == 1 ? hd : h1 & (h1 - 1), p2 = nu == 1 ? pd : p1 & (p1 - 1);
+            const int cls = nu == 0 ? (nd == 1 ? 3 : 4) : nu == 2 ? 2 : nd;
+            const int ii = __builtin_ctzll(h1), jj = __builtin_ctzll(p1);
+            const int kk = h2 ? __builtin_ctzll(h2) : 0, ll = p2 ? __builtin_ctzll(p2) : 0;
+            val = row_element<KIND>(H, up, dn, cls, ii, jj, kk, ll);
+        }
+        const i64 o = cnt[(row - row0) * nseg + blockIdx.y] + (i64)(qp & 0x0fffffffu);
+        cols[o] = col;
+        vals[o] = val;
+    };
+    for (i64 base = cbeg; base < cend; base += PAIR_COLS) {
+        const int nch = (int)min((i64)(PAIR_COLS / 64), (cend - base + 63) / 64);
+        u64 mk[PAIR_ROWS] = {};
+        auto fetch = [&](int c, u64 &a, u64 &b) {
+            const i64 col = min(base + c * 64 + lane, cend - 1);
+            a = w.dets[NW * col];
+            b = NW == 2 ? w.dets[NW * col + NW - 1] : 0ULL;
+        };
+        u64 a, b, an, bn;
+        fetch(0, a, b);
+        for (int c = 0; c < nch; ++c) {
+            fetch(min(c + 1, nch - 1), an, bn);
+            const u64 valid = __ballot(base + c * 64 + lane < cend);
+#pragma unroll
+            for (int r = 0; r < PAIR_ROWS; ++r) {
+                int d = __popcll(a ^ ra[r]);
+                if (NW == 2) d += __popcll(b ^ rb[r]);
+                const u64 h = __ballot(d <= 4) & valid;
+                if (FILL)
+                    mk[r] = lane == c ? h : mk[r];
+                else
+                    total[r] += __popcll(h);
+            }
+            a = an, b = bn;
+        }
+        if constexpr (FILL) {
+#pragma unroll
+            for (int r = 0; r < PAIR_ROWS; ++r) hits[wave][r][lane] = mk[r];
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
+            for (int r = 0; r < nrows; ++r) {
+                u64 m = hits[wave][r][lane];
+                const int pc = __popcll(m);
+                int incl = pc;
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int t = __shfl_up(incl, o);
+                    if (lane >= o) incl += t;
+                }
+                const int tot = __shfl(incl, 63);
+                if (tot == 0) continue;
+                const i64 row = rbase + r;
+                if (base <= row) {  // columns <= row
+                    int lc = tot;
+                    if (base + PAIR_COLS - 1 > row) {
+                        const i64 v = row + 1 - (base + lane * 64);
+                        lc = v <= 0 ? 0 : v >= 64 ? pc : __popcll(m & ((1ULL << v) - 1ULL));
+                        for (int o = 32; o > 0; o >>= 1) lc += __shfl_xor(lc, o);
+                    }
+                    if (lane == r) lw += lc;
+                }
+                int pos = __shfl(wr, r) + incl - pc;
+                if (lane == r) wr += tot;
+                for (u64 act = __ballot(m != 0); act; act = __ballot(m != 0)) {
+                    if (m) {
+                        const int slot = qn + __popcll(act & ((1ULL << lane) - 1ULL));
+                        qcol[wave][slot] = (int)base + lane * 64 + __builtin_ctzll(m);
+                        qpos[wave][slot] = ((unsigned)r << 28) | (unsigned)pos++;
+                        m &= m - 1;
+                    }
+                    qn += __popcll(act);
+                    if (qn >= 64) {
+                        __builtin_amdgcn_wave_barrier();
+                        asm volatile("" ::: "memory");
+                        qn -= 64;
+                        emit(qn + lane, true);
+                        __builtin_amdgcn_wave_barrier();
+                        asm volatile("" ::: "memory");
+                    }
+                }
+            }
+            __builtin_amdgcn_wave_barrier();
+            asm volatile("" ::: "memory");
+        }
+    }
+    if constexpr (FILL) {
+        emit(lane, lane < qn);
+        if (lane < nrows && lw) atomicAdd(&low[rbase + lane - row0], (unsigned long long)lw);
+    } else {
+#pragma unroll
+        for (int r = 0; r < PAIR_ROWS; ++r)
+            if (lane == r && r < nrows) cnt[(rbase + r - row0) * nseg + blockIdx.y] = total[r];
+    }
+}
+
+template <int KIND>
+__global__ void k_row_diagonal(WfnView w, HamView H, i64 row0, i64 row1, double *diag) {
+    constexpr int NW = KIND == PYCI_WFN_FULLCI ? 2 : 1;
+    const i64 row = row0 + (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (row >= row1) return;
+    diag[row - row0] = row_diagonal<KIND>(H, w.dets[NW * row], NW == 2 ? w.dets[NW * row + NW - 1] : 0ULL);
+}
+
+// rowptr[i] = place of row i's first split
+__global__ void k_split_rowptr(i64 nr, int nseg, const i64 *cnt, i64 *rowptr) {
+    const i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i <= nr) rowptr[i] = cnt[i * nseg];
+}
+
+template <int KIND>
+static void build_rows_pairs(pyci_op *op, const WfnView &w, const HamView &H, i64 row0, i64 row1, i64 ncol,
+                             DevBuf<i64> &rowptr_seg, DevBuf<int32_t> &cols, DevBuf<double> &vals,
+                             DevBuf<i64> &lowcnt_seg, DevBuf<double> &diag_seg, i64 &nnz_seg, i64 &low_total) {
+    pyci_ctx *ctx = op->ctx;
+    hipStream_t s = ctx->stream;
+    const i64 nr = row1 - row0, groups = (nr + PAIR_ROWS - 1) / PAIR_ROWS;
+    // at least 4,096 waves (half of what the chip holds) where the columns allow it
+    const i64 want = std::max<i64>(1, std::min((4096 + groups - 1) / groups, (ncol + PAIR_COLS - 1) / PAIR_COLS));
+    const i64 seglen = ((ncol + want - 1) / want + PAIR_COLS - 1) / PAIR_COLS * PAIR_COLS;
+    const i64 nseg = (ncol + seglen - 1) / seglen;
+    const dim3 grid((unsigned)((groups + 3) / 4), (unsigned)nseg);
+    DevBuf<i64> cnt((size_t)(nr * nseg + 1));
+    PE_HIP(hipMemsetAsync(cnt.p + nr * nseg, 0, sizeof(i64), s));
+    PE_HIP(hipMemsetAsync(lowcnt_seg.p, 0, sizeof(i64) * (nr + 1), s));
+    k_row_diagonal<KIND><<<grid_for(nr, 64), 64, 0, s>>>(w, H, row0, row1, diag_seg.p);
+    PE_LAUNCH_CHECK();
+    k_pair_rows<KIND, false><<<grid, 256, 0, s>>>(w, H, row0, row1, ncol, seglen, cnt.p, nullptr, nullptr, nullptr,
+                                                  nullptr);
+    PE_LAUNCH_CHECK();
+    nnz_seg = exclusive_scan(ctx, cnt.p, nr * nseg + 1);
+    PE_REQUIRE(nnz_seg < (i64)1 << 40, PYCI_ENOMEM, "sparse operator too large");
+    cols.alloc((size_t)nnz_seg);
+    vals.alloc((size_t)nnz_seg);
+    k_split_rowptr<<<grid_for(nr + 1, 256), 256, 0, s>>>(nr, (int)nseg, cnt.p, rowptr_seg.p);
+    PE_LAUNCH_CHECK();
+    k_pair_rows<KIND, true><<<grid, 256, 0, s>>>(w, H, row0, row1, ncol, seglen, cnt.p,
+                                                 reinterpret_cast<unsigned long long *>(lowcnt_seg.p), diag_seg.p,
+                                                 cols.p, vals.p);
+    PE_LAUNCH_CHECK();
+    DevBuf<i64> tmp((size_t)(nr + 1));
+    PE_HIP(hipMemcpyAsync(tmp.p, lowcnt_seg.p, sizeof(i64) * (nr + 1), hipMemcpyDeviceToDevice, s));
+    low_total = exclusive_scan(ctx, tmp.p, nr + 1);
+}
+
+// Whether testing pairs is the shorter way to the rows of a hashed set: its time grows
+// with the columns (0.35 ps a pair in both passes together), that of k_rows with a row's
+// excitations (5 ps each, and its rows are sorted afterwards). Builds by excitations / by
+// pairs, ms: GenCI of 48 spin orbitals and 12 electrons (42,012 excitations) 500
+// determinants 1.25 / 0.18, 20,000 6.5 / 0.94, 60,000 20.4 / 3.0, 200,000 75 / 19.8, 500,000
+// 224 / 108, of one spin projection (16,500) 300,000 69 / 41; FullCI of 24 orbitals, 5 + 5
+// electrons (12,600) 17,317 3.5 / 0.83, 200,000 46 / 30, 400,000 107 / 106; of 14 orbitals,
+// 4 + 4 (2,220) 100,000 9.7 / 8.8: both sides meet near 30 columns per excitation. Needs
+// every determinant to have the wave function's electron counts (the test sees only which
+// orbitals differ) and a row's split to stay below 2^28 entries.
+static bool pairs_pay(int kind, const pyci_wfn *wfn, const SetTraits &t, i64 nr, i64 ncol) {
+    if (kind == PYCI_WFN_DOCI || wfn->colex || !t.occ || nr < 1 || ncol < 1 || ncol >= ((i64)1 << 28)) return false;
+    const i64 n = wfn->nbasis, nu = wfn->nup, vu = n - nu;
+    const auto c2 = [](i64 x) { return x * (x - 1) / 2; };
+    i64 exc = nu * vu + c2(nu) * c2(vu);
+    if (kind == PYCI_WFN_FULLCI) {
+        const i64 nd = wfn->ndn, vd = n - nd;
+        exc += nu * vu * nd * vd + nd * vd + c2(nd) * c2(vd);
+    } else if (t.szh) {
+        exc = exc * 2 / 5;  // k_rows leaves out what changes the projection
+    }
+    return ncol < 28 * exc;
+}
+
 void build_rows(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn, i64 row0, i64 row1, i64 ncol,
                 DevBuf<i64> &rowptr_seg, DevBuf<int32_t> &cols, DevBuf<double> &vals, DevBuf<i64> &lowcnt_seg,
                 DevBuf<double> &diag_seg, i64 &nnz_seg, i64 &low_total) {
@@ -874,10 +1118,20 @@ void build_rows(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn, i64 row0,
     if (build_rows_sorted(op, wfn, w, H, row0, row1, ncol, rowptr_seg, cols, vals, lowcnt_seg, diag_seg, nnz_seg,
                           low_total))
         return;
-    w.szh = genci_split(wfn, s);
+    const SetTraits traits = op->kind == PYCI_WFN_DOCI ? SetTraits{0, true} : set_traits(wfn, s);
+    w.szh = traits.szh;
     rowptr_seg.alloc((size_t)(nr + 1));
     lowcnt_seg.alloc((size_t)(nr + 1));
     diag_seg.alloc((size_t)(nr > 0 ? nr : 1));
+    if (pairs_pay(op->kind, wfn, traits, nr, ncol)) {
+        if (op->kind == PYCI_WFN_FULLCI)
+            build_rows_pairs<PYCI_WFN_FULLCI>(op, w, H, row0, row1, ncol, rowptr_seg, cols, vals, lowcnt_seg, diag_seg,
+                                              nnz_seg, low_total);
+        else
+            build_rows_pairs<PYCI_WFN_GENCI>(op, w, H, row0, row1, ncol, rowptr_seg, cols, vals, lowcnt_seg, diag_seg,
+                                             nnz_seg, low_total);
+        return;
+    }
     DevBuf<int> mx(1);
     PE_HIP(hipMemsetAsync(mx.p, 0, sizeof(int), s));
     PE_HIP(hipMemsetAsync(rowptr_seg.p, 0, sizeof(i64) * (nr + 1), s));
