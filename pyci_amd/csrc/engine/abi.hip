@@ -69,6 +69,7 @@ static void op_build_all(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn) 
     op->nnz = nnz;
     op->size_ref = op->symmetric ? low : nnz;
     op->segments.assign(1, {op->nrow, op->ncol});
+    spmv_plan(op, wfn->kind == PYCI_WFN_FULLCI && wfn->colex && op->ncol == wfn->ndet);
 }
 
 __global__ void k_add_offset(i64 *a, i64 n, i64 off) {
@@ -394,6 +395,7 @@ int pyci_op_update(pyci_op *op, pyci_ham *ham, pyci_wfn *wfn) {
         op->nrow = newrows;
         op->ncol = wfn->ndet;
         op->segments.push_back({newrows, wfn->ndet});
+        spmv_plan(op, false);
     });
 }
 

@@ -207,6 +207,17 @@ struct DirectOp {
 };
 }  // namespace pe
 
+namespace pe {
+// How the single-vector product goes through an operator's rows (sigma.hip).
+struct SpmvPlan {
+    bool ordered = false;  // rows of a full space, sorted in column order
+    int npanel = 0;        // X staged in LDS by column panels (0: not used)
+    int nblk = 0;
+    DevBuf<int32_t> split;  // [row][npanel - 1]: entries before each panel after the first
+    DevBuf<int> bounds;     // [nblk + 1]: first row of each block
+};
+}  // namespace pe
+
 // Learned selector (mlp.hip): FP32 master parameters + Adam state, bf16
 // operand copies of the weights, and workspaces sized for the largest batch.
 struct pyci_mlp {
@@ -246,6 +257,7 @@ struct pyci_op {
     // beta-string count when the rows are the full FullCI space in colex order with
     // nup == ndn (the alpha <-> beta exchange is then J = a nb + b -> b nb + a), else 0
     pe::i64 swap_nb = 0;
+    pe::SpmvPlan spmv;
 };
 
 namespace pe {
@@ -403,6 +415,7 @@ void sigma_f64(const pyci_op *op, int nvec, const double *X, double *Y, hipStrea
 void sigma_f32(const pyci_op *op, int nvec, const float *X, float *Y, hipStream_t s, int sector = 0,
                DevBuf<unsigned char> *ws = nullptr);
 void ensure_vals32(pyci_op *op);
+void spmv_plan(pyci_op *op, bool column_ordered_space);
 // Davidson (davidson.hip)
 void davidson_solve(pyci_op *op, i64 n, const double *c0, i64 ncv, i64 maxiter, double tol, int precision,
                     double *evals, double *evecs, pyci_solve_stats *stats);

@@ -8,11 +8,15 @@
 // streams column indices (4 B) and values (8 B FP64 or 4 B FP32) with a stride of
 // 64 entries, so every load instruction of the wavefront is fully coalesced.
 // Rows are handed to blocks in contiguous per-XCD chunks (see xcd_row_block).
+#include <algorithm>
+
 #include "internal.hpp"
 
 namespace pe {
 
 constexpr int SPMV_WAVES = 4;  // wavefronts (rows) per 256-thread block
+constexpr i64 SPMV_LDS_MIN_NNZ = (i64)1 << 20;
+constexpr i64 SPMV_LDS_MIN_SEG = 32;
 constexpr int NUM_XCD = 8;
 
 // Blocks are dispatched round-robin over the 8 XCDs (block b runs on XCD b % 8).
@@ -112,27 +116,48 @@ k_spmm(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
     }
 }
 
-// Single vector: every lane issues U column/value loads (non-temporal: the CSR is
-// streamed once per sigma and must not evict X from L2) before their U dependent
-// X gathers, so each wavefront keeps U*64 entries in flight.
-template <int U, typename VT, typename XT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 4)))
+// Single vector, a row per wave: every lane issues the column and value loads of U entries
+// (non-temporal: the CSR is streamed once per sigma and must not evict X), also in a row's
+// last chunk, then their U gathers of X. The gathers bound it: an 8-byte element costs a
+// 128-byte line from L2 unless L1 still holds it.
+//   WAVES 16, U 1   rows of a full space, sorted in column order: 16 neighbouring rows (most
+//                   with the same alpha string) walk the same lines of X in step, so L1 serves
+//                   them; a wider window per lane spreads the waves over more lines than L1
+//                   holds. nbasis 12 (18.6 GB): 4.11 ms (4.5 TB/s) against 5.18-6.4 with U
+//                   2..16 and 4 waves; nbasis 10: 160 us against 164-224.
+//   WAVES 4, U 16   other large sets: nothing to share, most loads in flight (100,000 FullCI
+//                   determinants of 24 orbitals: 527 us, 572-643 with U 2..12).
+//   WAVES 4, U 2, 4 sets below a few thousand rows, one or two chunks a row: 3,000 GenCI
+//                   determinants 4.7 us (7.4 with U 16), DOCI of 11,628 rows of 71 5.8 (7.8).
+template <int U, int WAVES, typename VT, typename XT>
+__global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, WAVES == 4 ? 4 : 8)))
 k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__restrict__ cols,
        const VT *__restrict__ vals, const XT *__restrict__ X, XT *__restrict__ Y) {
     const int lane = threadIdx.x & 63;
     const i64 blk = xcd_row_block(blockIdx.x, nblocks);
-    const i64 row = blk * SPMV_WAVES + (threadIdx.x >> 6);
+    const i64 row = blk * WAVES + (threadIdx.x >> 6);
     if (blk >= nblocks || row >= nrow) return;
-    const i64 beg = rowptr[row], end = rowptr[row + 1];
+    const i64 beg = rowptr[row], len = rowptr[row + 1] - beg;
+    cols += beg;
+    vals += beg;
     XT acc = (XT)0;
-    i64 p = beg + lane;
-    for (; p + (U - 1) * 64 < end; p += U * 64) {
+    for (i64 p0 = 0; p0 < len; p0 += U * 64) {
         int c[U];
         VT v[U];
+        if (p0 + U * 64 <= len) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            c[u] = __builtin_nontemporal_load(&cols[p + u * 64]);
-            v[u] = __builtin_nontemporal_load(&vals[p + u * 64]);
+            for (int u = 0; u < U; ++u) {
+                c[u] = __builtin_nontemporal_load(&cols[p0 + lane + u * 64]);
+                v[u] = __builtin_nontemporal_load(&vals[p0 + lane + u * 64]);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const i64 p = p0 + lane + u * 64, q = p < len ? p : len - 1;
+                c[u] = __builtin_nontemporal_load(&cols[q]);
+                const VT t = __builtin_nontemporal_load(&vals[q]);
+                v[u] = p < len ? t : (VT)0;
+            }
         }
         XT x[U];
 #pragma unroll
@@ -140,9 +165,182 @@ k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
 #pragma unroll
         for (int u = 0; u < U; ++u) acc += (XT)v[u] * x[u];
     }
-    for (; p < end; p += 64) acc += (XT)__builtin_nontemporal_load(&vals[p]) * X[__builtin_nontemporal_load(&cols[p])];
     for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o);
     if (lane == 0) Y[row] = acc;
+}
+
+// Single vector with X in LDS: one block of 16 waves per CU takes a run of rows with an equal
+// share of the entries and goes through the columns in panels of SPMV_PANEL; a panel of X is
+// staged, then 16 lanes (or a wave) multiply a row's entries of that panel, whose places come
+// from the plan, with the next row's entries loaded while the current row's gathers come out
+// of LDS. Longer rows are taken by the whole block afterwards. For sets whose columns follow
+// no order the gathers then cost LDS cycles instead of a 128-byte line of L2 each: 60,000
+// GenCI determinants (32 M entries, 3 panels) 286 -> 119 us (3.3 TB/s), 100,000 FullCI ones
+// (5 panels) 580 -> 221 us, 17,317 (one panel) 51 -> 22.5 us.
+constexpr int SPMV_PANEL = 20000;
+constexpr int SPMV_LDS_WAVES = 16;
+
+// Sum over each 16 lanes by data-parallel moves (no LDS round trips).
+template <int CTRL>
+__device__ inline double dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int CTRL>
+__device__ inline float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+template <int LANES, typename XT>
+__device__ inline XT lanes_sum(XT v) {
+    v += dpp<0x128>(v);  // row_ror:8, 4, 2, 1: every lane of the 16 ends with the sum
+    v += dpp<0x124>(v);
+    v += dpp<0x122>(v);
+    v += dpp<0x121>(v);
+    if (LANES == 64) {
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+    }
+    return v;
+}
+
+template <int LANES, typename VT, typename XT>
+__global__ void __launch_bounds__(SPMV_LDS_WAVES * 64)
+k_spmv_lds(i64 ncol, int npanel, const i64 *__restrict__ rowptr, const int32_t *__restrict__ split,
+           const int *__restrict__ bounds, i64 long_len, const int32_t *__restrict__ cols,
+           const VT *__restrict__ vals, const XT *__restrict__ X, XT *__restrict__ Y) {
+    constexpr int U = LANES == 16 ? 8 : 4, NT = SPMV_LDS_WAVES * 64, STEP = NT / LANES;
+    extern __shared__ double lds[];
+    XT *xs = reinterpret_cast<XT *>(lds);
+    __shared__ XT red[STEP];
+    __shared__ int nlong, longs[32];
+    const int sub = threadIdx.x / LANES, l = threadIdx.x % LANES;  // STEP rows at a time
+    const int r0 = bounds[blockIdx.x], r1 = bounds[blockIdx.x + 1];
+    for (int p = 0; p < npanel; ++p) {
+        const i64 pb = (i64)p * SPMV_PANEL;
+        const int width = (int)min((i64)SPMV_PANEL, ncol - pb);
+        __syncthreads();
+        if (threadIdx.x == 0) nlong = 0;
+        for (int t = threadIdx.x; t < width; t += NT) xs[t] = X[pb + t];
+        __syncthreads();
+        // entries [beg, beg + len) of a row in this panel
+        auto segment = [&](int row, i64 &beg, int &len) {
+            beg = 0, len = 0;
+            if (row >= r1) return;
+            const i64 a = rowptr[row];
+            beg = p ? a + split[(i64)row * (npanel - 1) + p - 1] : a;
+            const i64 end = p + 1 < npanel ? a + split[(i64)row * (npanel - 1) + p] : rowptr[row + 1];
+            len = (int)(end - beg);
+        };
+        auto load = [&](i64 beg, int len, int at, int (&c)[U], VT (&v)[U]) {
+            const int32_t *cp = cols + beg;
+            const VT *vp = vals + beg;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int e = at + l + u * LANES;
+                c[u] = (int)pb;
+                v[u] = (VT)0;
+                if (e < len) {
+                    c[u] = __builtin_nontemporal_load(&cp[e]);
+                    v[u] = __builtin_nontemporal_load(&vp[e]);
+                }
+            }
+        };
+        auto dot = [&](const int (&c)[U], const VT (&v)[U]) {
+            XT s = (XT)0;
+#pragma unroll
+            for (int u = 0; u < U; ++u) s += (XT)v[u] * xs[c[u] - (int)pb];
+            return s;
+        };
+        int row = r0 + sub;
+        i64 beg, nbeg;
+        int len, nlen;
+        segment(row, beg, len);
+        segment(row + STEP, nbeg, nlen);
+        XT y = (p && row < r1) ? Y[row] : (XT)0;
+        int c[U], cn[U];
+        VT v[U], vn[U];
+        load(beg, len, 0, c, v);
+        for (; row < r1; row += STEP) {
+            const int nrow = row + STEP;
+            load(nbeg, nlen, 0, cn, vn);
+            i64 b2;
+            int l2;
+            segment(nrow + STEP, b2, l2);
+            const XT yn = (p && nrow < r1) ? Y[nrow] : (XT)0;
+            if (len > long_len) {
+                if (l == 0) longs[atomicAdd(&nlong, 1)] = row;
+            } else {
+                XT s = dot(c, v);
+                for (int at = U * LANES; at < len; at += U * LANES) {
+                    int ce[U];
+                    VT ve[U];
+                    load(beg, len, at, ce, ve);
+                    s += dot(ce, ve);
+                }
+                s = lanes_sum<LANES>(s);
+                if (l == 0) Y[row] = y + s;
+            }
+            beg = nbeg, len = nlen, nbeg = b2, nlen = l2, y = yn;
+#pragma unroll
+            for (int u = 0; u < U; ++u) c[u] = cn[u], v[u] = vn[u];
+        }
+        __syncthreads();
+        for (int t = 0; t < nlong; ++t) {
+            const int lr = longs[t];
+            segment(lr, beg, len);
+            XT s = (XT)0;
+            for (int at = sub * U * LANES; at < len; at += STEP * U * LANES) {
+                load(beg, len, at, c, v);
+                s += dot(c, v);
+            }
+            s = lanes_sum<LANES>(s);
+            if (l == 0) red[sub] = s;
+            __syncthreads();
+            if (threadIdx.x == 0) {
+                XT all = p ? Y[lr] : (XT)0;
+                for (int w = 0; w < STEP; ++w) all += red[w];
+                Y[lr] = all;
+            }
+            __syncthreads();
+        }
+    }
+}
+
+// Plan of k_spmv_lds: split[row][p - 1] = entries of a row with column < p SPMV_PANEL, and
+// bounds[b] = first row of block b (rows by their first entry in equal shares of nnz).
+__global__ void k_spmv_split(i64 nrow, int npanel, const i64 *rowptr, const int32_t *cols, int32_t *split) {
+    const i64 t = (i64)blockIdx.x * 256 + threadIdx.x;
+    if (t >= nrow * (npanel - 1)) return;
+    const i64 row = t / (npanel - 1), limit = (t - row * (npanel - 1) + 1) * SPMV_PANEL;
+    const i64 beg = rowptr[row];
+    i64 lo = beg, hi = rowptr[row + 1];
+    while (lo < hi) {
+        const i64 mid = (lo + hi) >> 1;
+        if ((i64)cols[mid] < limit)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    split[t] = (int32_t)(lo - beg);
+}
+
+__global__ void k_spmv_bounds(i64 nrow, i64 nnz, int nblk, const i64 *rowptr, int *bounds) {
+    const int b = blockIdx.x * 64 + threadIdx.x;
+    if (b > nblk) return;
+    const i64 want = (i64)((__int128)nnz * b / nblk);
+    i64 lo = 0, hi = nrow;
+    while (lo < hi && b < nblk) {
+        const i64 mid = (lo + hi) >> 1;
+        if (rowptr[mid] < want)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    bounds[b] = (int)(b < nblk ? lo : nrow);
 }
 
 // Generic nvec: loops over vector chunks of 8.
@@ -183,6 +381,80 @@ __global__ void __launch_bounds__(256) k_spmm_any(i64 nrow, i64 nblocks, int nv,
     }
 }
 
+// Which single-vector product serves an operator's rows, and the plan of the one that
+// needs one. Called when the rows are final (the operator's build).
+void spmv_plan(pyci_op *op, bool column_ordered_space) {
+    SpmvPlan &P = op->spmv;
+    P = SpmvPlan();
+    P.ordered = column_ordered_space;
+    const i64 nrow = op->nrow, npanel = (op->ncol + SPMV_PANEL - 1) / SPMV_PANEL;
+    if (column_ordered_space || nrow < 1 || op->nnz < SPMV_LDS_MIN_NNZ || op->nnz / (nrow * npanel) < SPMV_LDS_MIN_SEG ||
+        nrow >= ((i64)1 << 31))
+        return;
+    hipStream_t s = op->ctx->stream;
+    int cus = 0;
+    PE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, op->ctx->device));
+    P.npanel = (int)npanel;
+    P.nblk = cus;
+    P.bounds.alloc((size_t)(cus + 1));
+    P.split.alloc((size_t)(nrow * (npanel - 1)));
+    k_spmv_bounds<<<grid_for(cus + 1, 64), 64, 0, s>>>(nrow, op->nnz, cus, op->rowptr.p, P.bounds.p);
+    PE_LAUNCH_CHECK();
+    if (npanel > 1) {
+        k_spmv_split<<<grid_for(nrow * (npanel - 1), 256), 256, 0, s>>>(nrow, (int)npanel, op->rowptr.p, op->cols.p,
+                                                                       P.split.p);
+        PE_LAUNCH_CHECK();
+    }
+}
+
+template <int LANES, typename VT, typename XT>
+static void launch_lds(const pyci_op *op, const VT *vals, const XT *X, XT *Y, hipStream_t s) {
+    const size_t lds = sizeof(XT) * SPMV_PANEL;
+    static const bool attr = [&] {
+        PE_HIP(hipFuncSetAttribute((const void *)k_spmv_lds<LANES, VT, XT>,
+                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+        return true;
+    }();
+    (void)attr;
+    const SpmvPlan &P = op->spmv;
+    // at most 25 rows of a block are longer than a 24th of its share
+    const i64 long_len = std::max<i64>(1024, op->nnz / ((i64)P.nblk * 24));
+    k_spmv_lds<LANES, VT, XT><<<(unsigned)P.nblk, SPMV_LDS_WAVES * 64, lds, s>>>(
+        op->ncol, P.npanel, op->rowptr.p, P.split.p, P.bounds.p, long_len, op->cols.p, vals, X, Y);
+    PE_LAUNCH_CHECK();
+}
+
+template <typename VT, typename XT>
+static void spmv(const pyci_op *op, const VT *vals, const XT *X, XT *Y, hipStream_t s) {
+    const i64 nrow = op->nrow, mean = op->nnz / nrow;
+    const i64 *rp = op->rowptr.p;
+    const int32_t *c = op->cols.p;
+    const SpmvPlan &P = op->spmv;
+    if (P.npanel > 0) {
+        // 16 lanes a row take 64 rows at a time with a quarter of the instructions per entry
+        // (60,000 GenCI determinants 119 us, 160 with a wave a row); with few rows a block the
+        // last of its rounds is mostly empty (17,317 FullCI determinants 31 us, 22.5)
+        if (nrow >= (i64)P.nblk * 160)
+            launch_lds<16, VT, XT>(op, vals, X, Y, s);
+        else
+            launch_lds<64, VT, XT>(op, vals, X, Y, s);
+        return;
+    }
+    auto launch = [&](auto kern, int waves) {
+        const i64 nblocks = (nrow + waves - 1) / waves, grid = ((nblocks + NUM_XCD - 1) / NUM_XCD) * NUM_XCD;
+        kern<<<(unsigned)grid, waves * 64, 0, s>>>(nrow, nblocks, rp, c, vals, X, Y);
+        PE_LAUNCH_CHECK();
+    };
+    if (P.ordered && nrow >= 32768)
+        launch(k_spmv<1, 16, VT, XT>, 16);
+    else if (mean <= 128)
+        launch(k_spmv<2, 4, VT, XT>, 4);
+    else if (op->nnz < SPMV_LDS_MIN_NNZ)
+        launch(k_spmv<4, 4, VT, XT>, 4);
+    else
+        launch(k_spmv<16, 4, VT, XT>, 4);
+}
+
 template <typename VT, typename XT>
 static void spmm(const pyci_op *op, const VT *vals, int nvec, const XT *X, XT *Y, hipStream_t s) {
     const i64 nrow = op->nrow;
@@ -192,14 +464,7 @@ static void spmm(const pyci_op *op, const VT *vals, int nvec, const XT *X, XT *Y
     const i64 *rp = op->rowptr.p;
     const int32_t *c = op->cols.p;
     switch (nvec) {
-        case 1:
-            // 16 (FP64) or 8 (FP32) entries in flight per lane: 5.7 / 4.4 ms at FullCI
-            // nbasis 12 against 6.0 / 4.7 ms with 4
-            if constexpr (sizeof(XT) == 8)
-                k_spmv<16, VT, XT><<<(unsigned)grid, 256, 0, s>>>(nrow, nblocks, rp, c, vals, X, Y);
-            else
-                k_spmv<8, VT, XT><<<(unsigned)grid, 256, 0, s>>>(nrow, nblocks, rp, c, vals, X, Y);
-            break;
+        case 1: spmv<VT, XT>(op, vals, X, Y, s); return;
         case 2:
             // two FP64 values are one 16-byte piece; two FP32 values are not
             if constexpr (sizeof(XT) == 8)

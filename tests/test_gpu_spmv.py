@@ -1,0 +1,65 @@
+"""The single-vector products of a CSR operator (a wave per row; X staged in LDS by column
+panels) against scipy's product of the exported matrix."""
+import numpy as np
+import numpy.testing as npt
+import pytest
+import scipy.sparse as sp
+
+import pyci_amd as pyci
+from pyci_amd.synthetic import seeded_integrals, spin_orbital
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(op, symmetric, seed=0):
+    data, indices, indptr = op.export()
+    a = sp.csr_matrix((data, indices, indptr), shape=op.shape)
+    if symmetric:
+        a = a + sp.tril(a, -1).T
+    x = np.random.default_rng(seed).normal(size=op.shape[1])
+    row = np.diff(a.indptr).max()
+    bound = abs(a) @ abs(x)  # a row's products are summed in some order on either side
+    npt.assert_array_less(abs(op(x) - a @ x), 2 * row * np.finfo(float).eps * bound + 1e-300)
+
+
+# one panel of 20,000 columns and its neighbours, several panels, a dense reference row
+@pytest.mark.parametrize("kind,nb,nu,nd,ndet", [("fullci", 16, 3, 3, 19999), ("fullci", 16, 3, 3, 20000),
+                                                ("fullci", 16, 3, 3, 20001), ("genci", 32, 5, 0, 60011),
+                                                ("genci", 32, 5, 0, 40000), ("fullci", 18, 3, 3, 90001)])
+def test_lds_panels(kind, nb, nu, nd, ndet):
+    _, one, two = seeded_integrals(nb if kind == "fullci" else nb // 2, 4, 60)
+    if kind == "genci":
+        one, two = spin_orbital(one, two)
+    cls = pyci.fullci_wfn if kind == "fullci" else pyci.genci_wfn
+    w = cls(nb, nu, nd)
+    for e in range(3):
+        w.add_excited_dets(e)
+    first = w.to_det_array()
+    full = cls(nb, nu, nd)
+    full.add_all_dets()
+    rest = full.to_det_array()
+    dets = np.concatenate([first, rest[np.random.default_rng(ndet).permutation(len(rest))]])
+    _, at = np.unique(dets.reshape(len(dets), -1), axis=0, return_index=True)
+    dets = dets[np.sort(at)[:ndet]]
+    op = pyci.sparse_op(pyci.hamiltonian(0.0, one, two), cls(nb, nu, nd, dets))
+    assert op.size > 1 << 19
+    _check(op, True)
+
+
+@pytest.mark.parametrize("nrow,ncol", [(20500, 30000), (30000, 20100), (3000, 30000)])
+def test_lds_panels_of_a_part(nrow, ncol):
+    _, one, two = seeded_integrals(16, 4, 61)
+    full = pyci.fullci_wfn(16, 3, 3)
+    full.add_all_dets()
+    dets = full.to_det_array()[np.random.default_rng(1).permutation(len(full))[:30000]]
+    w = pyci.fullci_wfn(16, 3, 3, dets)
+    _check(pyci.sparse_op(pyci.hamiltonian(0.0, one, two), w, nrow, ncol, symmetric=False), False)
+
+
+def test_rows_of_full_spaces():
+    """Few short rows (DOCI), few rows and many ordered rows of a full FullCI space."""
+    for cls, nb, nu, nd in ((pyci.doci_wfn, 12, 5, 5), (pyci.fullci_wfn, 6, 3, 2), (pyci.fullci_wfn, 10, 5, 4)):
+        _, one, two = seeded_integrals(nb, 4, 62)
+        w = cls(nb, nu, nd)
+        w.add_all_dets()
+        _check(pyci.sparse_op(pyci.hamiltonian(0.0, one, two), w, storage="csr"), True)
