@@ -33,35 +33,63 @@ namespace pe {
 
 constexpr u64 EMPTY_KEY = ~0ULL;
 
+// The hash set of new determinants, two words a slot in one 16-byte piece, so that a
+// candidate touches one line of a table that is far larger than L2: the key, and the first
+// position (add_hci) or the numerator sum_i H_ai c_i (ENPT2).
 struct NewSet {
-    u64 *keys;
-    u64 *pos;
+    u64 *slot;
     u64 mask;
     unsigned long long *unique;  // number of claimed slots
     int *overflow;
     u64 *score = nullptr;  // pool only: max |H_ji c_i| as double bits (nonnegative, so integer max)
     int *plain = nullptr;  // pool only: 1 when some source passes the plain threshold
-    double *num = nullptr; // ENPT2 only: sum_i H_ai c_i of external determinant a
-    u64 *kdet = nullptr;   // ENPT2 only: the determinant words of each claimed slot (2 per slot)
 };
 
+// Two strings that fit one word are the key themselves; longer ones enter by their ranks.
+__host__ __device__ inline bool strings_fit(int nb) { return nb <= 32; }
+
 __device__ inline u64 set_key(const WfnView &w, u64 a, u64 b) {
-    if (w.nkey == 2) return (u64)colex_rank(a, w.binom) * (u64)w.nsd + (u64)colex_rank(b, w.binom);
-    return a;
+    if (w.nkey == 1) return a;
+    if (strings_fit(w.nb)) return a | (b << 32);
+    return (u64)colex_rank(a, w.binom) * (u64)w.nsd + (u64)colex_rank(b, w.binom);
 }
 
-// Inserts key with position p (keeps the minimum); returns the slot, or ~0 on
-// overflow. Claimed slots are counted.
-__device__ inline u64 set_insert(const NewSet &S, u64 key, u64 p) {
+// String of colex rank r with k electrons in nb orbitals.
+__device__ inline u64 colex_unrank(i64 r, int nb, int k, const i64 *binom) {
+    u64 str = 0;
+    int p = nb;
+    for (int q = k; q >= 1; --q) {
+        int t = p - 1;
+        while (binom[t * 65 + q] > r) --t;
+        str |= 1ULL << t;
+        r -= binom[t * 65 + q];
+        p = t;
+    }
+    return str;
+}
+
+// The determinant of a key.
+__device__ inline void key_det(const WfnView &w, u64 key, u64 &a, u64 &b) {
+    a = key, b = 0ULL;
+    if (w.nkey == 1) return;
+    if (strings_fit(w.nb)) {
+        a = key & 0xffffffffULL;
+        b = key >> 32;
+    } else {
+        const i64 ra = (i64)(key / (u64)w.nsd), rb = (i64)(key - (u64)ra * (u64)w.nsd);
+        a = colex_unrank(ra, w.nb, w.nup, w.binom);
+        b = colex_unrank(rb, w.nb, w.ndn, w.binom);
+    }
+}
+
+// Finds or claims the slot of key; returns it, or ~0 on overflow. Claimed slots are counted.
+__device__ inline u64 set_insert(const NewSet &S, u64 key) {
     u64 h = mix64(key) & S.mask;
     for (u64 step = 0; step <= S.mask; ++step) {
-        unsigned long long old = atomicCAS((unsigned long long *)&S.keys[h], (unsigned long long)EMPTY_KEY,
+        unsigned long long old = atomicCAS((unsigned long long *)&S.slot[2 * h], (unsigned long long)EMPTY_KEY,
                                            (unsigned long long)key);
         if (old == EMPTY_KEY) atomicAdd(S.unique, 1ULL);
-        if (old == EMPTY_KEY || old == key) {
-            atomicMin((unsigned long long *)&S.pos[h], (unsigned long long)p);
-            return h;
-        }
+        if (old == EMPTY_KEY || old == key) return h;
         h = (h + 1) & S.mask;
     }
     atomicOr(S.overflow, 1);
@@ -70,39 +98,52 @@ __device__ inline u64 set_insert(const NewSet &S, u64 key, u64 p) {
 
 #define GIX(p, q, r, s) ((((p) * n + (q)) * n + (r)) * n + (s))
 
-// Heat-bath lists of a GenCI Hamiltonian (n <= 64 spin-orbitals). For every
-// orbital pair p < q (pair index P = q (q - 1) / 2 + p) the pairs r < s ordered by
-// |V| descending, V = two_mo[p][q][r][s] - two_mo[p][q][s][r] (the double-excitation
-// element of add_hci, hci.cpp:219-220, with the same operands, so the same bits),
-// stored with its sign; for every (i, a) an upper bound of the single-excitation
-// element: |h_ia| + sum over all q of |two_mo[i][q][a][q] - two_mo[i][q][q][a]|.
-// A row then visits, per occupied pair, only the list prefix above eps / |c_i|, and
-// computes a single's element only where the bound reaches it.
+// Heat-bath lists of a Hamiltonian (n <= 64 orbitals or spin orbitals). For every orbital
+// pair p < q (pair index P = q (q - 1) / 2 + p) the pairs r < s ordered by |V| descending,
+// V = two_mo[p][q][r][s] - two_mo[p][q][s][r] (the same-spin double of add_hci,
+// hci.cpp:219-220, with the same operands, so the same bits), stored with its sign; for
+// FullCI also, for every ordered pair (p, q), all (r, s) by |two_mo[p][q][r][s]|, the
+// element of a double of both spins; for every (i, a) an upper bound of the
+// single-excitation element: |h_ia| + sum over all q of
+// |two_mo[i][q][a][q] - two_mo[i][q][q][a]| (FullCI: + |two_mo[i][q][a][q]|). A row then
+// visits, per occupied pair, only the list prefix above eps / |c_i|, and computes a single's
+// element only where the bound reaches it, instead of evaluating every excitation.
 struct HbLists {
     const double *v = nullptr;         // [P][npair]
-    const unsigned short *rs = nullptr;  // [P][npair]: r | s << 8
+    const double *vo = nullptr;        // [p * n + q][n * n] (FullCI)
     const double *sb = nullptr;        // [i][a]
+    const unsigned short *rs = nullptr, *rso = nullptr;  // r | s << 8 of each entry
     int npair = 0;
 };
-constexpr int HB_CAP = 2048;  // n (n - 1) / 2 <= 2016 for n <= 64
+constexpr int HB_CAP = 2048;      // n (n - 1) / 2 <= 2016 for n <= 64
+constexpr int HB_CAP_OPP = 4096;  // n n
 
-__global__ void __launch_bounds__(256) k_hb_lists(HamView H, int npair, double *lv, unsigned short *lrs) {
-    __shared__ double key[HB_CAP];
-    __shared__ unsigned short idx[HB_CAP];
+template <bool OPP>
+__global__ void __launch_bounds__(256) k_hb_lists(HamView H, int count, double *lv, unsigned short *lrs) {
+    constexpr int CAP = OPP ? HB_CAP_OPP : HB_CAP;
+    __shared__ double key[CAP];
+    __shared__ unsigned short idx[CAP];
     const int n = H.n, tid = threadIdx.x;
     const double *two = H.two;
     int p, q;
-    tri_decode((int)blockIdx.x, p, q);
-    int N = 1;
-    while (N < npair) N <<= 1;
-    for (int j = tid; j < N; j += 256) {
-        if (j < npair) {
-            int r, s;
-            tri_decode(j, r, s);
-            key[j] = fabs(two[GIX(p, q, r, s)] - two[GIX(p, q, s, r)]);
-        } else {
-            key[j] = -1.0;
+    if (OPP)
+        p = blockIdx.x / n, q = blockIdx.x % n;
+    else
+        tri_decode((int)blockIdx.x, p, q);
+    auto element = [&](int j, int &r, int &s) {
+        if (OPP) {
+            r = j / n, s = j % n;
+            return two[GIX(p, q, r, s)];
         }
+        tri_decode(j, r, s);
+        return two[GIX(p, q, r, s)] - two[GIX(p, q, s, r)];
+    };
+    int N = 1;
+    while (N < count) N <<= 1;
+    for (int j = tid; j < N; j += 256) {
+        int r, s;
+        const double k = j < count ? fabs(element(j, r, s)) : -1.0;
+        key[j] = k >= 0.0 ? k : -1.0;  // a NaN passes no threshold
         idx[j] = (unsigned short)j;
     }
     __syncthreads();
@@ -119,7 +160,8 @@ __global__ void __launch_bounds__(256) k_hb_lists(HamView H, int npair, double *
                     a = blk * 2 * stride + o;
                     b = a + stride;
                 }
-                if (key[a] < key[b]) {
+                // padding (index >= count) stays behind NaNs of the same key
+                if (key[a] < key[b] || (key[a] == key[b] && idx[a] > idx[b])) {
                     const double tk = key[a];
                     key[a] = key[b];
                     key[b] = tk;
@@ -131,22 +173,24 @@ __global__ void __launch_bounds__(256) k_hb_lists(HamView H, int npair, double *
             __syncthreads();
         }
     }
-    const i64 base = (i64)blockIdx.x * npair;
-    for (int t = tid; t < npair; t += 256) {
+    const i64 base = (i64)blockIdx.x * count;
+    for (int t = tid; t < count; t += 256) {
         int r, s;
-        tri_decode(idx[t], r, s);
-        lv[base + t] = two[GIX(p, q, r, s)] - two[GIX(p, q, s, r)];
+        lv[base + t] = element(idx[t], r, s);
         lrs[base + t] = (unsigned short)(r | (s << 8));
     }
 }
 
-__global__ void k_hb_single_bound(HamView H, double *sb) {
+__global__ void k_hb_single_bound(HamView H, int opp, double *sb) {
     const int n = H.n, e = (int)(blockIdx.x * blockDim.x + threadIdx.x);
     if (e >= n * n) return;
     const double *one = H.one, *two = H.two;
     const int i = e / n, a = e - i * n;
     double b = fabs(one[i * n + a]);
-    for (int q = 0; q < n; ++q) b += fabs(two[GIX(i, q, a, q)] - two[GIX(i, q, q, a)]);
+    for (int q = 0; q < n; ++q) {
+        b += fabs(two[GIX(i, q, a, q)] - two[GIX(i, q, q, a)]);
+        if (opp) b += fabs(two[GIX(i, q, a, q)]);
+    }
     sb[e] = b;
 }
 
@@ -167,15 +211,12 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
     const double cabs = fabs(coeffs[row]);
     const double eps_i = eps / cabs, eps_plain_i = eps_plain / cabs;
     // lane q holds the q-th occupied / virtual orbital of each string
-    int tmp;
     auto nth = [](u64 x, int t) {
         for (int s = 0; s < t && x; ++s) x &= x - 1;
         return x ? __builtin_ctzll(x) : 0;
     };
     const int packed = nth(up, lane) | (nth(~up & m, lane) << 8) | (nth(dn, lane) << 16) | (nth(~dn & m, lane) << 24);
-    (void)tmp;
     u64 local = 0;                 // PASS 1 count
-    i64 e_base = 0;                // running position inside the row (reference order)
 
     // Evaluates one candidate; returns true when it passes and is new.
     auto consider = [&](bool valid, u64 nu, u64 nd, double val, u64 pos, int sg) {
@@ -192,16 +233,15 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
         } else if (PASS == 5) {
             // the reference multiplies the element by (phase * c_i) (enpt2.cpp:122-205)
             if (pass) {
-                const u64 slot = set_insert(S, key, 0);
-                if (slot != ~0ULL) {
-                    atomicAdd(&S.num[slot], val * ((double)sg * coeffs[row]));
-                    S.kdet[2 * slot] = nu;
-                    S.kdet[2 * slot + 1] = nd;
-                }
+                const u64 slot = set_insert(S, key);
+                if (slot != ~0ULL)
+                    atomicAdd(reinterpret_cast<double *>(&S.slot[2 * slot + 1]), val * ((double)sg * coeffs[row]));
             }
         } else if (PASS == 2) {
             if (pass) {
-                const u64 slot = set_insert(S, key, pos);
+                const u64 slot = set_insert(S, key);
+                if (slot != ~0ULL)
+                    atomicMin((unsigned long long *)&S.slot[2 * slot + 1], (unsigned long long)pos);
                 if (S.score != nullptr && slot != ~0ULL) {
                     atomicMax((unsigned long long *)&S.score[slot],
                               (unsigned long long)__double_as_longlong(fabs(val) * cabs));
@@ -211,61 +251,8 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
         }
     };
 
-    if constexpr (KIND == PYCI_WFN_GENCI) {
-        // Position of a candidate in the reference's row order (for i, for j: single
-        // (i, j), then doubles (k > i, l > j)): the single (i, j) at off(i, j), the
-        // double (i, j, k, l) at off(i, j) + 1 + (k - i - 1)(nv - 1 - j) + (l - j - 1).
-        const int no = nou, nv = nvu;
-        const i64 hv = (i64)nv * (nv - 1) / 2;
-        auto off = [&](int i, int j) -> i64 {
-            return (i64)i * nv + hv * ((i64)i * (no - 1) - (i64)i * (i - 1) / 2) + j +
-                   (i64)(no - 1 - i) * ((i64)j * (nv - 1) - (i64)j * (j - 1) / 2);
-        };
-        const u64 rbase = (u64)row * (u64)rows_stride;
-        // singles, where the bound reaches the threshold
-        for (int e0 = 0; e0 < no * nv; e0 += 64) {
-            const int e = e0 + lane;
-            const bool in = e < no * nv;
-            const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
-            const int ii = __shfl(packed, i) & 255, jj = (__shfl(packed, j) >> 8) & 255;
-            const bool live = in && L.sb[ii * n + jj] * (1.0 + 1e-12) > eps_i;
-            double val = 0.0;
-            int sg = 1;
-            if (live) {
-                double v = one[ii * n + jj];
-                for (u64 x = up; x; x &= x - 1) {
-                    int q = __builtin_ctzll(x);
-                    v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                }
-                val = v;
-                if (PASS == 5) sg = phase1(up, ii, jj);
-            }
-            consider(live, up ^ (1ULL << ii) ^ (1ULL << jj), 0ULL, val, rbase + (u64)off(i, j), sg);
-        }
-        // doubles: per occupied pair, the list prefix above the threshold
-        for (int po = 0; po < no * (no - 1) / 2; ++po) {
-            int i, k;
-            tri_decode(po, i, k);
-            const int ii = __shfl(packed, i) & 255, kk = __shfl(packed, k) & 255;
-            const i64 lb = (i64)(kk * (kk - 1) / 2 + ii) * L.npair;
-            for (int t0 = 0; t0 < L.npair; t0 += 64) {
-                const int t = t0 + lane;
-                const bool in = t < L.npair;
-                const double V = in ? L.v[lb + t] : 0.0;
-                const bool above = in && fabs(V) > eps_i;
-                if (__ballot(above) == 0) break;  // the list is sorted: nothing further passes
-                const unsigned rs = in ? L.rs[lb + t] : 0u;
-                const int r = (int)(rs & 255u), s2 = (int)(rs >> 8);
-                const bool free = above && !((up >> r) & 1ULL) && !((up >> s2) & 1ULL);
-                // r and s as indices among the virtual orbitals
-                const int j = r - __popcll(up & ((1ULL << r) - 1ULL)), l = s2 - __popcll(up & ((1ULL << s2) - 1ULL));
-                int sg = 1;
-                if (PASS == 5 && free) sg = phase2(up, ii, kk, r, s2);
-                const u64 pos = rbase + (u64)(off(i, j) + 1 + (i64)(k - i - 1) * (nv - 1 - j) + (l - j - 1));
-                consider(free, up ^ (1ULL << ii) ^ (1ULL << kk) ^ (1ULL << r) ^ (1ULL << s2), 0ULL, V, pos, sg);
-            }
-        }
-    } else if (KIND == PYCI_WFN_DOCI) {
+    const u64 rbase = (u64)row * (u64)rows_stride;
+    if constexpr (KIND == PYCI_WFN_DOCI) {
         const int total = nou * nvu;
         for (int e0 = 0; e0 < total; e0 += 64) {
             const int e = e0 + lane;
@@ -274,120 +261,127 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
             const int pi = __shfl(packed, i), pj = __shfl(packed, j);
             const int k = pi & 255, l = (pj >> 8) & 255;
             double val = valid ? two[GIX(k, k, l, l)] : 0.0;
-            consider(valid, up ^ (1ULL << k) ^ (1ULL << l), 0ULL, val, (u64)row * (u64)rows_stride + (u64)e, 1);
+            consider(valid, up ^ (1ULL << k) ^ (1ULL << l), 0ULL, val, rbase + (u64)e, 1);
         }
     } else {
-        // alpha (or only) string: for i, for j: single, [1-1 block], same-spin doubles k > i, l > j
-        for (int i = 0; i < nou; ++i) {
-            for (int j = 0; j < nvu; ++j) {
-                const int ii = __shfl(packed, i) & 255, jj = (__shfl(packed, j) >> 8) & 255;
-                const int nsd = (KIND == PYCI_WFN_FULLCI) ? nod * nvd : 0;
-                const int ndbl = (nou - 1 - i) * (nvu - 1 - j);
-                const int bsize = 1 + nsd + ndbl;
-                for (int t0 = 0; t0 < bsize; t0 += 64) {
-                    const int t = t0 + lane;
-                    const bool valid = t < bsize;
-                    int k = 0, l = 0, cls = 0;
-                    if (valid && t > 0) {
-                        if (t < 1 + nsd) {
-                            cls = 1;
-                            k = (t - 1) / nvd;
-                            l = (t - 1) - k * nvd;
-                        } else {
-                            cls = 2;
-                            const int u = t - 1 - nsd, w2 = nvu - 1 - j;
-                            k = i + 1 + u / w2;
-                            l = j + 1 + (u - (u / w2) * w2);
-                        }
+        // Position of a candidate in the reference's row order (alpha: for i, for j: single
+        // (i, j), FullCI the doubles with a beta single (k, l), then the doubles (k > i,
+        // l > j); beta after alpha, without the second kind): the single (i, j) at off(i, j).
+        const i64 mixed = KIND == PYCI_WFN_FULLCI ? (i64)nod * nvd : 0;
+        auto off = [](int no, int nv, i64 mid, int i, int j) -> i64 {
+            const i64 hv = (i64)nv * (nv - 1) / 2;
+            return ((i64)i * nv + j) * (1 + mid) + hv * ((i64)i * (no - 1) - (i64)i * (i - 1) / 2) +
+                   (i64)(no - 1 - i) * ((i64)j * (nv - 1) - (i64)j * (j - 1) / 2);
+        };
+        const i64 beta0 = KIND == PYCI_WFN_FULLCI ? off(nou, nvu, mixed, nou, 0) : 0;
+        // index of orbital r among the empty orbitals of string d
+        auto hole = [](u64 d, int r) { return r - __popcll(d & ((1ULL << r) - 1ULL)); };
+        // the entries of a list above the threshold, in chunks of 64 lanes
+        auto walk = [&](const double *lv, const unsigned short *lrs, int len, auto &&take) {
+            for (int t0 = 0; t0 < len; t0 += 64) {
+                const int t = t0 + lane;
+                const double V = t < len ? lv[t] : 0.0;
+                const bool above = t < len && fabs(V) > eps_i;
+                if (__ballot(above) == 0) break;  // the list is sorted: nothing further passes
+                const unsigned rs = above ? lrs[t] : 0u;
+                take(above, V, (int)(rs & 255u), (int)(rs >> 8));
+            }
+        };
+        // singles and same-spin doubles of one spin
+        auto spin = [&](bool beta) {
+            const u64 d = beta ? dn : up;
+            const int no = beta ? nod : nou, nv = beta ? nvd : nvu, so = beta ? 16 : 0;
+            const i64 mid = beta ? 0 : mixed;
+            const u64 at0 = rbase + (u64)(beta ? beta0 : 0);
+            // singles, where the bound reaches the threshold
+            for (int e0 = 0; e0 < no * nv; e0 += 64) {
+                const int e = e0 + lane;
+                const bool in = e < no * nv;
+                const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
+                const int ii = (__shfl(packed, i) >> so) & 255, jj = (__shfl(packed, j) >> (so + 8)) & 255;
+                const bool live = in && L.sb[ii * n + jj] * (1.0 + 1e-12) > eps_i;
+                double val = 0.0;
+                int sg = 1;
+                if (live) {
+                    double v = one[ii * n + jj];
+                    for (u64 x = up; x; x &= x - 1) {
+                        const int q = __builtin_ctzll(x);
+                        if (beta)
+                            v += two[GIX(ii, q, jj, q)];
+                        else
+                            v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
                     }
-                    const int pk = __shfl(packed, k), pl = __shfl(packed, l);
-                    u64 nu = up ^ (1ULL << ii) ^ (1ULL << jj), nd = dn;
-                    double val = 0.0;
-                    int sg = 1;
-                    if (valid) {
-                        if (PASS == 5) sg = phase1(up, ii, jj);
-                        if (cls == 0) {
-                            double v = one[ii * n + jj];
-                            for (u64 x = up; x; x &= x - 1) {
-                                int q = __builtin_ctzll(x);
+                    if (KIND == PYCI_WFN_FULLCI)
+                        for (u64 x = dn; x; x &= x - 1) {
+                            const int q = __builtin_ctzll(x);
+                            if (beta)
                                 v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                            }
-                            if (KIND == PYCI_WFN_FULLCI)
-                                for (u64 x = dn; x; x &= x - 1) {
-                                    int q = __builtin_ctzll(x);
-                                    v += two[GIX(ii, q, jj, q)];
-                                }
-                            val = v;
-                        } else if (cls == 1) {
-                            const int kk = (pk >> 16) & 255, ll = (pl >> 24) & 255;
-                            nd = dn ^ (1ULL << kk) ^ (1ULL << ll);
-                            val = two[GIX(ii, kk, jj, ll)];
-                            if (PASS == 5) sg *= phase1(dn, kk, ll);
-                        } else {
-                            const int kk = pk & 255, ll = (pl >> 8) & 255;
-                            nu ^= (1ULL << kk) ^ (1ULL << ll);
-                            val = two[GIX(ii, kk, jj, ll)] - two[GIX(ii, kk, ll, jj)];
-                            if (PASS == 5) sg = phase2(up, ii, kk, jj, ll);
+                            else
+                                v += two[GIX(ii, q, jj, q)];
                         }
-                    }
-                    consider(valid, nu, nd, val, (u64)row * (u64)rows_stride + (u64)(e_base + t), sg);
+                    val = v;
+                    if (PASS == 5) sg = phase1(d, ii, jj);
                 }
-                e_base += bsize;
+                const u64 x = d ^ (1ULL << ii) ^ (1ULL << jj);
+                consider(live, beta ? up : x, beta ? x : dn, val, at0 + (u64)off(no, nv, mid, i, j), sg);
             }
-        }
-        if (KIND == PYCI_WFN_FULLCI) {
-            for (int i = 0; i < nod; ++i) {
-                for (int j = 0; j < nvd; ++j) {
-                    const int ii = (__shfl(packed, i) >> 16) & 255, jj = (__shfl(packed, j) >> 24) & 255;
-                    const int ndbl = (nod - 1 - i) * (nvd - 1 - j);
-                    const int bsize = 1 + ndbl;
-                    for (int t0 = 0; t0 < bsize; t0 += 64) {
-                        const int t = t0 + lane;
-                        const bool valid = t < bsize;
-                        int k = 0, l = 0;
-                        if (valid && t > 0) {
-                            const int u = t - 1, w2 = nvd - 1 - j;
-                            k = i + 1 + u / w2;
-                            l = j + 1 + (u - (u / w2) * w2);
-                        }
-                        const int pk = __shfl(packed, k), pl = __shfl(packed, l);
-                        u64 nd = dn ^ (1ULL << ii) ^ (1ULL << jj);
-                        double val = 0.0;
+            // doubles: the occupied pairs whose list begins above the threshold, a lane each
+            const int np = no * (no - 1) / 2;
+            for (int p0 = 0; p0 < np; p0 += 64) {
+                int i = 0, k = 0;
+                if (p0 + lane < np) tri_decode(p0 + lane, i, k);
+                const int ii0 = (__shfl(packed, i) >> so) & 255, kk0 = (__shfl(packed, k) >> so) & 255;
+                const i64 lb0 = (i64)(kk0 * (kk0 - 1) / 2 + ii0) * L.npair;
+                u64 todo = __ballot(p0 + lane < np && L.npair > 0 && fabs(L.v[lb0]) > eps_i);
+                for (; todo; todo &= todo - 1) {
+                    const int from = __builtin_ctzll(todo);
+                    const int pi = __shfl(i, from), pk = __shfl(k, from);
+                    const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
+                    const i64 lb = (i64)(kk * (kk - 1) / 2 + ii) * L.npair;
+                    walk(L.v + lb, L.rs + lb, L.npair, [&](bool above, double V, int r, int s2) {
+                        const bool free = above && !((d >> r) & 1ULL) && !((d >> s2) & 1ULL);
+                        const int j = hole(d, r), l = hole(d, s2);
                         int sg = 1;
-                        if (valid) {
-                            if (PASS == 5) sg = phase1(dn, ii, jj);
-                            if (t == 0) {
-                                double v = one[ii * n + jj];
-                                for (u64 x = up; x; x &= x - 1) {
-                                    int q = __builtin_ctzll(x);
-                                    v += two[GIX(ii, q, jj, q)];
-                                }
-                                for (u64 x = dn; x; x &= x - 1) {
-                                    int q = __builtin_ctzll(x);
-                                    v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                                }
-                                val = v;
-                            } else {
-                                const int kk = (pk >> 16) & 255, ll = (pl >> 24) & 255;
-                                nd ^= (1ULL << kk) ^ (1ULL << ll);
-                                val = two[GIX(ii, kk, jj, ll)] - two[GIX(ii, kk, ll, jj)];
-                                if (PASS == 5) sg = phase2(dn, ii, kk, jj, ll);
-                            }
-                        }
-                        consider(valid, up, nd, val, (u64)row * (u64)rows_stride + (u64)(e_base + t), sg);
-                    }
-                    e_base += bsize;
+                        if (PASS == 5 && free) sg = phase2(d, ii, kk, r, s2);
+                        const i64 o = off(no, nv, mid, pi, j) + 1 + mid + (i64)(pk - pi - 1) * (nv - 1 - j) + (l - j - 1);
+                        const u64 x = d ^ (1ULL << ii) ^ (1ULL << kk) ^ (1ULL << r) ^ (1ULL << s2);
+                        consider(free, beta ? up : x, beta ? x : dn, V, at0 + (u64)o, sg);
+                    });
                 }
             }
+        };
+        spin(false);
+        if constexpr (KIND == PYCI_WFN_FULLCI) {
+            // doubles of both spins
+            for (int p0 = 0; p0 < nou * nod; p0 += 64) {
+                const int e = p0 + lane < nou * nod ? p0 + lane : 0, i = e / nod, k = e - i * nod;
+                const int ii0 = __shfl(packed, i) & 255, kk0 = (__shfl(packed, k) >> 16) & 255;
+                u64 todo = __ballot(p0 + lane < nou * nod && fabs(L.vo[(i64)(ii0 * n + kk0) * n * n]) > eps_i);
+                for (; todo; todo &= todo - 1) {
+                    const int from = __builtin_ctzll(todo);
+                    const int pi = __shfl(i, from), pk = __shfl(k, from);
+                    const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
+                    const i64 lb = (i64)(ii * n + kk) * n * n;
+                    walk(L.vo + lb, L.rso + lb, n * n, [&](bool above, double V, int r, int s2) {
+                        const bool free = above && !((up >> r) & 1ULL) && !((dn >> s2) & 1ULL);
+                        int sg = 1;
+                        if (PASS == 5 && free) sg = phase1(up, ii, r) * phase1(dn, kk, s2);
+                        const i64 o = off(nou, nvu, mixed, pi, hole(up, r)) + 1 + (i64)pk * nvd + hole(dn, s2);
+                        consider(free, up ^ (1ULL << ii) ^ (1ULL << r), dn ^ (1ULL << kk) ^ (1ULL << s2), V,
+                                 rbase + (u64)o, sg);
+                    });
+                }
+            }
+            spin(true);
         }
     }
     if (lane == 0 && PASS == 1) atomicAdd(count, (unsigned long long)local);
 }
 
-__global__ void k_set_clear(u64 *keys, u64 *pos, u64 *score, int *plain, i64 n) {
+// slots empty, with `second` in their second word
+__global__ void k_set_clear(u64 *slot, u64 second, u64 *score, int *plain, i64 n) {
     for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
-        keys[i] = EMPTY_KEY;
-        pos[i] = ~0ULL;
+        reinterpret_cast<ulonglong2 *>(slot)[i] = ulonglong2{EMPTY_KEY, second};
         if (score) {
             score[i] = 0ULL;
             plain[i] = 0;
@@ -395,24 +389,29 @@ __global__ void k_set_clear(u64 *keys, u64 *pos, u64 *score, int *plain, i64 n) 
     }
 }
 
-// The heat-bath lists of a GenCI selection (HbLists), built for one call.
+// The heat-bath lists of a selection (HbLists), built for one call.
 struct HbTables {
-    DevBuf<double> v, sb;
+    DevBuf<double> v;
     DevBuf<unsigned short> rs;
     HbLists L;
-    void build(const HamView &H, hipStream_t s) {
+    void build(const HamView &H, bool opp, hipStream_t s) {
         const int n = H.n, npair = n * (n - 1) / 2;
         PE_REQUIRE(npair <= HB_CAP, PYCI_EUNSUPPORTED, "too many orbitals for the heat-bath lists");
-        v.alloc((size_t)std::max(1, npair * npair));
-        rs.alloc((size_t)std::max(1, npair * npair));
-        sb.alloc((size_t)std::max(1, n * n));
+        const size_t np2 = (size_t)npair * npair, n2 = (size_t)n * n, n4 = opp ? n2 * n2 : 0;
+        v.alloc(np2 + n4 + n2);
+        rs.alloc(np2 + n4);
+        double *vo = v.p + np2, *sb = vo + n4;
         if (npair > 0) {
-            k_hb_lists<<<(unsigned)npair, 256, 0, s>>>(H, npair, v.p, rs.p);
+            k_hb_lists<false><<<(unsigned)npair, 256, 0, s>>>(H, npair, v.p, rs.p);
             PE_LAUNCH_CHECK();
         }
-        k_hb_single_bound<<<grid_for((i64)n * n, 256), 256, 0, s>>>(H, sb.p);
+        if (opp) {
+            k_hb_lists<true><<<(unsigned)n2, 256, 0, s>>>(H, (int)n2, vo, rs.p + np2);
+            PE_LAUNCH_CHECK();
+        }
+        k_hb_single_bound<<<grid_for((i64)n2, 256), 256, 0, s>>>(H, opp ? 1 : 0, sb);
         PE_LAUNCH_CHECK();
-        L = HbLists{v.p, rs.p, sb.p, npair};
+        L = HbLists{v.p, vo, sb, rs.p, rs.p + np2, npair};
     }
 };
 
@@ -438,46 +437,27 @@ __global__ void k_set_owners(NewSet S, i64 cap, unsigned long long *cursor, u64 
     const i64 step = (i64)gridDim.x * blockDim.x;
     for (i64 h0 = (i64)blockIdx.x * blockDim.x + (threadIdx.x & ~63); h0 < cap; h0 += step) {
         const i64 h = h0 + lane;
-        const bool claimed = h < cap && S.keys[h] != EMPTY_KEY;
+        const bool claimed = h < cap && S.slot[2 * h] != EMPTY_KEY;
         const u64 b = __ballot(claimed);
         unsigned long long base = 0;
         if (lane == 0 && b) base = atomicAdd(cursor, (unsigned long long)__popcll(b));
         base = __shfl(base, 0);
         if (claimed) {
             const unsigned long long o = base + (unsigned long long)__popcll(b & ((1ULL << lane) - 1ULL));
-            pos_out[o] = S.pos[h];
+            pos_out[o] = S.slot[2 * h + 1];
             slot_out[o] = (u64)h;
         }
     }
 }
 
-// String of colex rank r with k electrons in nb orbitals.
-__device__ inline u64 colex_unrank(i64 r, int nb, int k, const i64 *binom) {
-    u64 str = 0;
-    int p = nb;
-    for (int q = k; q >= 1; --q) {
-        int t = p - 1;
-        while (binom[t * 65 + q] > r) --t;
-        str |= 1ULL << t;
-        r -= binom[t * 65 + q];
-        p = t;
-    }
-    return str;
-}
-
-// The determinants of the sorted owner slots: a one-word key is the determinant,
-// a FullCI key is rank(alpha) * nsd + rank(beta) (set_key).
+// The determinants of the sorted owner slots.
 __global__ void k_emit_owners(WfnView w, NewSet S, const u64 *slots, i64 n, u64 *out) {
     const i64 o = (i64)blockIdx.x * blockDim.x + threadIdx.x;
     if (o >= n) return;
-    const u64 key = S.keys[slots[o]];
-    if (w.nkey == 1) {
-        out[o] = key;
-    } else {
-        const i64 ra = (i64)(key / (u64)w.nsd), rb = (i64)(key - (u64)ra * (u64)w.nsd);
-        out[2 * o] = colex_unrank(ra, w.nb, w.nup, w.binom);
-        out[2 * o + 1] = colex_unrank(rb, w.nb, w.ndn, w.binom);
-    }
+    u64 a, b;
+    key_det(w, S.slot[2 * slots[o]], a, b);
+    out[w.nkey * o] = a;
+    if (w.nkey == 2) out[2 * o + 1] = b;
 }
 
 // Passes 1-2 of the selection: the set of new candidates (|H_ji| > eps/|c_i|,
@@ -485,7 +465,7 @@ __global__ void k_emit_owners(WfnView w, NewSet S, const u64 *slots, i64 n, u64 
 // claimed slots ordered by that position (a radix sort), which is the order of
 // first occurrence in the serial enumeration: slots[0 .. nnew).
 struct HciRun {
-    DevBuf<u64> keys, pos, score, slots;
+    DevBuf<u64> table, score, slots;
     DevBuf<int> plain, ovf;
     DevBuf<unsigned long long> cnt;
     NewSet S{};
@@ -513,9 +493,9 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
     R.cnt.alloc(2);
     R.ovf.alloc(1);
     PE_HIP(hipMemsetAsync(R.cnt.p, 0, sizeof(unsigned long long) * 2, s));
-    R.S = NewSet{nullptr, nullptr, 0, R.cnt.p + 1, R.ovf.p};
+    R.S = NewSet{nullptr, 0, R.cnt.p + 1, R.ovf.p};
     HbTables hb;
-    if (wfn->kind == PYCI_WFN_GENCI) hb.build(H, s);
+    if (wfn->kind != PYCI_WFN_DOCI) hb.build(H, wfn->kind == PYCI_WFN_FULLCI, s);
     launch_hci<1>(wfn->kind, w, H, dc, eps, eps_plain, R.stride, R.S, R.cnt.p, s, hb.L);
     unsigned long long upper = 0;
     PE_HIP(hipMemcpyAsync(&upper, R.cnt.p, sizeof(upper), hipMemcpyDeviceToHost, s));
@@ -527,18 +507,17 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
     const i64 want = (i64)std::min<unsigned long long>(upper, 1ULL << 29);
     while (cap < 2 * want) cap <<= 1;
     for (;;) {
-        R.keys.alloc((size_t)cap);
-        R.pos.alloc((size_t)cap);
+        R.table.alloc((size_t)(2 * cap));
         if (pool) {
             R.score.alloc((size_t)cap);
             R.plain.alloc((size_t)cap);
         }
-        k_set_clear<<<4096, 256, 0, s>>>(R.keys.p, R.pos.p, pool ? R.score.p : nullptr, pool ? R.plain.p : nullptr,
+        k_set_clear<<<4096, 256, 0, s>>>(R.table.p, ~0ULL, pool ? R.score.p : nullptr, pool ? R.plain.p : nullptr,
                                          cap);
         PE_LAUNCH_CHECK();
         PE_HIP(hipMemsetAsync(R.cnt.p + 1, 0, sizeof(unsigned long long), s));
         PE_HIP(hipMemsetAsync(R.ovf.p, 0, sizeof(int), s));
-        R.S = NewSet{R.keys.p, R.pos.p, (u64)(cap - 1), R.cnt.p + 1, R.ovf.p};
+        R.S = NewSet{R.table.p, (u64)(cap - 1), R.cnt.p + 1, R.ovf.p};
         if (pool) {
             R.S.score = R.score.p;
             R.S.plain = R.plain.p;
@@ -658,30 +637,21 @@ void hci_pool_device(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double eps,
 
 // H_aa in the reference's order (compute_enpt2_thread_gather, enpt2.cpp:37-70;
 // GenCI :237-255): per occupied j, one_mo[j,j], same-spin pairs, then for FullCI
-// the opposite-spin pairs; then the beta string's own terms.
-__device__ inline double pt2_diag(const HamView &H, u64 up, u64 dn) {
-    const int n = H.n;
-    const double *one = H.one, *two = H.two;
+// the opposite-spin pairs; then the beta string's own terms. jk[j n + l] =
+// two[j,l,j,l] - two[j,l,l,j] and jj[j n + l] = two[j,l,j,l] are staged in LDS: every
+// external determinant reads about half its electron count squared of them.
+__device__ inline double pt2_diag(int n, const double *h, const double *jk, const double *jj, u64 up, u64 dn) {
     double d = 0.0;
     for (u64 x = up; x; x &= x - 1) {
         const int j = __builtin_ctzll(x);
-        d += one[j * (n + 1)];
-        for (u64 y = x & (x - 1); y; y &= y - 1) {
-            const int l = __builtin_ctzll(y);
-            d += two[GIX(j, l, j, l)] - two[GIX(j, l, l, j)];
-        }
-        for (u64 y = dn; y; y &= y - 1) {
-            const int l = __builtin_ctzll(y);
-            d += two[GIX(j, l, j, l)];
-        }
+        d += h[j];
+        for (u64 y = x & (x - 1); y; y &= y - 1) d += jk[j * n + __builtin_ctzll(y)];
+        for (u64 y = dn; y; y &= y - 1) d += jj[j * n + __builtin_ctzll(y)];
     }
     for (u64 x = dn; x; x &= x - 1) {
         const int j = __builtin_ctzll(x);
-        d += one[j * (n + 1)];
-        for (u64 y = x & (x - 1); y; y &= y - 1) {
-            const int l = __builtin_ctzll(y);
-            d += two[GIX(j, l, j, l)] - two[GIX(j, l, l, j)];
-        }
+        d += h[j];
+        for (u64 y = x & (x - 1); y; y &= y - 1) d += jk[j * n + __builtin_ctzll(y)];
     }
     return d;
 }
@@ -690,29 +660,36 @@ constexpr int PT2_BLOCKS = 1024;
 
 // partial[b] = block b's sum of num^2 / (e - H_aa) over its slots (grid-stride,
 // then a fixed-order tree in LDS, so the total does not depend on timing).
-__global__ void __launch_bounds__(256) k_pt2_terms(NewSet S, i64 cap, HamView H, double e, double *partial) {
+__global__ void __launch_bounds__(256) k_pt2_terms(WfnView w, NewSet S, i64 cap, HamView H, double e,
+                                                   double *partial) {
+    extern __shared__ double tab[];
     __shared__ double red[256];
+    const int n = H.n;
+    double *h = tab, *jk = h + n, *jj = jk + n * n;
+    for (int t = threadIdx.x; t < n * n; t += 256) {
+        const int j = t / n, l = t - j * n;
+        const double c = H.two[GIX(j, l, j, l)];
+        jk[t] = c - H.two[GIX(j, l, l, j)];
+        if (w.nkey == 2) jj[t] = c;
+        if (j == l) h[j] = H.one[j * (n + 1)];
+    }
+    __syncthreads();
     double acc = 0.0;
-    for (i64 h = (i64)blockIdx.x * 256 + threadIdx.x; h < cap; h += (i64)gridDim.x * 256) {
-        if (S.keys[h] == EMPTY_KEY) continue;
-        const double x = S.num[h];
-        acc += x * x / (e - pt2_diag(H, S.kdet[2 * h], S.kdet[2 * h + 1]));
+    for (i64 s = (i64)blockIdx.x * 256 + threadIdx.x; s < cap; s += (i64)gridDim.x * 256) {
+        const ulonglong2 slot = reinterpret_cast<const ulonglong2 *>(S.slot)[s];
+        if (slot.x == EMPTY_KEY) continue;
+        u64 a, b;
+        key_det(w, slot.x, a, b);
+        const double x = __longlong_as_double((long long)slot.y);
+        acc += x * x / (e - pt2_diag(n, h, jk, jj, a, b));
     }
     red[threadIdx.x] = acc;
     __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-        if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    for (int v = 128; v > 0; v >>= 1) {
+        if ((int)threadIdx.x < v) red[threadIdx.x] += red[threadIdx.x + v];
         __syncthreads();
     }
     if (threadIdx.x == 0) partial[blockIdx.x] = red[0];
-}
-
-__global__ void k_pt2_clear(double *num, u64 *kdet, i64 n) {
-    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) {
-        num[i] = 0.0;
-        kdet[2 * i] = 0ULL;
-        kdet[2 * i + 1] = 0ULL;
-    }
 }
 
 // (d) -> (d, d): the FullCI set of a DOCI set, in the same order (FullCIWfn(const
@@ -757,10 +734,10 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
     DevBuf<unsigned long long> cnt(2);
     DevBuf<int> ovf(1);
     PE_HIP(hipMemsetAsync(cnt.p, 0, sizeof(unsigned long long) * 2, s));
-    NewSet S{nullptr, nullptr, 0, cnt.p + 1, ovf.p};
+    NewSet S{nullptr, 0, cnt.p + 1, ovf.p};
     // pass 1: passing external candidates (with repeats) bound the set size
     HbTables hb;
-    if (wfn->kind == PYCI_WFN_GENCI) hb.build(H, s);
+    hb.build(H, wfn->kind == PYCI_WFN_FULLCI, s);
     launch_hci<1>(wfn->kind, w, H, dc.p, eps, eps, 0, S, cnt.p, s, hb.L);
     unsigned long long upper = 0;
     PE_HIP(hipMemcpyAsync(&upper, cnt.p, sizeof(upper), hipMemcpyDeviceToHost, s));
@@ -769,23 +746,15 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
     i64 cap = 1024;
     const i64 want = (i64)std::min<unsigned long long>(upper, 1ULL << 29);
     while (cap < 2 * want) cap <<= 1;
-    DevBuf<u64> keys, pos, kdet;
-    DevBuf<double> num;
+    DevBuf<u64> table;
     unsigned long long uniq = 0;
     for (;;) {
-        keys.alloc((size_t)cap);
-        pos.alloc((size_t)cap);
-        num.alloc((size_t)cap);
-        kdet.alloc((size_t)(2 * cap));
-        k_set_clear<<<4096, 256, 0, s>>>(keys.p, pos.p, nullptr, nullptr, cap);
-        PE_LAUNCH_CHECK();
-        k_pt2_clear<<<4096, 256, 0, s>>>(num.p, kdet.p, cap);
+        table.alloc((size_t)(2 * cap));
+        k_set_clear<<<4096, 256, 0, s>>>(table.p, 0ULL, nullptr, nullptr, cap);
         PE_LAUNCH_CHECK();
         PE_HIP(hipMemsetAsync(cnt.p + 1, 0, sizeof(unsigned long long), s));
         PE_HIP(hipMemsetAsync(ovf.p, 0, sizeof(int), s));
-        S = NewSet{keys.p, pos.p, (u64)(cap - 1), cnt.p + 1, ovf.p};
-        S.num = num.p;
-        S.kdet = kdet.p;
+        S = NewSet{table.p, (u64)(cap - 1), cnt.p + 1, ovf.p};
         launch_hci<5>(wfn->kind, w, H, dc.p, eps, eps, 0, S, nullptr, s, hb.L);
         int of = 0;
         PE_HIP(hipMemcpyAsync(&uniq, cnt.p + 1, sizeof(uniq), hipMemcpyDeviceToHost, s));
@@ -796,7 +765,10 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
         cap <<= 2;
     }
     DevBuf<double> part(PT2_BLOCKS);
-    k_pt2_terms<<<PT2_BLOCKS, 256, 0, s>>>(S, cap, H, e, part.p);
+    const size_t lds = sizeof(double) * (size_t)(H.n + H.n * H.n * (w.nkey == 2 ? 2 : 1));
+    if (lds > 60000)  // 63 and 64 orbitals of two spins: above 64 KB with the reduction's
+        PE_HIP(hipFuncSetAttribute((const void *)k_pt2_terms, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    k_pt2_terms<<<PT2_BLOCKS, 256, lds, s>>>(w, S, cap, H, e, part.p);
     PE_LAUNCH_CHECK();
     std::vector<double> hp(PT2_BLOCKS);
     PE_HIP(hipMemcpyAsync(hp.data(), part.p, sizeof(double) * PT2_BLOCKS, hipMemcpyDeviceToHost, s));
