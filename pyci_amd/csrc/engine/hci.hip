@@ -14,9 +14,9 @@
 //   pass 2 inserts each candidate's 64-bit key with the minimum position,
 //   then the claimed slots, one per new determinant, are sorted by that
 //   position (a radix sort) and written in that order.
-// One wavefront handles one source row; the outer (i, j) loops run uniformly
-// and lanes cover the inner excitation block, so ballot compaction preserves
-// the reference order.
+// One block handles one source row: its waves walk the lists of excitations above the
+// threshold (HbLists), and a candidate's position in the reference's loop order is known
+// in closed form.
 //
 // The same passes also build a candidate pool for the learned selector: the
 // insertion threshold is then a looser eps_pool, and each candidate records its
@@ -38,7 +38,7 @@ constexpr u64 EMPTY_KEY = ~0ULL;
 // position (add_hci) or the numerator sum_i H_ai c_i (ENPT2).
 struct NewSet {
     u64 *slot;
-    u64 mask;
+    u64 cap;  // slots
     unsigned long long *unique;  // number of claimed slots
     int *overflow;
     u64 *score = nullptr;  // pool only: max |H_ji c_i| as double bits (nonnegative, so integer max)
@@ -82,15 +82,15 @@ __device__ inline void key_det(const WfnView &w, u64 key, u64 &a, u64 &b) {
     }
 }
 
-// Finds or claims the slot of key; returns it, or ~0 on overflow. Claimed slots are counted.
-__device__ inline u64 set_insert(const NewSet &S, u64 key) {
-    u64 h = mix64(key) & S.mask;
-    for (u64 step = 0; step <= S.mask; ++step) {
+// Finds or claims the slot of key (counted in claims); returns it, or ~0 on overflow.
+__device__ inline u64 set_insert(const NewSet &S, u64 key, int &claims) {
+    u64 h = __umul64hi(mix64(key), S.cap);
+    for (u64 step = 0; step < S.cap; ++step) {
         unsigned long long old = atomicCAS((unsigned long long *)&S.slot[2 * h], (unsigned long long)EMPTY_KEY,
                                            (unsigned long long)key);
-        if (old == EMPTY_KEY) atomicAdd(S.unique, 1ULL);
+        if (old == EMPTY_KEY) ++claims;
         if (old == EMPTY_KEY || old == key) return h;
-        h = (h + 1) & S.mask;
+        h = h + 1 < S.cap ? h + 1 : 0;
     }
     atomicOr(S.overflow, 1);
     return ~0ULL;
@@ -112,6 +112,8 @@ struct HbLists {
     const double *v = nullptr;         // [P][npair]
     const double *vo = nullptr;        // [p * n + q][n * n] (FullCI)
     const double *sb = nullptr;        // [i][a]
+    const double *top = nullptr, *topo = nullptr;  // |V| of each list's first entry
+    const double *most = nullptr;      // the largest of sb, top and topo
     const unsigned short *rs = nullptr, *rso = nullptr;  // r | s << 8 of each entry
     int npair = 0;
 };
@@ -119,7 +121,8 @@ constexpr int HB_CAP = 2048;      // n (n - 1) / 2 <= 2016 for n <= 64
 constexpr int HB_CAP_OPP = 4096;  // n n
 
 template <bool OPP>
-__global__ void __launch_bounds__(256) k_hb_lists(HamView H, int count, double *lv, unsigned short *lrs) {
+__global__ void __launch_bounds__(256) k_hb_lists(HamView H, int count, double *lv, unsigned short *lrs,
+                                                  double *top) {
     constexpr int CAP = OPP ? HB_CAP_OPP : HB_CAP;
     __shared__ double key[CAP];
     __shared__ unsigned short idx[CAP];
@@ -173,6 +176,7 @@ __global__ void __launch_bounds__(256) k_hb_lists(HamView H, int count, double *
             __syncthreads();
         }
     }
+    if (tid == 0) top[blockIdx.x] = key[0];
     const i64 base = (i64)blockIdx.x * count;
     for (int t = tid; t < count; t += 256) {
         int r, s;
@@ -194,14 +198,37 @@ __global__ void k_hb_single_bound(HamView H, int opp, double *sb) {
     sb[e] = b;
 }
 
+// most = max of v[0 .. n) (negative entries, of lists without a number, do not count)
+__global__ void __launch_bounds__(256) k_hb_most(const double *v, int n, double *most) {
+    __shared__ double red[4];
+    double m = 0.0;
+    for (int t = threadIdx.x; t < n; t += 256) m = v[t] > m || v[t] != v[t] ? v[t] : m;
+    for (int o = 32; o > 0; o >>= 1) {
+        const double x = __shfl_xor(m, o);
+        m = x > m || x != x ? x : m;
+    }
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        for (int w = 1; w < 4; ++w) m = red[w] > m || red[w] != red[w] ? red[w] : m;
+        *most = m;
+    }
+}
+
 // PASS 1: count, 2: insert, 5: ENPT2 numerators (insert, then add the signed
-// H_ai c_i of every passing candidate).
+// H_ai c_i of every passing candidate). A block of 4 waves per row shares out the
+// row's lists: the reference determinant's row alone holds a large part of all passing
+// candidates and one wave would still walk it when the others are done. Counters leave a
+// block in one atomic (one per wave and chunk on the same address took over half of the
+// ENPT2 pass).
+constexpr int HCI_WAVES = 4;
+
 template <int KIND, int PASS>
-__global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double *coeffs, double eps, double eps_plain,
+__global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, const double *coeffs, double eps, double eps_plain,
                                              i64 rows_stride, NewSet S, unsigned long long *count, HbLists L) {
-    const int lane = threadIdx.x & 63;
-    const i64 row = (i64)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (row >= w.ndet) return;
+    __shared__ unsigned long long sums[HCI_WAVES];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const i64 row = blockIdx.x;
     const int n = H.n;
     const double *one = H.one, *two = H.two;
     const u64 m = full_mask(n);
@@ -210,13 +237,16 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
     const int nou = __popcll(up), nvu = n - nou, nod = __popcll(dn), nvd = n - nod;
     const double cabs = fabs(coeffs[row]);
     const double eps_i = eps / cabs, eps_plain_i = eps_plain / cabs;
+    // a row of the tail, whose threshold no element reaches
+    if (KIND != PYCI_WFN_DOCI && *L.most * (1.0 + 1e-12) <= eps_i) return;  // uniform per block
     // lane q holds the q-th occupied / virtual orbital of each string
     auto nth = [](u64 x, int t) {
         for (int s = 0; s < t && x; ++s) x &= x - 1;
         return x ? __builtin_ctzll(x) : 0;
     };
     const int packed = nth(up, lane) | (nth(~up & m, lane) << 8) | (nth(dn, lane) << 16) | (nth(~dn & m, lane) << 24);
-    u64 local = 0;                 // PASS 1 count
+    u64 local = 0;   // PASS 1: passing candidates of the wave
+    int claims = 0;  // slots this lane has claimed
 
     // Evaluates one candidate; returns true when it passes and is new.
     auto consider = [&](bool valid, u64 nu, u64 nd, double val, u64 pos, int sg) {
@@ -233,13 +263,13 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
         } else if (PASS == 5) {
             // the reference multiplies the element by (phase * c_i) (enpt2.cpp:122-205)
             if (pass) {
-                const u64 slot = set_insert(S, key);
+                const u64 slot = set_insert(S, key, claims);
                 if (slot != ~0ULL)
                     atomicAdd(reinterpret_cast<double *>(&S.slot[2 * slot + 1]), val * ((double)sg * coeffs[row]));
             }
         } else if (PASS == 2) {
             if (pass) {
-                const u64 slot = set_insert(S, key);
+                const u64 slot = set_insert(S, key, claims);
                 if (slot != ~0ULL)
                     atomicMin((unsigned long long *)&S.slot[2 * slot + 1], (unsigned long long)pos);
                 if (S.score != nullptr && slot != ~0ULL) {
@@ -254,7 +284,7 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
     const u64 rbase = (u64)row * (u64)rows_stride;
     if constexpr (KIND == PYCI_WFN_DOCI) {
         const int total = nou * nvu;
-        for (int e0 = 0; e0 < total; e0 += 64) {
+        for (int e0 = wave * 64; e0 < total; e0 += HCI_WAVES * 64) {
             const int e = e0 + lane;
             const bool valid = e < total;
             const int i = valid ? e / nvu : 0, j = valid ? e - (e / nvu) * nvu : 0;
@@ -276,6 +306,7 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
         const i64 beta0 = KIND == PYCI_WFN_FULLCI ? off(nou, nvu, mixed, nou, 0) : 0;
         // index of orbital r among the empty orbitals of string d
         auto hole = [](u64 d, int r) { return r - __popcll(d & ((1ULL << r) - 1ULL)); };
+        int turn = 0;  // lists seen: the waves take them in turn
         // the entries of a list above the threshold, in chunks of 64 lanes
         auto walk = [&](const double *lv, const unsigned short *lrs, int len, auto &&take) {
             for (int t0 = 0; t0 < len; t0 += 64) {
@@ -294,7 +325,7 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
             const i64 mid = beta ? 0 : mixed;
             const u64 at0 = rbase + (u64)(beta ? beta0 : 0);
             // singles, where the bound reaches the threshold
-            for (int e0 = 0; e0 < no * nv; e0 += 64) {
+            for (int e0 = wave * 64; e0 < no * nv; e0 += HCI_WAVES * 64) {
                 const int e = e0 + lane;
                 const bool in = e < no * nv;
                 const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
@@ -331,9 +362,9 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
                 int i = 0, k = 0;
                 if (p0 + lane < np) tri_decode(p0 + lane, i, k);
                 const int ii0 = (__shfl(packed, i) >> so) & 255, kk0 = (__shfl(packed, k) >> so) & 255;
-                const i64 lb0 = (i64)(kk0 * (kk0 - 1) / 2 + ii0) * L.npair;
-                u64 todo = __ballot(p0 + lane < np && L.npair > 0 && fabs(L.v[lb0]) > eps_i);
+                u64 todo = __ballot(p0 + lane < np && L.top[kk0 * (kk0 - 1) / 2 + ii0] > eps_i);
                 for (; todo; todo &= todo - 1) {
+                    if (turn++ % HCI_WAVES != wave) continue;
                     const int from = __builtin_ctzll(todo);
                     const int pi = __shfl(i, from), pk = __shfl(k, from);
                     const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
@@ -356,8 +387,9 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
             for (int p0 = 0; p0 < nou * nod; p0 += 64) {
                 const int e = p0 + lane < nou * nod ? p0 + lane : 0, i = e / nod, k = e - i * nod;
                 const int ii0 = __shfl(packed, i) & 255, kk0 = (__shfl(packed, k) >> 16) & 255;
-                u64 todo = __ballot(p0 + lane < nou * nod && fabs(L.vo[(i64)(ii0 * n + kk0) * n * n]) > eps_i);
+                u64 todo = __ballot(p0 + lane < nou * nod && L.topo[ii0 * n + kk0] > eps_i);
                 for (; todo; todo &= todo - 1) {
+                    if (turn++ % HCI_WAVES != wave) continue;
                     const int from = __builtin_ctzll(todo);
                     const int pi = __shfl(i, from), pk = __shfl(k, from);
                     const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
@@ -375,7 +407,17 @@ __global__ void __launch_bounds__(256) k_hci(WfnView w, HamView H, const double 
             spin(true);
         }
     }
-    if (lane == 0 && PASS == 1) atomicAdd(count, (unsigned long long)local);
+    if (PASS != 1) {
+        for (int o = 32; o > 0; o >>= 1) claims += __shfl_xor(claims, o);
+        local = (u64)claims;
+    }
+    if (lane == 0) sums[wave] = local;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        unsigned long long all = 0;
+        for (int v = 0; v < HCI_WAVES; ++v) all += sums[v];
+        if (all) atomicAdd(PASS == 1 ? count : S.unique, all);
+    }
 }
 
 // slots empty, with `second` in their second word
@@ -398,55 +440,79 @@ struct HbTables {
         const int n = H.n, npair = n * (n - 1) / 2;
         PE_REQUIRE(npair <= HB_CAP, PYCI_EUNSUPPORTED, "too many orbitals for the heat-bath lists");
         const size_t np2 = (size_t)npair * npair, n2 = (size_t)n * n, n4 = opp ? n2 * n2 : 0;
-        v.alloc(np2 + n4 + n2);
+        const size_t nto = opp ? n2 : 0;
+        v.alloc(np2 + n4 + n2 + npair + nto + 1);
         rs.alloc(np2 + n4);
-        double *vo = v.p + np2, *sb = vo + n4;
+        double *vo = v.p + np2, *sb = vo + n4, *top = sb + n2, *topo = top + npair, *most = topo + nto;
         if (npair > 0) {
-            k_hb_lists<false><<<(unsigned)npair, 256, 0, s>>>(H, npair, v.p, rs.p);
+            k_hb_lists<false><<<(unsigned)npair, 256, 0, s>>>(H, npair, v.p, rs.p, top);
             PE_LAUNCH_CHECK();
         }
         if (opp) {
-            k_hb_lists<true><<<(unsigned)n2, 256, 0, s>>>(H, (int)n2, vo, rs.p + np2);
+            k_hb_lists<true><<<(unsigned)n2, 256, 0, s>>>(H, (int)n2, vo, rs.p + np2, topo);
             PE_LAUNCH_CHECK();
         }
         k_hb_single_bound<<<grid_for((i64)n2, 256), 256, 0, s>>>(H, opp ? 1 : 0, sb);
         PE_LAUNCH_CHECK();
-        L = HbLists{v.p, vo, sb, rs.p, rs.p + np2, npair};
+        k_hb_most<<<1, 256, 0, s>>>(sb, (int)(n2 + npair + nto), most);
+        PE_LAUNCH_CHECK();
+        L = HbLists{v.p, vo, sb, top, topo, most, rs.p, rs.p + np2, npair};
     }
 };
 
 template <int PASS>
 static void launch_hci(int kind, const WfnView &w, const HamView &H, const double *c, double eps, double eps_plain,
                        i64 stride, const NewSet &S, unsigned long long *count, hipStream_t s, const HbLists &L) {
-    unsigned g = grid_for(w.ndet, 4);
+    const unsigned g = (unsigned)w.ndet, t = HCI_WAVES * 64;
     if (kind == PYCI_WFN_DOCI)
-        k_hci<PYCI_WFN_DOCI, PASS><<<g, 256, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+        k_hci<PYCI_WFN_DOCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     else if (kind == PYCI_WFN_FULLCI)
-        k_hci<PYCI_WFN_FULLCI, PASS><<<g, 256, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+        k_hci<PYCI_WFN_FULLCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     else
-        k_hci<PYCI_WFN_GENCI, PASS><<<g, 256, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+        k_hci<PYCI_WFN_GENCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     PE_LAUNCH_CHECK();
 }
 
 void wfn_index_append(pyci_wfn *w, i64 first);
 
-// Claimed slots of the set as (first position, slot) pairs, in no particular order:
-// one cursor increment per wave.
-__global__ void k_set_owners(NewSet S, i64 cap, unsigned long long *cursor, u64 *pos_out, u64 *slot_out) {
-    const int lane = threadIdx.x & 63;
-    const i64 step = (i64)gridDim.x * blockDim.x;
-    for (i64 h0 = (i64)blockIdx.x * blockDim.x + (threadIdx.x & ~63); h0 < cap; h0 += step) {
-        const i64 h = h0 + lane;
-        const bool claimed = h < cap && S.slot[2 * h] != EMPTY_KEY;
-        const u64 b = __ballot(claimed);
-        unsigned long long base = 0;
-        if (lane == 0 && b) base = atomicAdd(cursor, (unsigned long long)__popcll(b));
-        base = __shfl(base, 0);
-        if (claimed) {
-            const unsigned long long o = base + (unsigned long long)__popcll(b & ((1ULL << lane) - 1ULL));
-            pos_out[o] = S.slot[2 * h + 1];
-            slot_out[o] = (u64)h;
+// Claimed slots of the set as (first position, slot) pairs, in no particular order: one
+// cursor increment per block and 4,096 slots.
+constexpr int OWN_ITEMS = 16;
+
+__global__ void __launch_bounds__(256) k_set_owners(NewSet S, i64 cap, unsigned long long *cursor, u64 *pos_out,
+                                                    u64 *slot_out) {
+    __shared__ unsigned long long base;
+    __shared__ int wsum[4];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (i64 h0 = (i64)blockIdx.x * 256 * OWN_ITEMS; h0 < cap; h0 += (i64)gridDim.x * 256 * OWN_ITEMS) {
+        u64 b[OWN_ITEMS];
+        int n = 0;
+#pragma unroll
+        for (int t = 0; t < OWN_ITEMS; ++t) {
+            const i64 h = h0 + t * 256 + threadIdx.x;
+            b[t] = __ballot(h < cap && S.slot[2 * h] != EMPTY_KEY);
+            n += __popcll(b[t]);
         }
+        if (lane == 0) wsum[wave] = n;
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const int all = wsum[0] + wsum[1] + wsum[2] + wsum[3];
+            base = all ? atomicAdd(cursor, (unsigned long long)all) : 0ULL;
+        }
+        __syncthreads();
+        unsigned long long o = base;
+        for (int v = 0; v < wave; ++v) o += (unsigned long long)wsum[v];
+#pragma unroll
+        for (int t = 0; t < OWN_ITEMS; ++t) {
+            if ((b[t] >> lane) & 1ULL) {
+                const i64 h = h0 + t * 256 + threadIdx.x;
+                const unsigned long long at = o + (unsigned long long)__popcll(b[t] & ((1ULL << lane) - 1ULL));
+                pos_out[at] = S.slot[2 * h + 1];
+                slot_out[at] = (u64)h;
+            }
+            o += (unsigned long long)__popcll(b[t]);
+        }
+        __syncthreads();
     }
 }
 
@@ -458,6 +524,23 @@ __global__ void k_emit_owners(WfnView w, NewSet S, const u64 *slots, i64 n, u64 
     key_det(w, S.slot[2 * slots[o]], a, b);
     out[w.nkey * o] = a;
     if (w.nkey == 2) out[2 * o + 1] = b;
+}
+
+// Slots for up to `upper` new determinants: half as many again, a multiple of 256. (The
+// slot of a hash is its high product with the capacity, so any capacity will do; with powers
+// of two the table was three times the candidates on average, and it is cleared, probed and
+// scanned from HBM.) Grown where the cap of 2^29 candidates makes it too small.
+static i64 set_capacity(unsigned long long upper) {
+    const i64 want = (i64)std::min<unsigned long long>(upper, 1ULL << 29);
+    return std::max<i64>(1024, (want + want / 2 + 255) / 256 * 256);
+}
+
+// The table's memory: the context's, kept between calls up to 4 GB (allocating and freeing
+// it on each call took longer than filling it), else the caller's own.
+static u64 *set_table(pyci_ctx *ctx, DevBuf<u64> &own, i64 cap) {
+    DevBuf<u64> &buf = 2 * cap <= (i64)1 << 29 ? ctx->hci_table : own;
+    buf.ensure((size_t)(2 * cap));
+    return buf.p;
 }
 
 // Passes 1-2 of the selection: the set of new candidates (|H_ji| > eps/|c_i|,
@@ -502,22 +585,19 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
     PE_HIP(hipStreamSynchronize(s));
     R.nnew = 0;
     if (upper == 0) return;
-    // hash set capacity: 2x the candidate count, capped; grown on overflow
-    i64 cap = 1024;
-    const i64 want = (i64)std::min<unsigned long long>(upper, 1ULL << 29);
-    while (cap < 2 * want) cap <<= 1;
+    i64 cap = set_capacity(upper);
     for (;;) {
-        R.table.alloc((size_t)(2 * cap));
+        u64 *table = set_table(ctx, R.table, cap);
         if (pool) {
             R.score.alloc((size_t)cap);
             R.plain.alloc((size_t)cap);
         }
-        k_set_clear<<<4096, 256, 0, s>>>(R.table.p, ~0ULL, pool ? R.score.p : nullptr, pool ? R.plain.p : nullptr,
+        k_set_clear<<<4096, 256, 0, s>>>(table, ~0ULL, pool ? R.score.p : nullptr, pool ? R.plain.p : nullptr,
                                          cap);
         PE_LAUNCH_CHECK();
         PE_HIP(hipMemsetAsync(R.cnt.p + 1, 0, sizeof(unsigned long long), s));
         PE_HIP(hipMemsetAsync(R.ovf.p, 0, sizeof(int), s));
-        R.S = NewSet{R.table.p, (u64)(cap - 1), R.cnt.p + 1, R.ovf.p};
+        R.S = NewSet{table, (u64)cap, R.cnt.p + 1, R.ovf.p};
         if (pool) {
             R.S.score = R.score.p;
             R.S.plain = R.plain.p;
@@ -528,7 +608,7 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
         PE_HIP(hipMemcpyAsync(&uniq, R.cnt.p + 1, sizeof(uniq), hipMemcpyDeviceToHost, s));
         PE_HIP(hipMemcpyAsync(&of, R.ovf.p, sizeof(int), hipMemcpyDeviceToHost, s));
         PE_HIP(hipStreamSynchronize(s));
-        if (!of && 2 * (i64)uniq <= cap) {
+        if (!of && 3 * (i64)uniq <= 2 * cap) {
             R.S_unique_host = uniq;
             break;
         }
@@ -543,8 +623,8 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
     DevBuf<u64> pos_in((size_t)nnew), slot_in((size_t)nnew), pos_out((size_t)nnew);
     R.slots.alloc((size_t)nnew);
     PE_HIP(hipMemsetAsync(R.cnt.p, 0, sizeof(unsigned long long), s));
-    k_set_owners<<<(unsigned)std::min<i64>(4096, grid_for(cap, 256)), 256, 0, s>>>(R.S, cap, R.cnt.p, pos_in.p,
-                                                                                   slot_in.p);
+    k_set_owners<<<(unsigned)std::min<i64>(4096, grid_for(cap, 256 * OWN_ITEMS)), 256, 0, s>>>(R.S, cap, R.cnt.p,
+                                                                                             pos_in.p, slot_in.p);
     PE_LAUNCH_CHECK();
     // positions are below nd * stride
     int end_bit = 1;
@@ -674,15 +754,36 @@ __global__ void __launch_bounds__(256) k_pt2_terms(WfnView w, NewSet S, i64 cap,
         if (j == l) h[j] = H.one[j * (n + 1)];
     }
     __syncthreads();
+    // claimed slots of a sparse table: a wave collects 64 of them before it evaluates any
+    __shared__ ulonglong2 queue[4][128];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     double acc = 0.0;
-    for (i64 s = (i64)blockIdx.x * 256 + threadIdx.x; s < cap; s += (i64)gridDim.x * 256) {
-        const ulonglong2 slot = reinterpret_cast<const ulonglong2 *>(S.slot)[s];
-        if (slot.x == EMPTY_KEY) continue;
+    auto term = [&](int at) {
+        const ulonglong2 slot = queue[wave][at];
         u64 a, b;
         key_det(w, slot.x, a, b);
         const double x = __longlong_as_double((long long)slot.y);
         acc += x * x / (e - pt2_diag(n, h, jk, jj, a, b));
+    };
+    auto settle = [] {
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+    };
+    int qn = 0;
+    for (i64 s0 = (i64)blockIdx.x * 256 + wave * 64; s0 < cap; s0 += (i64)gridDim.x * 256) {  // cap: a multiple of 256
+        const ulonglong2 slot = reinterpret_cast<const ulonglong2 *>(S.slot)[s0 + lane];
+        const bool claimed = slot.x != EMPTY_KEY;
+        const u64 b = __ballot(claimed);
+        if (claimed) queue[wave][qn + __popcll(b & ((1ULL << lane) - 1ULL))] = slot;
+        qn += __popcll(b);
+        settle();
+        if (qn >= 64) {
+            qn -= 64;
+            term(qn + lane);
+            settle();
+        }
     }
+    if (lane < qn) term(lane);
     red[threadIdx.x] = acc;
     __syncthreads();
     for (int v = 128; v > 0; v >>= 1) {
@@ -743,24 +844,22 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
     PE_HIP(hipMemcpyAsync(&upper, cnt.p, sizeof(upper), hipMemcpyDeviceToHost, s));
     PE_HIP(hipStreamSynchronize(s));
     if (upper == 0) return 0.0;
-    i64 cap = 1024;
-    const i64 want = (i64)std::min<unsigned long long>(upper, 1ULL << 29);
-    while (cap < 2 * want) cap <<= 1;
-    DevBuf<u64> table;
+    i64 cap = set_capacity(upper);
+    DevBuf<u64> own;
     unsigned long long uniq = 0;
     for (;;) {
-        table.alloc((size_t)(2 * cap));
-        k_set_clear<<<4096, 256, 0, s>>>(table.p, 0ULL, nullptr, nullptr, cap);
+        u64 *table = set_table(ctx, own, cap);
+        k_set_clear<<<4096, 256, 0, s>>>(table, 0ULL, nullptr, nullptr, cap);
         PE_LAUNCH_CHECK();
         PE_HIP(hipMemsetAsync(cnt.p + 1, 0, sizeof(unsigned long long), s));
         PE_HIP(hipMemsetAsync(ovf.p, 0, sizeof(int), s));
-        S = NewSet{table.p, (u64)(cap - 1), cnt.p + 1, ovf.p};
+        S = NewSet{table, (u64)cap, cnt.p + 1, ovf.p};
         launch_hci<5>(wfn->kind, w, H, dc.p, eps, eps, 0, S, nullptr, s, hb.L);
         int of = 0;
         PE_HIP(hipMemcpyAsync(&uniq, cnt.p + 1, sizeof(uniq), hipMemcpyDeviceToHost, s));
         PE_HIP(hipMemcpyAsync(&of, ovf.p, sizeof(int), hipMemcpyDeviceToHost, s));
         PE_HIP(hipStreamSynchronize(s));
-        if (!of && 2 * (i64)uniq <= cap) break;
+        if (!of && 3 * (i64)uniq <= 2 * cap) break;
         PE_REQUIRE(cap < ((i64)1 << 34), PYCI_ENOMEM, "ENPT2 hash set too large");
         cap <<= 2;
     }

@@ -153,6 +153,7 @@ struct pyci_ctx {
     hipStream_t stream2 = nullptr;
     pe::DevBuf<unsigned char> mf_ws2;
     std::unique_ptr<pe::DavBufs> dav[2];  // solver working memory per sector stream
+    pe::DevBuf<pe::u64> hci_table;    // hash set of the selection and ENPT2 passes (at most 4 GB)
     pe::HostBuf<double> rdm_out;      // page-locked result of the full-space density matrices (at most 16 MB)
     double *noalloc_ws = nullptr;     // the fixed workspace of the allocation-free product on this device
 };
