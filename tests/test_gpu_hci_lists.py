@@ -1,0 +1,30 @@
+"""FullCI selection and ENPT2 through sorted integral lists against the CPU oracle, which
+evaluates every excitation: same determinants in the same order, same energy."""
+import numpy as np
+import numpy.testing as npt
+import pytest
+
+import pyci_amd as pyci
+
+pytestmark = pytest.mark.gpu
+
+
+# no electrons or no holes of a spin, no same-spin pairs, the longest strings that are
+# their own key and the first that are ranked, a list of 2,048 and the longest lists
+@pytest.mark.parametrize("nb,nu,nd", [(7, 3, 0), (6, 6, 3), (20, 1, 1), (32, 2, 2), (33, 2, 1), (46, 2, 1), (64, 1, 1)])
+def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
+    rng = np.random.default_rng(nb)
+    one = rng.normal(size=(nb, nb))
+    two = rng.normal(size=(nb,) * 4) * 10.0 ** rng.uniform(-4, 0, size=(nb,) * 4)  # no symmetry assumed
+    strings = [[sum(1 << int(p) for p in rng.permutation(nb)[:k]) for _ in range(25)] for k in (nu, nd)]
+    dets = np.unique(np.array(strings, dtype=np.uint64).T, axis=0)
+    c = rng.normal(size=len(dets)) * 10.0 ** rng.uniform(-3, 0, size=len(dets))
+    ham = pyci.hamiltonian(0.0, one, two)
+    for eps in (0.0, 3e-3, 0.3, 1e9):
+        w = pyci.fullci_wfn(nb, nu, nd, dets.reshape(-1, 2, 1))
+        expect = oracle.add_hci("fullci", nb, nu, nd, dets, one, two, c, eps).reshape(-1, 2)
+        e = pyci.compute_enpt2(ham, w, c, -1e3, eps=eps)
+        ref, _ = oracle.enpt2("fullci", nb, nu, nd, dets, one, two, c, -1e3, eps)
+        npt.assert_allclose(e, ref, rtol=1e-11)
+        assert pyci.add_hci(ham, w, c, eps=eps) == len(expect)
+        npt.assert_array_equal(w.to_det_array().reshape(-1, 2)[len(dets):], expect)
