@@ -111,48 +111,49 @@ __device__ void block_sums_to(double (&acc)[M], double *out) {
     }
 }
 
-// partial[b][ma][mb] = sum over rows of block b of A[:, i] * B[:, j] (8x8 tile per
-// blockIdx.y). With gate0 set the launch is the second Gram-Schmidt pass and does
-// nothing when the first pass sufficed.
+// partial[b][ma][mb] = sum over the rows of block b of A[:, i] * B[:, j], a 16 x 16 tile per
+// blockIdx.y on the FP64 matrix cores: a chunk of 16 rows is four MFMA steps, lane quarter q
+// supplying rows 4q .. 4q+3 of its column in one 32-byte load, so each column is read in
+// whole 128-byte pieces, and the sum over rows needs no cross-lane step (an 8 x 8 register
+// tile per thread spent its time in the 64-value reduction: 34 us for 24 x 4 columns of
+// 152,000 rows, here 9). With gate0 set the launch is the second Gram-Schmidt pass
+// and does nothing when the first pass sufficed.
+typedef double f64x4 __attribute__((ext_vector_type(4)));
+
 __global__ void __launch_bounds__(DT) k_gram(i64 nd, const double *A, i64 lda, int ma, const double *B, i64 ldb,
                                              int mb, double *partial, const double *gate0, const double *gate1) {
     if (gate0 && !second_pass(gate0, gate1, gridDim.x)) return;
-    const int tiles_j = (mb + 7) / 8;
-    const int i0 = (blockIdx.y / tiles_j) * 8, j0 = (blockIdx.y % tiles_j) * 8;
-    const int ni = min(8, ma - i0), nj = min(8, mb - j0);
-    double acc[8][8];
+    const int tiles_j = (mb + 15) / 16;
+    const int i0 = (blockIdx.y / tiles_j) * 16, j0 = (blockIdx.y % tiles_j) * 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
+    const bool ia = i0 + lr < ma, jb = j0 + lr < mb;
+    const double *a = A + (i64)(i0 + (ia ? lr : 0)) * lda, *b = B + (i64)(j0 + (jb ? lr : 0)) * ldb;
+    const i64 step = (i64)gridDim.x * (DT / 64) * 16;
+    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
+    for (i64 r = ((i64)blockIdx.x * (DT / 64) + wave) * 16 + 4 * lk; r - 4 * lk < nd; r += step) {
+        double x[4], y[4];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = 0.0;
-    for (i64 r = (i64)blockIdx.x * DT + threadIdx.x; r < nd; r += (i64)gridDim.x * DT) {
-        double a[8], b[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) a[i] = (i < ni) ? A[(i64)(i0 + i) * lda + r] : 0.0;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) b[j] = (j < nj) ? B[(i64)(j0 + j) * ldb + r] : 0.0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-#pragma unroll
-            for (int j = 0; j < 8; ++j) acc[i][j] += a[i] * b[j];
-    }
-    __shared__ double red[DT / 64][64];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            double v = acc[i][j];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-            if (lane == 0) red[wave][i * 8 + j] = v;
+        for (int q = 0; q < 4; ++q) {
+            const i64 row = r + q < nd ? r + q : nd - 1;
+            x[q] = a[row];
+            y[q] = b[row];
         }
-    __syncthreads();
-    if (threadIdx.x < 64) {
-        const int i = threadIdx.x / 8, j = threadIdx.x % 8;
-        double v = 0.0;
-        for (int w = 0; w < DT / 64; ++w) v += red[w][threadIdx.x];
-        if (i < ni && j < nj) partial[((i64)blockIdx.x * ma + i0 + i) * mb + j0 + j] = v;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (!ia || r + q >= nd) x[q] = 0.0;
+            if (!jb || r + q >= nd) y[q] = 0.0;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q], y[q], acc, 0, 0, 0);
     }
+    __shared__ double red[DT / 64][256];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) red[wave][(4 * q + lk) * 16 + lr] = acc[q];
+    __syncthreads();
+    const int i = threadIdx.x / 16, j = threadIdx.x % 16;
+    double v = 0.0;
+    for (int w = 0; w < DT / 64; ++w) v += red[w][threadIdx.x];
+    if (i0 + i < ma && j0 + j < mb) partial[((i64)blockIdx.x * ma + i0 + i) * mb + j0 + j] = v;
 }
 
 // out[t] = sum over b of partial[b][t]; one 256-thread block per output element.
@@ -182,21 +183,35 @@ __global__ void k_gemm_update(i64 nd, const double *V, i64 ldv, int m, const dou
 // T[:, j] -= V[:, 0:m] C[:, j] with C row-major (C[i * k + j]), as the Gram products leave it
 __global__ void k_gemm_sub_rm(i64 nd, const double *V, int m, const double *C, int k, double *T) {
     for (i64 r = (i64)blockIdx.x * blockDim.x + threadIdx.x; r < nd; r += (i64)gridDim.x * blockDim.x) {
-        for (int j = 0; j < k; ++j) {
-            double acc = 0.0;
-            for (int i = 0; i < m; ++i) acc += V[(i64)i * nd + r] * C[i * k + j];
-            T[(i64)j * nd + r] -= acc;
+        for (int j0 = 0; j0 < k; j0 += 8) {
+            double acc[8] = {};
+            for (int i = 0; i < m; ++i) {
+                const double v = V[(i64)i * nd + r];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (j0 + j < k) acc[j] += v * C[i * k + j0 + j];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (j0 + j < k) T[(i64)(j0 + j) * nd + r] -= acc[j];
         }
     }
 }
 
-// T[:, j] = V[:, 0:m] C[:, j]
+// T[:, j] = V[:, 0:m] C[:, j], V read once for every 8 columns
 __global__ void k_gemm_set(i64 nd, const double *V, i64 ldv, int m, const double *C, int k, double *T, i64 ldt) {
     for (i64 r = (i64)blockIdx.x * blockDim.x + threadIdx.x; r < nd; r += (i64)gridDim.x * blockDim.x) {
-        for (int j = 0; j < k; ++j) {
-            double acc = 0.0;
-            for (int i = 0; i < m; ++i) acc += V[(i64)i * ldv + r] * C[j * m + i];
-            T[(i64)j * ldt + r] = acc;
+        for (int j0 = 0; j0 < k; j0 += 8) {
+            double acc[8] = {};
+            for (int i = 0; i < m; ++i) {
+                const double v = V[(i64)i * ldv + r];
+#pragma unroll
+                for (int j = 0; j < 8; ++j)
+                    if (j0 + j < k) acc[j] += v * C[(j0 + j) * m + i];
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if (j0 + j < k) T[(i64)(j0 + j) * ldt + r] = acc[j];
         }
     }
 }
@@ -749,7 +764,7 @@ struct Davidson {
 
     // out (ma x mb, row-major [i][j] on the device) = A^T B
     void gram(const double *A, int ma, const double *B, int mb, double *dst) {
-        dim3 grid((unsigned)nblk, (unsigned)(((ma + 7) / 8) * ((mb + 7) / 8)));
+        dim3 grid((unsigned)nblk, (unsigned)(((ma + 15) / 16) * ((mb + 15) / 16)));
         k_gram<<<grid, DT, 0, s>>>(nd, A, nd, ma, B, nd, mb, partial.p, nullptr, nullptr);
         PE_LAUNCH_CHECK();
         const int cnt = ma * mb;
@@ -841,7 +856,7 @@ struct Davidson {
             update(m, pb.p + pC2, col, p2, p0, p1);
             k_scale_final<<<(unsigned)nblk, DT, 0, s>>>(col, nd, p0, p1, p2, nblk, 1, pair);
         } else if (m <= kCgsMax) {
-            const dim3 grid((unsigned)nblk, (unsigned)((m + 7) / 8));
+            const dim3 grid((unsigned)nblk, (unsigned)((m + 15) / 16));
             k_gram<<<grid, DT, 0, s>>>(nd, V.p, nd, m, col, nd, 1, pb.p + pC1, nullptr, nullptr);
             PE_LAUNCH_CHECK();
             k_update_norm<<<(unsigned)nblk, DT, 0, s>>>(nd, V.p, m, pb.p + pC1, col, p1, nullptr, nullptr);

@@ -394,6 +394,33 @@ __device__ inline void tri_decode(int t, int &i, int &k) {
     i = t - kk * (kk - 1) / 2;
 }
 
+// Sum over each 16 (or 64) lanes by data-parallel moves, without an LDS round trip per step.
+template <int CTRL>
+__device__ inline double dpp(double v) {
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, 0xf, 0xf, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, 0xf, 0xf, true);
+    return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+template <int CTRL>
+__device__ inline float dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+
+template <int LANES, typename XT>
+__device__ inline XT lanes_sum(XT v) {
+    v += dpp<0x128>(v);  // row_ror:8, 4, 2, 1: every lane of the 16 ends with the sum
+    v += dpp<0x124>(v);
+    v += dpp<0x122>(v);
+    v += dpp<0x121>(v);
+    if (LANES == 64) {
+        v += __shfl_xor(v, 16);
+        v += __shfl_xor(v, 32);
+    }
+    return v;
+}
+
 // ---------------------------------------------------------------------------
 // Host helpers
 // ---------------------------------------------------------------------------
