@@ -111,53 +111,69 @@ __device__ void block_sums_to(double (&acc)[M], double *out) {
     }
 }
 
-// partial[b][ma][mb] = sum over the rows of block b of A[:, i] * B[:, j], a 16 x 16 tile per
-// blockIdx.y on the FP64 matrix cores: a chunk of 16 rows is four MFMA steps, lane quarter q
-// supplying rows 4q .. 4q+3 of its column in one 32-byte load, so each column is read in
-// whole 128-byte pieces, and the sum over rows needs no cross-lane step (an 8 x 8 register
-// tile per thread spent its time in the 64-value reduction: 34 us for 24 x 4 columns of
-// 152,000 rows, here 9). With gate0 set the launch is the second Gram-Schmidt pass
-// and does nothing when the first pass sufficed.
-typedef double f64x4 __attribute__((ext_vector_type(4)));
+// Sums over the 64 lanes of N values (32 or 64) by recursive halving: at each step a lane
+// passes on half of the values it holds and adds the partner's share of the other half, so
+// that N values take N - 1 exchanges (+ 1) instead of 6 N. Every value is added up in the
+// order of the shuffle tree xor 32, 16, .., 1. Lane l ends with value l (N = 64) or l / 2.
+template <int N>
+__device__ double halving_sum(double (&v)[N]) {
+    const int lane = threadIdx.x & 63;
+    int o = 32;
+#pragma unroll
+    for (int n = N; n > 1; n >>= 1, o >>= 1) {
+        const bool up = lane & o;
+#pragma unroll
+        for (int t = 0; t < n / 2; ++t) {
+            const double keep = up ? v[t + n / 2] : v[t], pass = up ? v[t] : v[t + n / 2];
+            v[t] = keep + __shfl_xor(pass, o);
+        }
+    }
+    if (N == 32) v[0] += __shfl_xor(v[0], 1);
+    return v[0];
+}
 
+// partial[b][ma][mb] = sum over rows of block b of A[:, i] * B[:, j] (8 x NJ tile per
+// blockIdx.y). The tile's reduction over the lanes bounds it at one or two rows a
+// thread: 24 x 4 columns of 152,000 rows took 34 us with 64 shuffle trees and take 10 with
+// the halving sum of 32 values (the same bits). With gate0 set the launch is the second
+// Gram-Schmidt pass and does nothing when the first pass sufficed.
+template <int NJ>
 __global__ void __launch_bounds__(DT) k_gram(i64 nd, const double *A, i64 lda, int ma, const double *B, i64 ldb,
                                              int mb, double *partial, const double *gate0, const double *gate1) {
     if (gate0 && !second_pass(gate0, gate1, gridDim.x)) return;
-    const int tiles_j = (mb + 15) / 16;
-    const int i0 = (blockIdx.y / tiles_j) * 16, j0 = (blockIdx.y % tiles_j) * 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, lr = lane & 15, lk = lane >> 4;
-    const bool ia = i0 + lr < ma, jb = j0 + lr < mb;
-    const double *a = A + (i64)(i0 + (ia ? lr : 0)) * lda, *b = B + (i64)(j0 + (jb ? lr : 0)) * ldb;
-    const i64 step = (i64)gridDim.x * (DT / 64) * 16;
-    f64x4 acc = {0.0, 0.0, 0.0, 0.0};
-    for (i64 r = ((i64)blockIdx.x * (DT / 64) + wave) * 16 + 4 * lk; r - 4 * lk < nd; r += step) {
-        double x[4], y[4];
+    const int tiles_j = (mb + NJ - 1) / NJ;
+    const int i0 = (blockIdx.y / tiles_j) * 8, j0 = (blockIdx.y % tiles_j) * NJ;
+    const int ni = min(8, ma - i0), nj = min(NJ, mb - j0);
+    double acc[8 * NJ];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const i64 row = r + q < nd ? r + q : nd - 1;
-            x[q] = a[row];
-            y[q] = b[row];
-        }
+    for (int t = 0; t < 8 * NJ; ++t) acc[t] = 0.0;
+    for (i64 r = (i64)blockIdx.x * DT + threadIdx.x; r < nd; r += (i64)gridDim.x * DT) {
+        double a[8], b[NJ];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (!ia || r + q >= nd) x[q] = 0.0;
-            if (!jb || r + q >= nd) y[q] = 0.0;
-        }
+        for (int i = 0; i < 8; ++i) a[i] = (i < ni) ? A[(i64)(i0 + i) * lda + r] : 0.0;
 #pragma unroll
-        for (int q = 0; q < 4; ++q) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(x[q], y[q], acc, 0, 0, 0);
+        for (int j = 0; j < NJ; ++j) b[j] = (j < nj) ? B[(i64)(j0 + j) * ldb + r] : 0.0;
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) acc[i * NJ + j] += a[i] * b[j];
     }
-    __shared__ double red[DT / 64][256];
-#pragma unroll
-    for (int q = 0; q < 4; ++q) red[wave][(4 * q + lk) * 16 + lr] = acc[q];
+    __shared__ double red[DT / 64][8 * NJ];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const double sum = halving_sum<8 * NJ>(acc);
+    if (NJ == 8 || !(lane & 1)) red[wave][NJ == 8 ? lane : lane >> 1] = sum;
     __syncthreads();
-    const int i = threadIdx.x / 16, j = threadIdx.x % 16;
-    double v = 0.0;
-    for (int w = 0; w < DT / 64; ++w) v += red[w][threadIdx.x];
-    if (i0 + i < ma && j0 + j < mb) partial[((i64)blockIdx.x * ma + i0 + i) * mb + j0 + j] = v;
+    if (threadIdx.x < 8 * NJ) {
+        const int i = threadIdx.x / NJ, j = threadIdx.x % NJ;
+        double v = 0.0;
+        for (int w = 0; w < DT / 64; ++w) v += red[w][threadIdx.x];
+        if (i < ni && j < nj) partial[((i64)blockIdx.x * ma + i0 + i) * mb + j0 + j] = v;
+    }
 }
 
-// out[t] = sum over b of partial[b][t]; one 256-thread block per output element.
-__global__ void __launch_bounds__(256) k_reduce_partials(const double *partial, int nblk, int count, double *out) {
+// out[t] (and out2[t]) = sum over b of partial[b][t]; one 256-thread block per element.
+__global__ void __launch_bounds__(256) k_reduce_partials(const double *partial, int nblk, int count, double *out,
+                                                         double *out2 = nullptr) {
     const int t = blockIdx.x;
     double v = 0.0;
     for (int b = threadIdx.x; b < nblk; b += 256) v += partial[(i64)b * count + t];
@@ -165,7 +181,11 @@ __global__ void __launch_bounds__(256) k_reduce_partials(const double *partial, 
     __shared__ double red[4];
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
     __syncthreads();
-    if (threadIdx.x == 0) out[t] = red[0] + red[1] + red[2] + red[3];
+    if (threadIdx.x == 0) {
+        const double sum = red[0] + red[1] + red[2] + red[3];
+        out[t] = sum;
+        if (out2) out2[t] = sum;
+    }
 }
 
 // T[:, j] += alpha * V[:, 0:m] C[:, j]   (C is m x k column-major on the device)
@@ -396,6 +416,165 @@ __global__ void __launch_bounds__(DT) k_ritz1(i64 nd, const double *__restrict__
     }
 }
 
+// Scale that normalises a vector of squared norm n1sq; one whose norm fell below 1e-10 of
+// its norm before orthogonalisation (square n0sq) is numerically dependent on the basis
+// and is zeroed instead (the host drops it later).
+__device__ inline double checked_scale(double n0sq, double n1sq) {
+    const double n0 = sqrt(fmax(n0sq, 0.0)), n1 = sqrt(fmax(n1sq, 0.0));
+    return (n1 > 1e-10 * fmax(n0, 1e-300) && n1 > 1e-300) ? 1.0 / n1 : 0.0;
+}
+
+// Whole spaces of up to 2,048 determinants, one root: everything between the Rayleigh-Ritz
+// step and the next sigma in one block, which holds its two rows per thread of the basis in
+// registers: the residual and correction of k_ritz1, both Gram-Schmidt passes (the
+// second where the first removed more than half of the squared norm) and the
+// normalisation. Five launches of 3-4 us each, whose data fits one CU, become one.
+constexpr int SMALL_ND = 2048;
+constexpr int ST = 1024;
+
+// out[i] = sum of v[i] over the block's threads, for all of them
+template <int N>
+__device__ void small_sums(double (&v)[N], double *red, double *out) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const double t = lanes_sum<64>(v[i]);
+        if (lane == 0) red[wave * N + i] = t;
+    }
+    __syncthreads();
+    if (threadIdx.x < N) {
+        double t = 0.0;
+        for (int w = 0; w < ST / 64; ++w) t += red[w * N + threadIdx.x];
+        out[threadIdx.x] = t;
+    }
+    __syncthreads();
+}
+
+template <int M>
+__global__ void __launch_bounds__(ST) k_step_small(int nd, const double *__restrict__ V, const double *__restrict__ W,
+                                                   RitzCoef cf, const double *__restrict__ diag,
+                                                   double *__restrict__ T, double *res2, double *pair) {
+    __shared__ double red[ST / 64 * (M + 2)], out[M + 2];
+    double v[2][M], t[2];
+    double acc[M + 2] = {};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int r = threadIdx.x + u * ST;
+        t[u] = 0.0;
+#pragma unroll
+        for (int i = 0; i < M; ++i) v[u][i] = 0.0;
+        if (r < nd) {
+            double x = 0.0, wx = 0.0;
+#pragma unroll
+            for (int i = 0; i < M; ++i) {
+                v[u][i] = V[(i64)i * nd + r];
+                x += v[u][i] * cf.y[i];
+                wx += W[(i64)i * nd + r] * cf.y[i];
+            }
+            const double res = wx - cf.theta * x;
+            double den = cf.theta - diag[r];
+            if (fabs(den) < 1e-8) den = (den < 0.0) ? -1e-8 : 1e-8;
+            t[u] = res / den;
+            acc[M] += res * res;
+            acc[M + 1] += t[u] * t[u];
+        }
+#pragma unroll
+        for (int i = 0; i < M; ++i) acc[i] += v[u][i] * t[u];
+    }
+    small_sums<M + 2>(acc, red, out);
+    const double n0 = out[M + 1];
+    if (threadIdx.x == 0) *res2 = out[M];
+    double nn = n0;
+    for (int pass = 0; pass < 2; ++pass) {  // uniform: every thread sees the same sums
+        double c[M], s2[1] = {0.0};
+#pragma unroll
+        for (int i = 0; i < M; ++i) c[i] = out[i];
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            double a = 0.0;
+#pragma unroll
+            for (int i = 0; i < M; ++i) a += v[u][i] * c[i];
+            t[u] -= a;
+            s2[0] += t[u] * t[u];
+        }
+        small_sums<1>(s2, red, out);
+        nn = out[0];
+        if (pass || !(nn < 0.5 * n0)) break;
+        __syncthreads();
+        double d[M];
+#pragma unroll
+        for (int i = 0; i < M; ++i) d[i] = v[0][i] * t[0] + v[1][i] * t[1];
+        small_sums<M>(d, red, out);
+    }
+    const double sc = checked_scale(n0, nn);
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+        if (threadIdx.x + u * ST < nd) T[threadIdx.x + u * ST] = t[u] * sc;
+    if (threadIdx.x == 0) {
+        pair[0] = n0;
+        pair[1] = nn;
+    }
+}
+
+// dst[i] = A[:, i] . x of such a space, i < M
+template <int M>
+__global__ void __launch_bounds__(ST) k_dots_small(int nd, const double *__restrict__ A, const double *__restrict__ x,
+                                                   double *dst) {
+    __shared__ double red[ST / 64 * M], out[M];
+    double acc[M] = {};
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int r = threadIdx.x + u * ST;
+        if (r < nd) {
+            const double xr = x[r];
+#pragma unroll
+            for (int i = 0; i < M; ++i) acc[i] += A[(i64)i * nd + r] * xr;
+        }
+    }
+    small_sums<M>(acc, red, out);
+    if (threadIdx.x < M) dst[threadIdx.x] = out[threadIdx.x];
+}
+
+// Corrections src[:, cols[j]] to dst[:, j], projected on the parity sector sgn (0: copied).
+struct ColList {
+    int c[16];
+};
+
+__global__ void k_put_block(const double *src, double *dst, i64 nd, i64 nb, double sgn, ColList cols, int cnt) {
+    for (i64 J = (i64)blockIdx.x * DT + threadIdx.x; J < nd; J += (i64)gridDim.x * DT) {
+        const i64 P = sgn != 0.0 ? J % nb * nb + J / nb : J;
+        for (int j = 0; j < cnt; ++j) {
+            const double *s = src + (i64)cols.c[j] * nd;
+            double x = s[J];
+            if (sgn != 0.0) x = 0.5 * (x + sgn * s[P]);
+            dst[(i64)j * nd + J] = x;
+        }
+    }
+}
+
+// B[:, j] = sum over i < cnt of B[:, i] C[i * kept + j] (j < kept <= cnt <= 16, in place: a
+// thread has read its row before it writes it), and the same rows row-major for the sigma.
+template <typename XT>
+__global__ void __launch_bounds__(DT) k_block_columns(i64 nd, double *B, int cnt, const double *C, int kept,
+                                                      XT *rows) {
+    for (i64 r = (i64)blockIdx.x * DT + threadIdx.x; r < nd; r += (i64)gridDim.x * DT) {
+        double acc[16] = {};
+        for (int i = 0; i < cnt; ++i) {
+            const double v = B[(i64)i * nd + r];
+#pragma unroll
+            for (int j = 0; j < 16; ++j)
+                if (j < kept) acc[j] += v * C[i * kept + j];
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (j < kept) {
+                B[(i64)j * nd + r] = acc[j];
+                if (rows) rows[r * kept + j] = (XT)acc[j];
+            }
+    }
+}
+
 // d[r] = (diag[r] + diag[P r]) / 2 for P's index map (r = Ia nb + Ib -> Ib nb + Ia):
 // the same bits at r and P r.
 __global__ void k_symdiag(const double *diag, double *d, i64 nd, i64 nb) {
@@ -480,19 +659,6 @@ __global__ void k_scale(double *x, i64 n, double s) {
     for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) x[i] *= s;
 }
 
-// Normalises x by the norm whose square is nn[1]; a vector whose norm fell below
-// 1e-10 of its norm before orthogonalisation (square in nn[0]) is numerically
-// dependent on the basis and is zeroed instead (the host drops it later).
-__device__ inline double checked_scale(double n0sq, double n1sq) {
-    const double n0 = sqrt(fmax(n0sq, 0.0)), n1 = sqrt(fmax(n1sq, 0.0));
-    return (n1 > 1e-10 * fmax(n0, 1e-300) && n1 > 1e-300) ? 1.0 / n1 : 0.0;
-}
-
-__global__ void k_scale_checked(double *x, i64 n, const double *nn) {
-    const double s = checked_scale(nn[0], nn[1]);
-    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (i64)gridDim.x * blockDim.x) x[i] *= s;
-}
-
 // Final normalisation of an orthogonalised correction from the partial squared
 // norms (npart per block) before Gram-Schmidt (p0), after the first pass (p1) and
 // after the second (p2, used when `gated` and the second pass ran). Writes the
@@ -552,43 +718,68 @@ __global__ void k_row2col(i64 nd, int k, const S *src, D *dst, i64 ld) {
 }
 
 // ---------------------------------------------------------------------------
-// Host: cyclic Jacobi eigensolver for the small symmetric Rayleigh matrix.
+// Host: cyclic Jacobi eigensolver for the small symmetric Rayleigh matrix. Its rotations
+// start from the identity and keep a positive share of each basis vector, which fixes
+// the signs of the Ritz vectors. The GPU idles meanwhile on a lone run of one root, so with
+// `mirror` a rotation works on rows of the matrix, mirrors them into the columns, and is left
+// out where rounding would swallow it. Blocks rotate rows and columns: a mixed-precision
+// block turns the last bits of its FP32 phase into the signs of its eigenvectors, and these
+// stay what they were.
 // ---------------------------------------------------------------------------
-static void jacobi_eig(int m, std::vector<double> a, std::vector<double> &w, std::vector<double> &v) {
+static void jacobi_eig(int m, std::vector<double> a, std::vector<double> &w, std::vector<double> &v, bool mirror) {
     // a: m x m row-major symmetric; returns ascending w and eigenvectors as columns of v (row-major m x m)
-    v.assign((size_t)m * m, 0.0);
-    for (int i = 0; i < m; ++i) v[(size_t)i * m + i] = 1.0;
+    std::vector<double> z((size_t)m * m, 0.0);  // rows: the rotated basis vectors
+    for (int i = 0; i < m; ++i) z[(size_t)i * m + i] = 1.0;
     for (int sweep = 0; sweep < 100; ++sweep) {
         double off = 0.0, tot = 0.0;
         for (int p = 0; p < m; ++p)
             for (int q = 0; q < m; ++q) {
-                double x = a[(size_t)p * m + q] * a[(size_t)p * m + q];
+                const double x = a[(size_t)p * m + q] * a[(size_t)p * m + q];
                 tot += x;
                 if (p != q) off += x;
             }
         if (off <= 1e-30 * tot || off == 0.0) break;
         for (int p = 0; p < m - 1; ++p)
             for (int q = p + 1; q < m; ++q) {
-                double apq = a[(size_t)p * m + q];
+                double *rp = &a[(size_t)p * m], *rq = &a[(size_t)q * m];
+                const double apq = rp[q];
                 if (apq == 0.0) continue;
-                double app = a[(size_t)p * m + p], aqq = a[(size_t)q * m + q];
-                double tau = (aqq - app) / (2.0 * apq);
-                double t = (tau >= 0 ? 1.0 : -1.0) / (std::fabs(tau) + std::sqrt(1.0 + tau * tau));
-                double c = 1.0 / std::sqrt(1.0 + t * t), s = t * c;
-                for (int r = 0; r < m; ++r) {
-                    double arp = a[(size_t)r * m + p], arq = a[(size_t)r * m + q];
-                    a[(size_t)r * m + p] = c * arp - s * arq;
-                    a[(size_t)r * m + q] = s * arp + c * arq;
+                const double app = rp[p], aqq = rq[q];
+                const double tau = (aqq - app) / (2.0 * apq);
+                if (mirror && std::fabs(tau) > 1e19) {  // an angle below 1e-19
+                    rp[q] = rq[p] = 0.0;
+                    continue;
+                }
+                const double t = (tau >= 0 ? 1.0 : -1.0) / (std::fabs(tau) + std::sqrt(1.0 + tau * tau));
+                const double c = 1.0 / std::sqrt(1.0 + t * t), sn = t * c;
+                if (!mirror) {
+                    double *col = a.data();
+                    for (int r = 0; r < m; ++r, col += m) {
+                        const double x = col[p], y = col[q];
+                        col[p] = c * x - sn * y;
+                        col[q] = sn * x + c * y;
+                    }
                 }
                 for (int r = 0; r < m; ++r) {
-                    double apr = a[(size_t)p * m + r], aqr = a[(size_t)q * m + r];
-                    a[(size_t)p * m + r] = c * apr - s * aqr;
-                    a[(size_t)q * m + r] = s * apr + c * aqr;
+                    const double x = rp[r], y = rq[r];
+                    rp[r] = c * x - sn * y;
+                    rq[r] = sn * x + c * y;
                 }
+                if (mirror) {
+                    rp[p] = app - t * apq;
+                    rq[q] = aqq + t * apq;
+                    rp[q] = rq[p] = 0.0;
+                    double *col = a.data();
+                    for (int r = 0; r < m; ++r, col += m) {  // the 2 x 2 block is in place already
+                        col[p] = r == p || r == q ? col[p] : rp[r];
+                        col[q] = r == p || r == q ? col[q] : rq[r];
+                    }
+                }
+                double *zp = &z[(size_t)p * m], *zq = &z[(size_t)q * m];
                 for (int r = 0; r < m; ++r) {
-                    double vrp = v[(size_t)r * m + p], vrq = v[(size_t)r * m + q];
-                    v[(size_t)r * m + p] = c * vrp - s * vrq;
-                    v[(size_t)r * m + q] = s * vrp + c * vrq;
+                    const double x = zp[r], y = zq[r];
+                    zp[r] = c * x - sn * y;
+                    zq[r] = sn * x + c * y;
                 }
             }
     }
@@ -596,13 +787,12 @@ static void jacobi_eig(int m, std::vector<double> a, std::vector<double> &w, std
     std::iota(order.begin(), order.end(), 0);
     std::stable_sort(order.begin(), order.end(),
                      [&](int x, int y) { return a[(size_t)x * m + x] < a[(size_t)y * m + y]; });
-    std::vector<double> vv((size_t)m * m);
+    v.resize((size_t)m * m);
     w.resize(m);
     for (int c = 0; c < m; ++c) {
         w[c] = a[(size_t)order[c] * m + order[c]];
-        for (int r = 0; r < m; ++r) vv[(size_t)r * m + c] = v[(size_t)r * m + order[c]];
+        for (int r = 0; r < m; ++r) v[(size_t)r * m + c] = z[(size_t)order[c] * m + r];
     }
-    v.swap(vv);
 }
 
 // What the first parity sector's run tells the second one, which runs
@@ -648,7 +838,7 @@ struct Davidson {
     // dv / hb layout (doubles): Ritz coefficients Y (m x k) and theta go down; the
     // squared residual norms, the new G block and the norm pairs of the added
     // columns come back in one copy
-    size_t oY, oTH, oYK, oRES, oC1, oC2, oNRM, oPAIR, oG, osz;
+    size_t oY, oTH, oYK, oRES, oC1, oC2, oNRM, oPAIR, oG, oG2, osz;
     size_t pRES, pN0, pN1, pN2, pC1, pC2;  // in pb: nblk entries per block-partial quantity
     static constexpr int kCgsMax = 128;    // basis size up to which Gram-Schmidt runs on partials
 
@@ -676,13 +866,14 @@ struct Davidson {
         oY = 0;
         oTH = oY + M * 16;
         oYK = oTH + 16;
-        oRES = oYK + M * 32;
+        oRES = oYK + std::max<size_t>(M * 32, 2 * 16 * 16);
         oC1 = oRES + 16;
         oC2 = oC1 + M;
         oNRM = oC2 + M;
         oPAIR = oNRM + 3 * 16;
         oG = oPAIR + 2 * 16;
-        osz = oG + M * 16;
+        oG2 = oG + M * 16;
+        osz = oG2 + M * 16;
         dv.ensure(osz);
         hb.ensure(osz);
         PE_HIP(hipHostGetDevicePointer((void **)&hd, hb.p, 0));
@@ -755,6 +946,19 @@ struct Davidson {
             gram(A, m_, x, 1, dst);
             return;
         }
+        if (nd <= SMALL_ND) {
+            switch (m_) {
+#define PE_DS(M)                                                            \
+    case M:                                                                 \
+        k_dots_small<M><<<1, ST, 0, s>>>((int)nd, A, x, dst);               \
+        break;
+                PE_DS(1) PE_DS(2) PE_DS(3) PE_DS(4) PE_DS(5) PE_DS(6) PE_DS(7) PE_DS(8)
+                PE_DS(9) PE_DS(10) PE_DS(11) PE_DS(12) PE_DS(13) PE_DS(14) PE_DS(15) PE_DS(16)
+#undef PE_DS
+            }
+            PE_LAUNCH_CHECK();
+            return;
+        }
         dots(A, m_, x, partial.p, nullptr, nullptr, half ? hnb() : 0u);
         k_reduce_partials<<<(unsigned)m_, 256, 0, s>>>(partial.p, nblk, m_, dst);
         PE_LAUNCH_CHECK();
@@ -763,12 +967,16 @@ struct Davidson {
     unsigned g1() const { return (unsigned)std::min<i64>(4096, (nd + 255) / 256); }
 
     // out (ma x mb, row-major [i][j] on the device) = A^T B
-    void gram(const double *A, int ma, const double *B, int mb, double *dst) {
-        dim3 grid((unsigned)nblk, (unsigned)(((ma + 15) / 16) * ((mb + 15) / 16)));
-        k_gram<<<grid, DT, 0, s>>>(nd, A, nd, ma, B, nd, mb, partial.p, nullptr, nullptr);
+    void gram(const double *A, int ma, const double *B, int mb, double *dst, double *dst2 = nullptr) {
+        const int nj = mb <= 4 ? 4 : 8;
+        dim3 grid((unsigned)nblk, (unsigned)(((ma + 7) / 8) * ((mb + nj - 1) / nj)));
+        if (nj == 4)
+            k_gram<4><<<grid, DT, 0, s>>>(nd, A, nd, ma, B, nd, mb, partial.p, nullptr, nullptr);
+        else
+            k_gram<8><<<grid, DT, 0, s>>>(nd, A, nd, ma, B, nd, mb, partial.p, nullptr, nullptr);
         PE_LAUNCH_CHECK();
         const int cnt = ma * mb;
-        k_reduce_partials<<<(unsigned)cnt, 256, 0, s>>>(partial.p, nblk, cnt, dst);
+        k_reduce_partials<<<(unsigned)cnt, 256, 0, s>>>(partial.p, nblk, cnt, dst, dst2);
         PE_LAUNCH_CHECK();
     }
 
@@ -780,15 +988,21 @@ struct Davidson {
         return h;  // [i][j]
     }
 
-    // W[:, c0:c0+cnt] = H V[:, c0:c0+cnt]
-    void apply(int c0, int cnt, bool fp32) {
+    void ensure32(int cnt) {
+        row32.ensure((size_t)(nd * std::max(cnt, k)));
+        out32.ensure((size_t)(nd * std::max(cnt, k)));
+    }
+
+    // W[:, c0:c0+cnt] = H V[:, c0:c0+cnt] (rows_ready: already row-major in rowbuf / row32)
+    void apply(int c0, int cnt, bool fp32, bool rows_ready = false) {
         const double *src = V.p + (i64)c0 * nd;
         double *dst = W.p + (i64)c0 * nd;
         if (fp32) {
-            row32.ensure((size_t)(nd * std::max(cnt, k)));
-            out32.ensure((size_t)(nd * std::max(cnt, k)));
-            k_col2row<double, float><<<g1(), 256, 0, s>>>(nd, cnt, src, nd, row32.p);
-            PE_LAUNCH_CHECK();
+            ensure32(cnt);
+            if (!rows_ready) {
+                k_col2row<double, float><<<g1(), 256, 0, s>>>(nd, cnt, src, nd, row32.p);
+                PE_LAUNCH_CHECK();
+            }
             sigma_f32(op, cnt, row32.p, out32.p, s, sector, ws);
             k_row2col<float, double><<<g1(), 256, 0, s>>>(nd, cnt, out32.p, dst, nd);
             PE_LAUNCH_CHECK();
@@ -796,8 +1010,10 @@ struct Davidson {
         } else if (cnt == 1) {
             sigma_f64(op, 1, src, dst, s, sector, ws);
         } else {
-            k_col2row<double, double><<<g1(), 256, 0, s>>>(nd, cnt, src, nd, rowbuf.p);
-            PE_LAUNCH_CHECK();
+            if (!rows_ready) {
+                k_col2row<double, double><<<g1(), 256, 0, s>>>(nd, cnt, src, nd, rowbuf.p);
+                PE_LAUNCH_CHECK();
+            }
             sigma_f64(op, cnt, rowbuf.p, rowout.p, s, sector, ws);
             k_row2col<double, double><<<g1(), 256, 0, s>>>(nd, cnt, rowout.p, dst, nd);
             PE_LAUNCH_CHECK();
@@ -856,12 +1072,12 @@ struct Davidson {
             update(m, pb.p + pC2, col, p2, p0, p1);
             k_scale_final<<<(unsigned)nblk, DT, 0, s>>>(col, nd, p0, p1, p2, nblk, 1, pair);
         } else if (m <= kCgsMax) {
-            const dim3 grid((unsigned)nblk, (unsigned)((m + 15) / 16));
-            k_gram<<<grid, DT, 0, s>>>(nd, V.p, nd, m, col, nd, 1, pb.p + pC1, nullptr, nullptr);
+            const dim3 grid((unsigned)nblk, (unsigned)((m + 7) / 8));
+            k_gram<4><<<grid, DT, 0, s>>>(nd, V.p, nd, m, col, nd, 1, pb.p + pC1, nullptr, nullptr);
             PE_LAUNCH_CHECK();
             k_update_norm<<<(unsigned)nblk, DT, 0, s>>>(nd, V.p, m, pb.p + pC1, col, p1, nullptr, nullptr);
             PE_LAUNCH_CHECK();
-            k_gram<<<grid, DT, 0, s>>>(nd, V.p, nd, m, col, nd, 1, pb.p + pC2, p0, p1);
+            k_gram<4><<<grid, DT, 0, s>>>(nd, V.p, nd, m, col, nd, 1, pb.p + pC2, p0, p1);
             PE_LAUNCH_CHECK();
             k_update_norm<<<(unsigned)nblk, DT, 0, s>>>(nd, V.p, m, pb.p + pC2, col, p2, p0, p1);
             PE_LAUNCH_CHECK();
@@ -881,31 +1097,31 @@ struct Davidson {
         ++m;
     }
 
-    // Block Gram-Schmidt of the cnt corrections in V[:, m0 .. m0 + cnt): twice
-    // against V[:, 0:m0] (each pass reads the basis once for the whole block), then
-    // Cholesky-QR twice within the block; a column whose squared norm falls below
-    // 1e-20 of its value before orthogonalisation is dependent and dropped. The
-    // kept columns end orthonormal at m0 .. m0 + kept; returns kept.
-    int orthonormalize_block(int m0, int cnt) {
+    // The corrections T[:, add[j]] as new basis columns V[:, m0 .. m0 + kept): block
+    // Gram-Schmidt twice against V[:, 0:m0] (each pass reads the basis once for the whole
+    // block), then Cholesky-QR twice within the block; a column whose squared norm falls below
+    // 1e-20 of its value before orthogonalisation is dependent and dropped. Returns kept. The
+    // first Gram product also brings the squared norms before, and the last combination
+    // leaves the columns row-major in rowbuf / row32 for the sigma.
+    int orthonormalize_block(int m0, const std::vector<int> &add, int cnt, bool fp32) {
         double *blk = V.p + (i64)m0 * nd;
-        const size_t ss = (size_t)cnt * cnt;
-        gram(blk, cnt, blk, cnt, dv.p + oG);  // squared norms before (diagonal)
-        PE_HIP(hipMemcpyAsync(hb.p + oG, dv.p + oG, sizeof(double) * ss, hipMemcpyDeviceToHost, s));
-        PE_HIP(hipStreamSynchronize(s));
-        std::vector<double> ref(cnt);
-        for (int j = 0; j < cnt; ++j) ref[(size_t)j] = hb.p[oG + (size_t)j * cnt + j];
-        if (m0 > 0)
-            for (int pass = 0; pass < 2; ++pass) {
-                gram(V.p, m0, blk, cnt, dv.p + oG);
-                k_gemm_sub_rm<<<g1(), 256, 0, s>>>(nd, V.p, m0, dv.p + oG, cnt, blk);
-                PE_LAUNCH_CHECK();
-            }
+        ColList cl{};
+        for (int j = 0; j < cnt; ++j) cl.c[j] = add[(size_t)j];
+        k_put_block<<<g1(), DT, 0, s>>>(T.p, blk, nd, swap_nb, sector != 0 ? (double)sector : 0.0, cl, cnt);
+        PE_LAUNCH_CHECK();
+        gram(V.p, m0 + cnt, blk, cnt, dv.p + oG, hd + oG);
+        for (int pass = 0; pass < 2 && m0 > 0; ++pass) {
+            if (pass) gram(V.p, m0, blk, cnt, dv.p + oG);
+            k_gemm_sub_rm<<<g1(), 256, 0, s>>>(nd, V.p, m0, dv.p + oG, cnt, blk);
+            PE_LAUNCH_CHECK();
+        }
+        std::vector<double> ref;
         for (int round = 0; round < 2 && cnt > 0; ++round) {
-            gram(blk, cnt, blk, cnt, dv.p + oG);
-            PE_HIP(hipMemcpyAsync(hb.p + oG, dv.p + oG, sizeof(double) * (size_t)cnt * cnt, hipMemcpyDeviceToHost,
-                                  s));
+            gram(blk, cnt, blk, cnt, hd + oG2);
             PE_HIP(hipStreamSynchronize(s));
-            const double *S = hb.p + oG;
+            if (round == 0)
+                for (int j = 0; j < cnt; ++j) ref.push_back(hb.p[oG + (size_t)(m0 + j) * cnt + j]);
+            const double *S = hb.p + oG2;
             // Cholesky of S with dependent columns dropped: R (upper, over kept columns)
             std::vector<int> keep;
             std::vector<double> R((size_t)cnt * cnt, 0.0);
@@ -926,9 +1142,17 @@ struct Davidson {
                     for (int i = 0; i < cnt; ++i) R[(size_t)i * cnt + j] = 0.0;
                 }
             }
-            // M (cnt x kept, column-major) = inverse of R restricted to the kept columns
             const int kept = (int)keep.size();
-            std::vector<double> M((size_t)cnt * std::max(kept, 1), 0.0);
+            std::vector<double> nref((size_t)kept);
+            for (int a = 0; a < kept; ++a) nref[(size_t)a] = ref[(size_t)keep[(size_t)a]];
+            ref.swap(nref);
+            if (kept == 0) {
+                cnt = 0;
+                break;
+            }
+            // inverse of R restricted to the kept columns, [cnt][kept]
+            double *Q = hb.p + oYK + (size_t)round * 16 * 16;  // the first round's may still be on its way
+            std::fill(Q, Q + (size_t)cnt * kept, 0.0);
             for (int a = 0; a < kept; ++a) {
                 // column a of R_kept^{-1}: back substitution
                 std::vector<double> z((size_t)kept, 0.0);
@@ -939,23 +1163,19 @@ struct Davidson {
                         x += R[(size_t)keep[(size_t)b] * cnt + keep[(size_t)c]] * z[(size_t)c];
                     z[(size_t)b] = -x / R[(size_t)keep[(size_t)b] * cnt + keep[(size_t)b]];
                 }
-                for (int b = 0; b <= a; ++b) M[(size_t)a * cnt + keep[(size_t)b]] = z[(size_t)b];
+                for (int b = 0; b <= a; ++b) Q[(size_t)keep[(size_t)b] * kept + a] = z[(size_t)b];
             }
-            std::vector<double> nref((size_t)kept);
-            for (int a = 0; a < kept; ++a) nref[(size_t)a] = ref[(size_t)keep[(size_t)a]];
-            ref.swap(nref);
-            if (kept == 0) {
-                cnt = 0;
-                break;
-            }
-            std::memcpy(hb.p + oYK, M.data(), sizeof(double) * M.size());
-            PE_HIP(hipMemcpyAsync(dv.p + oYK, hb.p + oYK, sizeof(double) * M.size(), hipMemcpyHostToDevice, s));
-            k_gemm_set<<<g1(), 256, 0, s>>>(nd, blk, nd, cnt, dv.p + oYK, kept, rowbuf.p, nd);
+            double *dq = dv.p + oYK + (size_t)round * 16 * 16;
+            PE_HIP(hipMemcpyAsync(dq, Q, sizeof(double) * (size_t)cnt * kept, hipMemcpyHostToDevice, s));
+            if (round == 0)
+                k_block_columns<double><<<g1(), DT, 0, s>>>(nd, blk, cnt, dq, kept, nullptr);
+            else if (fp32)
+                k_block_columns<float><<<g1(), DT, 0, s>>>(nd, blk, cnt, dq, kept, row32.p);
+            else
+                k_block_columns<double><<<g1(), DT, 0, s>>>(nd, blk, cnt, dq, kept, rowbuf.p);
             PE_LAUNCH_CHECK();
-            PE_HIP(hipMemcpyAsync(blk, rowbuf.p, sizeof(double) * nd * kept, hipMemcpyDeviceToDevice, s));
             cnt = kept;
         }
-        PE_HIP(hipStreamSynchronize(s));  // the host-side M must outlive its copy
         for (int j = 0; j < cnt; ++j) {
             hb.p[oPAIR + 2 * j] = 1.0;
             hb.p[oPAIR + 2 * j + 1] = 1.0;
@@ -1042,12 +1262,27 @@ struct Davidson {
     // The speculative one-root pass (k = 1, m < mmax, m <= 16): the correction goes
     // straight to V[:, m] with its squared norm (pN0) and its first Gram-Schmidt
     // coefficients (pC1), see k_ritz1.
-    void ritz_spec(const std::vector<double> &y, const std::vector<double> &theta) {
+    // With `whole` the rest of the iteration up to the sigma as well (k_step_small).
+    void ritz_spec(const std::vector<double> &y, const std::vector<double> &theta, bool whole) {
         RitzCoef cf{};
         for (int i = 0; i < m; ++i) cf.y[i] = hb.p[oY + i] = y[(size_t)i * m];
         cf.theta = hb.p[oTH] = theta[0];
         y_dev = false;  // in hb only (finish_x uploads them when it needs them)
         double *t = V.p + (i64)m * nd;
+        if (whole) {
+            switch (m) {
+#define PE_ST(M)                                                                                               \
+    case M:                                                                                                    \
+        k_step_small<M><<<1, ST, 0, s>>>((int)nd, V.p, W.p, cf, dg, t, hd + oRES, hd + oPAIR);                \
+        break;
+                PE_ST(1) PE_ST(2) PE_ST(3) PE_ST(4) PE_ST(5) PE_ST(6) PE_ST(7) PE_ST(8)
+                PE_ST(9) PE_ST(10) PE_ST(11) PE_ST(12) PE_ST(13) PE_ST(14) PE_ST(15) PE_ST(16)
+#undef PE_ST
+                default: throw EngineError(PYCI_EUNSUPPORTED, "basis too large for the one-column passes");
+            }
+            PE_LAUNCH_CHECK();
+            return;
+        }
         switch (m) {
 #define PE_R1(M)                                                                                               \
     case M:                                                                                                    \
@@ -1101,27 +1336,17 @@ struct Davidson {
     // Thick restart on the lowest kk Ritz vectors: they are orthonormal and G
     // becomes diag(w).
     void restart(int kk, const std::vector<double> &w, const std::vector<double> &y) {
-        if (kk > k) {
-            RV.ensure((size_t)(nd * 2 * k));
-            RW.ensure((size_t)(nd * 2 * k));
-            for (int j = 0; j < kk; ++j)
-                for (int i = 0; i < m; ++i) hb.p[oYK + (size_t)j * m + i] = y[(size_t)i * m + j];
-            PE_HIP(hipMemcpyAsync(dv.p + oYK, hb.p + oYK, sizeof(double) * (size_t)m * kk, hipMemcpyHostToDevice, s));
-            k_gemm_set<<<g1(), 256, 0, s>>>(nd, V.p, nd, m, dv.p + oYK, kk, RV.p, nd);
-            PE_LAUNCH_CHECK();
-            k_gemm_set<<<g1(), 256, 0, s>>>(nd, W.p, nd, m, dv.p + oYK, kk, RW.p, nd);
-            PE_LAUNCH_CHECK();
-            put_basis(RV.p, kk);
-            PE_HIP(hipMemcpyAsync(W.p, RW.p, sizeof(double) * nd * kk, hipMemcpyDeviceToDevice, s));
-        } else {
-            // the Ritz vectors of this iteration are the whole restart
-            k_gemm_set<<<g1(), 256, 0, s>>>(nd, V.p, nd, m, dv.p + oY, k, X.p, nd);
-            PE_LAUNCH_CHECK();
-            k_gemm_set<<<g1(), 256, 0, s>>>(nd, W.p, nd, m, dv.p + oY, k, WX.p, nd);
-            PE_LAUNCH_CHECK();
-            put_basis(X.p, k);
-            PE_HIP(hipMemcpyAsync(W.p, WX.p, sizeof(double) * nd * k, hipMemcpyDeviceToDevice, s));
-        }
+        RV.ensure((size_t)(nd * 2 * k));
+        RW.ensure((size_t)(nd * 2 * k));
+        for (int j = 0; j < kk; ++j)
+            for (int i = 0; i < m; ++i) hb.p[oYK + (size_t)j * m + i] = y[(size_t)i * m + j];
+        PE_HIP(hipMemcpyAsync(dv.p + oYK, hb.p + oYK, sizeof(double) * (size_t)m * kk, hipMemcpyHostToDevice, s));
+        k_gemm_set<<<g1(), 256, 0, s>>>(nd, V.p, nd, m, dv.p + oYK, kk, RV.p, nd);
+        PE_LAUNCH_CHECK();
+        k_gemm_set<<<g1(), 256, 0, s>>>(nd, W.p, nd, m, dv.p + oYK, kk, RW.p, nd);
+        PE_LAUNCH_CHECK();
+        put_basis(RV.p, kk);
+        PE_HIP(hipMemcpyAsync(W.p, RW.p, sizeof(double) * nd * kk, hipMemcpyDeviceToDevice, s));
         std::fill(G.begin(), G.end(), 0.0);
         for (int j = 0; j < kk; ++j) G[(size_t)j * mmax + j] = w[(size_t)j];
         m = kk;
@@ -1179,14 +1404,16 @@ struct Davidson {
             std::vector<double> gm((size_t)m * m), w, y;
             for (int i = 0; i < m; ++i)
                 for (int j = 0; j < m; ++j) gm[(size_t)i * m + j] = G[(size_t)i * mmax + j];
-            jacobi_eig(m, gm, w, y);
+            jacobi_eig(m, std::move(gm), w, y, k == 1);
             theta.assign(w.begin(), w.begin() + k);
             // one root with room for the next column: the correction comes out of the
             // Ritz pass already in its basis slot (in a sector only where the sigma keeps
             // the sector to the last bit: there is no projection on this path)
             const bool fused = spec && exact && m < nd && m + 1 <= mmax && m <= 16;
+            // a space that one block holds: up to the sigma in one launch
+            const bool whole = fused && nd <= SMALL_ND;
             if (fused)
-                ritz_spec(y, theta);
+                ritz_spec(y, theta, whole);
             else
                 ritz(y, theta, false);
             mx = m;
@@ -1199,7 +1426,10 @@ struct Davidson {
                 }
                 m0 = m;
                 if (!fused) put_correction(0);
-                orthonormalize_device(0, fused);
+                if (whole)
+                    ++m;
+                else
+                    orthonormalize_device(0, fused);
                 apply(m0, 1, fp32);
                 dots_to(V.p, m0 + 1, W.p + (i64)m0 * nd, hd + oG, sector != 0 && exact);
                 nspec = 1;
@@ -1283,15 +1513,11 @@ struct Davidson {
                     accept_G(m0, 1);
                 } else if (room > 1) {
                     // block Gram-Schmidt: the basis is read once per pass for all corrections
-                    for (int a = 0; a < room; ++a) {
-                        put_correction(add[(size_t)a]);
-                        ++m;
-                    }
-                    m = m0;
-                    const int kept = orthonormalize_block(m0, room);
+                    if (fp32) ensure32(room);
+                    const int kept = orthonormalize_block(m0, add, room, fp32);
                     m = m0 + kept;
                     if (kept > 0) {
-                        apply(m0, kept, fp32);
+                        apply(m0, kept, fp32, kept > 1 || fp32);
                         gram(V.p, m, W.p + (i64)m0 * nd, kept, hd + oG);
                         readback();
                         accept_G(m0, kept);
