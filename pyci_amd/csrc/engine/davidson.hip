@@ -115,28 +115,33 @@ __device__ void block_sums_to(double (&acc)[M], double *out) {
 // passes on half of the values it holds and adds the partner's share of the other half, so
 // that N values take N - 1 exchanges (+ 1) instead of 6 N. Every value is added up in the
 // order of the shuffle tree xor 32, 16, .., 1. Lane l ends with value l (N = 64) or l / 2.
+template <int N, int O, int L>
+__device__ inline void halve(double (&v)[L]) {
+    if constexpr (N > 1) {
+        const bool up = threadIdx.x & O;
+#pragma unroll
+        for (int t = 0; t < N / 2; ++t) {
+            const double keep = up ? v[t + N / 2] : v[t], pass = up ? v[t] : v[t + N / 2];
+            v[t] = keep + __shfl_xor(pass, O);
+        }
+        halve<N / 2, O / 2, L>(v);
+    }
+}
+
 template <int N>
 __device__ double halving_sum(double (&v)[N]) {
-    const int lane = threadIdx.x & 63;
-    int o = 32;
-#pragma unroll
-    for (int n = N; n > 1; n >>= 1, o >>= 1) {
-        const bool up = lane & o;
-#pragma unroll
-        for (int t = 0; t < n / 2; ++t) {
-            const double keep = up ? v[t + n / 2] : v[t], pass = up ? v[t] : v[t + n / 2];
-            v[t] = keep + __shfl_xor(pass, o);
-        }
-    }
+    halve<N, 32, N>(v);
     if (N == 32) v[0] += __shfl_xor(v[0], 1);
     return v[0];
 }
 
 // partial[b][ma][mb] = sum over rows of block b of A[:, i] * B[:, j] (8 x NJ tile per
-// blockIdx.y). The tile's reduction over the lanes bounds it at one or two rows a
-// thread: 24 x 4 columns of 152,000 rows took 34 us with 64 shuffle trees and take 10 with
-// the halving sum of 32 values (the same bits). With gate0 set the launch is the second
-// Gram-Schmidt pass and does nothing when the first pass sufficed.
+// blockIdx.y). At one or two rows a thread its time is the loads' latency and the
+// tile's reduction over the lanes: every load is unconditional (columns past the tile
+// repeat its last one and are not stored), so that all of a row are in flight together, and
+// the lanes are summed by halving. 24 x 4 columns of 152,000 rows: 34 -> 8 us, the same
+// bits. With gate0 set the launch is the second Gram-Schmidt pass and does nothing when
+// the first pass sufficed.
 template <int NJ>
 __global__ void __launch_bounds__(DT) k_gram(i64 nd, const double *A, i64 lda, int ma, const double *B, i64 ldb,
                                              int mb, double *partial, const double *gate0, const double *gate1) {
@@ -150,9 +155,9 @@ __global__ void __launch_bounds__(DT) k_gram(i64 nd, const double *A, i64 lda, i
     for (i64 r = (i64)blockIdx.x * DT + threadIdx.x; r < nd; r += (i64)gridDim.x * DT) {
         double a[8], b[NJ];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) a[i] = (i < ni) ? A[(i64)(i0 + i) * lda + r] : 0.0;
+        for (int i = 0; i < 8; ++i) a[i] = A[(i64)(i0 + min(i, ni - 1)) * lda + r];
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) b[j] = (j < nj) ? B[(i64)(j0 + j) * ldb + r] : 0.0;
+        for (int j = 0; j < NJ; ++j) b[j] = B[(i64)(j0 + min(j, nj - 1)) * ldb + r];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
@@ -205,11 +210,17 @@ __global__ void k_gemm_sub_rm(i64 nd, const double *V, int m, const double *C, i
     for (i64 r = (i64)blockIdx.x * blockDim.x + threadIdx.x; r < nd; r += (i64)gridDim.x * blockDim.x) {
         for (int j0 = 0; j0 < k; j0 += 8) {
             double acc[8] = {};
-            for (int i = 0; i < m; ++i) {
-                const double v = V[(i64)i * nd + r];
+            for (int i0 = 0; i0 < m; i0 += 8) {
+                double v[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (j0 + j < k) acc[j] += v * C[i * k + j0 + j];
+                for (int u = 0; u < 8; ++u) v[u] = V[(i64)min(i0 + u, m - 1) * nd + r];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i0 + u < m) {
+#pragma unroll
+                        for (int j = 0; j < 8; ++j)
+                            if (j0 + j < k) acc[j] += v[u] * C[(i0 + u) * k + j0 + j];
+                    }
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -218,16 +229,22 @@ __global__ void k_gemm_sub_rm(i64 nd, const double *V, int m, const double *C, i
     }
 }
 
-// T[:, j] = V[:, 0:m] C[:, j], V read once for every 8 columns
+// T[:, j] = V[:, 0:m] C[:, j], V read once for every 8 columns of T, 8 of its own in flight
 __global__ void k_gemm_set(i64 nd, const double *V, i64 ldv, int m, const double *C, int k, double *T, i64 ldt) {
     for (i64 r = (i64)blockIdx.x * blockDim.x + threadIdx.x; r < nd; r += (i64)gridDim.x * blockDim.x) {
         for (int j0 = 0; j0 < k; j0 += 8) {
             double acc[8] = {};
-            for (int i = 0; i < m; ++i) {
-                const double v = V[(i64)i * ldv + r];
+            for (int i0 = 0; i0 < m; i0 += 8) {
+                double v[8];
 #pragma unroll
-                for (int j = 0; j < 8; ++j)
-                    if (j0 + j < k) acc[j] += v * C[(j0 + j) * m + i];
+                for (int u = 0; u < 8; ++u) v[u] = V[(i64)min(i0 + u, m - 1) * ldv + r];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i0 + u < m) {
+#pragma unroll
+                        for (int j = 0; j < 8; ++j)
+                            if (j0 + j < k) acc[j] += v[u] * C[(j0 + j) * m + i0 + u];
+                    }
             }
 #pragma unroll
             for (int j = 0; j < 8; ++j)
@@ -614,14 +631,25 @@ __global__ void __launch_bounds__(DT) k_ritz(i64 nd, const double *V, const doub
         double x[16], w[16];
 #pragma unroll
         for (int j = 0; j < 16; ++j) x[j] = w[j] = 0.0;
-        for (int i = 0; i < m; ++i) {
-            const double v = V[(i64)i * ld + r], ww = W[(i64)i * ld + r];
+        // four columns' loads in flight at once, added in their order
+        for (int i0 = 0; i0 < m; i0 += 4) {
+            double v[4], ww[4];
 #pragma unroll
-            for (int j = 0; j < 16; ++j)
-                if (j < k) {
-                    const double y = Y[j * m + i];
-                    x[j] += v * y;
-                    w[j] += ww * y;
+            for (int u = 0; u < 4; ++u) {
+                const i64 i = min(i0 + u, m - 1);
+                v[u] = V[i * ld + r];
+                ww[u] = W[i * ld + r];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                if (i0 + u < m) {
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        if (j < k) {
+                            const double y = Y[j * m + i0 + u];
+                            x[j] += v[u] * y;
+                            w[j] += ww[u] * y;
+                        }
                 }
         }
         const double d = diag[r];
