@@ -232,7 +232,7 @@ struct pyci_mlp {
     // workspaces (grown on demand)
     pe::i64 cap = 0;           // rows the workspaces hold (multiple of 128)
     pe::DevBuf<uint16_t> x, xt, h1, h1t, h2t, dz2, dz2t, dz1t;
-    pe::DevBuf<float> y, ypart, dy, tgt, wpart, red;
+    pe::DevBuf<float> ypart, dy, tgt, wpart, red;
 };
 
 struct pyci_op {

@@ -14,7 +14,7 @@
 //             z2 = h1 W2   : A = h1  [R][256],  Bt = w2t [256][256]  -> h2t, y partials
 //   backward  dh1 = dz2 W2^T: A = dz2 [R][256], Bt = w2  [256][256]  -> dz1t (ReLU mask)
 //             dW2 = h1^T dz2: A = h1t [256][R], Bt = dz2t [256][R]   (split over samples)
-//             dW1 = x^T dz1 : A = xt  [128][R], Bt = dz1t [256][R]   (rows >= 64 are zero)
+//             dW1 = x^T dz1 : A = xt  [64][R], Bt = dz1t [256][R]    (same launch)
 // All reductions run in a fixed order, so results do not depend on scheduling.
 #include <algorithm>
 #include <cmath>
@@ -64,11 +64,19 @@ struct Epi {
     float *ypart = nullptr;           // L2: [N/64][M]
     const uint16_t *mask_t = nullptr; // BWD1: h1t [n][m], ld = ldt
     float *out = nullptr;             // F32: [split][M][N]
+    const uint16_t *a2 = nullptr, *bt2 = nullptr;  // F32: a second product of m2 rows, same N, K, lda, ldb
+    float *out2 = nullptr;
+    int m2 = 0;
 };
 
-// 256 threads = 4 waves; block tile 128 x 128, wave tile 64 x 64 (2 x 2 MFMA
-// tiles of 32 x 32). Requires M % 128 == 0, N % 128 == 0, K % 16 == 0 and
-// kchunk % 16 == 0 (checked by the host). Fragment layout of
+// 256 threads = 4 waves; block tile 64 x 128, wave tile 32 x 64 (two MFMA tiles of 32 x 32).
+// Requires M % 64 == 0, N % 128 == 0, K % 64 == 0 and kchunk % 64 == 0 (checked by the
+// host). Operands come straight from L2, four k steps ahead: at 8,192 samples a product is
+// 1 GF and its time is how many blocks share it and how long their loads wait. (Tiles
+// of 128 x 128 without the lookahead gave 64-128 blocks on 256 CUs: 18 us for the layer-2
+// products, 2 x 18 for the weight gradients; every element is still summed over k in the
+// same instructions in the same order.) The weight gradients of both layers are one launch:
+// block rows from M / 64 on belong to the second product. Fragment layout of
 // v_mfma_f32_32x32x16_bf16: lane l supplies row (l % 32) of A and column
 // (l % 32) of B with k = 8 (l / 32) + e, e < 8; accumulator register r of lane l
 // holds row 8 (r / 4) + 4 (l / 32) + r % 4, column l % 32.
@@ -77,32 +85,52 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, i64 K, const ui
                                                    const uint16_t *__restrict__ Bt, i64 ldb, i64 kchunk, Epi ep) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 31, hh = lane >> 5;
-    const int m0 = blockIdx.x * 128 + (wave >> 1) * 64;
+    int m0 = blockIdx.x * 64 + (wave >> 1) * 32;
     const int n0 = blockIdx.y * 128 + (wave & 1) * 64;
+    float *out = ep.out;
+    if (MODE == EPI_F32 && (int)blockIdx.x * 64 >= M) {
+        m0 -= M;
+        M = ep.m2;
+        A = ep.a2;
+        Bt = ep.bt2;
+        out = ep.out2;
+    }
     const i64 kb = (i64)blockIdx.z * kchunk;
     const i64 ke = (kb + kchunk < K) ? kb + kchunk : K;
     const uint16_t *a0 = A + (i64)(m0 + r) * lda + 8 * hh;
-    const uint16_t *a1 = a0 + 32 * lda;
     const uint16_t *b0 = Bt + (i64)(n0 + r) * ldb + 8 * hh;
     const uint16_t *b1 = b0 + 32 * ldb;
-    f32x16 c[2][2];
+    f32x16 c[1][2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int j = 0; j < 2; ++j) c[0][j] = f32x16{};
+    bf16x8 fa[4], fb0[4], fb1[4];
 #pragma unroll
-        for (int j = 0; j < 2; ++j) c[i][j] = f32x16{};
-#pragma unroll 2
-    for (i64 k = kb; k < ke; k += 16) {
-        const bf16x8 fa0 = ld_frag(a0 + k), fa1 = ld_frag(a1 + k);
-        const bf16x8 fb0 = ld_frag(b0 + k), fb1 = ld_frag(b1 + k);
-        c[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa0, fb0, c[0][0], 0, 0, 0);
-        c[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa0, fb1, c[0][1], 0, 0, 0);
-        c[1][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa1, fb0, c[1][0], 0, 0, 0);
-        c[1][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa1, fb1, c[1][1], 0, 0, 0);
+    for (int u = 0; u < 4; ++u) {
+        fa[u] = ld_frag(a0 + kb + 16 * u);
+        fb0[u] = ld_frag(b0 + kb + 16 * u);
+        fb1[u] = ld_frag(b1 + kb + 16 * u);
+    }
+    for (i64 k = kb; k < ke; k += 64) {
+        const i64 kn = k + 64 < ke ? k + 64 : kb;
+        bf16x8 na[4], nb0[4], nb1[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            na[u] = ld_frag(a0 + kn + 16 * u);
+            nb0[u] = ld_frag(b0 + kn + 16 * u);
+            nb1[u] = ld_frag(b1 + kn + 16 * u);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            c[0][0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[u], fb0[u], c[0][0], 0, 0, 0);
+            c[0][1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[u], fb1[u], c[0][1], 0, 0, 0);
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) fa[u] = na[u], fb0[u] = nb0[u], fb1[u] = nb1[u];
     }
     if (MODE == EPI_F32) {
-        float *o = ep.out + (i64)blockIdx.z * M * N;
+        float *o = out + (i64)blockIdx.z * M * N;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 1; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -114,7 +142,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, i64 K, const ui
     }
     if (MODE == EPI_L1 || MODE == EPI_BWD1) {
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 1; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) {
                 const int n = n0 + 32 * j + r;
@@ -146,9 +174,9 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, i64 K, const ui
         return;
     }
     // EPI_L2: h2 = bf16(relu(z2 + b2)); partial y over this wave's 64 columns
-    float ysum[2][16];
+    float ysum[1][16];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 1; ++i)
 #pragma unroll
         for (int q = 0; q < 16; ++q) ysum[i][q] = 0.0f;
 #pragma unroll
@@ -156,7 +184,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, i64 K, const ui
         const int n = n0 + 32 * j + r;
         const float b = ep.bias[n], w = ep.w3[n];
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int i = 0; i < 1; ++i)
 #pragma unroll
             for (int g = 0; g < 4; ++g) {
                 const int mb = m0 + 32 * i + 8 * g + 4 * hh;
@@ -177,7 +205,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, i64 K, const ui
     }
     float *yp = ep.ypart + (i64)(n0 >> 6) * M;
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < 1; ++i)
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
             float s = ysum[i][q];
@@ -186,7 +214,7 @@ __global__ void __launch_bounds__(256) k_gemm_bf16(int M, int N, i64 K, const ui
         }
 }
 
-// Features of R samples: x [R][64] and xt [128][R] (bf16 0/1). Sample s < n is
+// Features of R samples: x [R][64] and xt [64][R] (bf16 0/1). Sample s < n is
 // determinant sel(s): s + first when elig == nullptr, otherwise a counter-based
 // draw from the eligible list (with its target copied); rows s >= n are zero.
 __global__ void k_features(int kind, int nbasis, const u64 *__restrict__ dets, int nkey, i64 first, i64 n, i64 R,
@@ -228,77 +256,123 @@ __global__ void k_features(int kind, int nbasis, const u64 *__restrict__ dets, i
     *reinterpret_cast<uint4 *>(x + s * FPAD + 8 * g) = pk;
 }
 
-// y = ((p0 + p1) + p2) + p3 + b3; with targets also dy = 2 (y - t) / n (0 for
-// rows >= n) and the loss sum / n in out[0], db3 = sum dy in out[1]. One block.
-__global__ void __launch_bounds__(1024) k_y_loss(const float *ypart, i64 R, i64 n, const float *params,
-                                                 const float *tgt, float *y, float *dy, float *out) {
-    const float b3 = params[OB3];
-    float ls = 0.0f, ds = 0.0f;
-    for (i64 m = threadIdx.x; m < R; m += 1024) {
-        const float v = ((ypart[m] + ypart[R + m]) + ypart[2 * R + m]) + ypart[3 * R + m] + b3;
-        y[m] = v;
-        if (tgt) {
-            float d = 0.0f;
-            if (m < n) {
-                const float e = v - tgt[m];
-                ls += e * e;
-                d = 2.0f * e / (float)n;
-            }
-            dy[m] = d;
-            ds += d;
-        }
-    }
-    if (!tgt) return;
-    __shared__ float sl[1024], sd[1024];
-    sl[threadIdx.x] = ls;
-    sd[threadIdx.x] = ds;
-    __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) {
-            sl[threadIdx.x] += sl[threadIdx.x + o];
-            sd[threadIdx.x] += sd[threadIdx.x + o];
-        }
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        out[0] = sl[0] / (float)n;
-        out[1] = sd[0];
-    }
+__device__ inline float y_of(const float *ypart, i64 R, i64 m, float b3) {
+    return ((ypart[m] + ypart[R + m]) + ypart[2 * R + m]) + ypart[3 * R + m] + b3;
 }
 
-// dz2 = bf16(dy[m] w3[f] [h2 > 0]) into dz2 [R][256] and dz2t [256][R], via a
-// 64 x 64 LDS transpose. Block (64, 4); grid (R / 64, 256 / 64).
-__global__ void __launch_bounds__(256) k_dz2(const uint16_t *__restrict__ h2t, const float *__restrict__ dy,
-                                             const float *__restrict__ w3, i64 R, uint16_t *__restrict__ dz2,
+__global__ void k_y(const float *ypart, i64 R, i64 n, const float *params, float *y) {
+    const i64 m = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+    if (m < n) y[m] = y_of(ypart, R, m, params[OB3]);
+}
+
+// dy = 2 (y - t) / n (0 for rows >= n) and dz2 = bf16(dy[m] w3[f] [h2 > 0]) into dz2 [R][256]
+// and dz2t [256][R], 64 x 64 per block through LDS, every global access 16 bytes. Grid
+// (R / 64, 256 / 64); the first column of blocks stores dy.
+__global__ void __launch_bounds__(256) k_dz2(const uint16_t *__restrict__ h2t, const float *__restrict__ ypart,
+                                             const float *__restrict__ tgt, const float *__restrict__ params, i64 R,
+                                             i64 n, float *__restrict__ dy, uint16_t *__restrict__ dz2,
                                              uint16_t *__restrict__ dz2t) {
-    __shared__ uint16_t tile[64][65];
+    __shared__ uint16_t tile[64][66];  // [f][m]; an odd number of words a row
+    __shared__ float sd[64];
     const i64 mb = (i64)blockIdx.x * 64;
     const int fb = blockIdx.y * 64;
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const float d = dy[mb + tx];
-    for (int fy = ty; fy < 64; fy += 4) {
-        const int f = fb + fy;
-        const i64 o = (i64)f * R + mb + tx;
-        const uint16_t hv = h2t[o];
-        const uint16_t v = (hv != 0) ? f2bf(d * w3[f]) : (uint16_t)0;
-        dz2t[o] = v;
-        tile[fy][tx] = v;
+    if (threadIdx.x < 64) {
+        const i64 m = mb + threadIdx.x;
+        float d = 0.0f;
+        if (m < n) {
+            const float e = y_of(ypart, R, m, params[OB3]) - tgt[m];
+            d = 2.0f * e / (float)n;
+        }
+        sd[threadIdx.x] = d;
+        if (fb == 0) dy[m] = d;
     }
     __syncthreads();
-    for (int my = ty; my < 64; my += 4) dz2[(mb + my) * HID + fb + tx] = tile[tx][my];
+    const int g = threadIdx.x & 7;
+    for (int f = threadIdx.x >> 3; f < 64; f += 32) {
+        const i64 o = (i64)(fb + f) * R + mb + 8 * g;
+        const uint4 h = *reinterpret_cast<const uint4 *>(h2t + o);
+        const uint32_t hw[4] = {h.x, h.y, h.z, h.w};
+        const float w = params[OW3 + fb + f];
+        uint32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const uint32_t lo = (hw[e] & 0xffffu) ? f2bf(sd[8 * g + 2 * e] * w) : 0u;
+            const uint32_t hi = (hw[e] >> 16) ? f2bf(sd[8 * g + 2 * e + 1] * w) : 0u;
+            v[e] = lo | (hi << 16);
+            *reinterpret_cast<uint32_t *>(&tile[f][8 * g + 2 * e]) = v[e];
+        }
+        *reinterpret_cast<uint4 *>(dz2t + o) = uint4{v[0], v[1], v[2], v[3]};
+    }
+    __syncthreads();
+    for (int m = threadIdx.x >> 3; m < 64; m += 32) {
+        uint32_t v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            v[e] = (uint32_t)tile[8 * g + 2 * e][m] | ((uint32_t)tile[8 * g + 2 * e + 1][m] << 16);
+        *reinterpret_cast<uint4 *>(dz2 + (mb + m) * HID + fb + 8 * g) = uint4{v[0], v[1], v[2], v[3]};
+    }
 }
 
-// out[row] = sum_m X[row][m] (* w[m]); one 256-thread block per row, fixed order.
-__global__ void __launch_bounds__(256) k_rowsum(const uint16_t *__restrict__ X, i64 ld, i64 ncols,
-                                                const float *__restrict__ w, float *__restrict__ out) {
-    const uint16_t *row = X + (i64)blockIdx.x * ld;
+// The sums over samples of one step in one launch, each in a fixed order: blocks 0-767 the
+// bias gradients (rows of dz1t, dz2t) and the output weights' (rows of h2t times dy), block
+// 768 the loss and the output bias gradient (1,024 strided partial sums, then halving).
+__global__ void __launch_bounds__(256) k_sample_sums(const uint16_t *__restrict__ dz1t,
+                                                     const uint16_t *__restrict__ dz2t,
+                                                     const uint16_t *__restrict__ h2t, const float *__restrict__ dy,
+                                                     const float *__restrict__ ypart, const float *__restrict__ tgt,
+                                                     const float *__restrict__ params, i64 R, i64 n, float *grads,
+                                                     float *loss) {
+    __shared__ float sl[1024], sd[1024];
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 3 * HID) {
+        const float b3 = params[OB3];
+        for (int q = tid; q < 1024; q += 256) {
+            float ls = 0.0f, ds = 0.0f;
+            for (i64 m = q; m < R; m += 1024) {
+                const float d = dy[m];
+                if (m < n) {
+                    const float e = y_of(ypart, R, m, b3) - tgt[m];
+                    ls += e * e;
+                }
+                ds += d;
+            }
+            sl[q] = ls;
+            sd[q] = ds;
+        }
+        __syncthreads();
+        for (int o = 512; o > 0; o >>= 1) {
+            for (int q = tid; q < o; q += 256) {
+                sl[q] += sl[q + o];
+                sd[q] += sd[q + o];
+            }
+            __syncthreads();
+        }
+        if (tid == 0) {
+            loss[0] = sl[0] / (float)n;
+            grads[OB3] = sd[0];
+        }
+        return;
+    }
+    const int which = blockIdx.x / HID, f = blockIdx.x - which * HID;
+    const uint16_t *row = (which == 0 ? dz1t : which == 1 ? dz2t : h2t) + (i64)f * R;
+    const float *w = which == 2 ? dy : nullptr;
     float s = 0.0f;
-    for (i64 m = threadIdx.x; m < ncols; m += 256) s += w ? bf2f(row[m]) * w[m] : bf2f(row[m]);
+    for (i64 m = tid; m < R; m += 8 * 256) {  // eight loads in flight, added in order
+        float x[8], wx[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const i64 q = m + u * 256 < R ? m + u * 256 : m;
+            x[u] = bf2f(row[q]);
+            wx[u] = w ? w[q] : 0.0f;
+        }
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (m + u * 256 < R) s += w ? x[u] * wx[u] : x[u];
+    }
     for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    __shared__ float red[4];
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
+    if ((tid & 63) == 0) sl[tid >> 6] = s;
     __syncthreads();
-    if (threadIdx.x == 0) out[blockIdx.x] = ((red[0] + red[1]) + red[2]) + red[3];
+    if (tid == 0) grads[(which == 0 ? OB1 : which == 1 ? OB2 : OW3) + f] = ((sl[0] + sl[1]) + sl[2]) + sl[3];
 }
 
 // dst[i] = sum_z part[z * stride + i], z ascending.
@@ -310,16 +384,37 @@ __global__ void k_sum_splits(const float *part, int nsplit, i64 stride, i64 coun
     dst[i] = s;
 }
 
-__global__ void k_adam(float *p, const float *g, float *m, float *v, i64 n, float lr, float b1, float b2, float eps,
-                       float bc1, float bc2) {
+// One Adam update of every parameter, with the weight gradients summed from their splits (z
+// ascending) and the bf16 operand copies of the new weights.
+__global__ void k_update(float *p, const float *g, const float *part1, const float *part2, int nsplit, float *m,
+                         float *v, float lr, float b1, float b2, float eps, float bc1, float bc2, uint16_t *w1t,
+                         uint16_t *w2t, uint16_t *w2) {
     const i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= n) return;
-    const float gi = g[i];
+    if (i >= NPARAM) return;
+    const bool is1 = i < OB1, is2 = i >= OW2 && i < OB2;
+    float gi;
+    if (is1 || is2) {
+        const float *part = is1 ? part1 + i : part2 + (i - OW2);
+        const i64 stride = is1 ? FPAD * HID : HID * HID;
+        gi = 0.0f;
+        for (int z = 0; z < nsplit; ++z) gi += part[(i64)z * stride];
+    } else {
+        gi = g[i];
+    }
     const float mi = b1 * m[i] + (1.0f - b1) * gi;
     const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
     m[i] = mi;
     v[i] = vi;
-    p[i] -= lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+    const float pn = p[i] - lr * (mi / bc1) / (sqrtf(vi / bc2) + eps);
+    p[i] = pn;
+    if (is2) {
+        const int j = (int)(i - OW2);
+        const uint16_t h = f2bf(pn);
+        w2[j] = h;
+        w2t[(j % HID) * HID + j / HID] = h;
+    } else if (is1) {
+        w1t[(i % HID) * FPAD + i / HID] = f2bf(pn);
+    }
 }
 
 // bf16 operand copies of the weights.
@@ -365,20 +460,18 @@ static void ensure_workspace(pyci_mlp *m, i64 R) {
     hipStream_t s = m->ctx->stream;
     PE_HIP(hipStreamSynchronize(s));
     m->x.alloc((size_t)R * FPAD);
-    m->xt.alloc((size_t)128 * R);
-    PE_HIP(hipMemsetAsync(m->xt.p, 0, sizeof(uint16_t) * 128 * R, s));  // rows >= 64 stay zero
+    m->xt.alloc((size_t)FPAD * R);
     m->h1.alloc((size_t)R * HID);
     m->h1t.alloc((size_t)R * HID);
     m->h2t.alloc((size_t)R * HID);
     m->dz2.alloc((size_t)R * HID);
     m->dz2t.alloc((size_t)R * HID);
     m->dz1t.alloc((size_t)R * HID);
-    m->y.alloc((size_t)R);
     m->ypart.alloc((size_t)4 * R);
     m->dy.alloc((size_t)R);
     m->tgt.alloc((size_t)R);
     const i64 nsplit = (R + KCHUNK - 1) / KCHUNK;
-    m->wpart.alloc((size_t)nsplit * HID * HID);
+    m->wpart.alloc((size_t)nsplit * (HID * HID + FPAD * HID));
     m->red.alloc(8);
     m->cap = R;
 }
@@ -386,11 +479,12 @@ static void ensure_workspace(pyci_mlp *m, i64 R) {
 template <int MODE>
 static void gemm(hipStream_t s, i64 M, i64 N, i64 K, const uint16_t *A, i64 lda, const uint16_t *Bt, i64 ldb,
                  i64 kchunk, const Epi &ep) {
-    PE_REQUIRE(M % 128 == 0 && N % 128 == 0 && K % 16 == 0 && kchunk % 16 == 0 && lda % 8 == 0 && ldb % 8 == 0,
+    PE_REQUIRE(M % 64 == 0 && ep.m2 % 64 == 0 && N % 128 == 0 && K % 64 == 0 && kchunk % 64 == 0 && lda % 8 == 0 &&
+                   ldb % 8 == 0,
                PYCI_EINVAL, "mlp product shape");
     PE_REQUIRE(M < (1LL << 31) && N < (1LL << 31), PYCI_EINVAL, "mlp product too large");
     const unsigned nz = (unsigned)((K + kchunk - 1) / kchunk);
-    dim3 grid((unsigned)(M / 128), (unsigned)(N / 128), nz);
+    dim3 grid((unsigned)((M + ep.m2) / 64), (unsigned)(N / 128), nz);
     k_gemm_bf16<MODE><<<grid, 256, 0, s>>>((int)M, (int)N, K, A, lda, Bt, ldb, kchunk, ep);
     PE_LAUNCH_CHECK();
 }
@@ -415,16 +509,14 @@ static void forward(pyci_mlp *m, i64 R, bool train) {
     gemm<EPI_L2>(s, R, HID, HID, m->h1.p, HID, m->w2t.p, HID, HID, e2);
 }
 
-// Loss and gradient (into m->grads) of the R featurised rows, n of them real,
-// with targets in m->tgt. Returns nothing; the loss is left in m->red[0].
-static void loss_backward(pyci_mlp *m, i64 R, i64 n) {
+// Loss and gradient of the R featurised rows, n of them real, with targets in m->tgt: the
+// bias and output gradients into m->grads, the splits of dW2 and, behind them, of dW1 into
+// m->wpart, the loss into m->red[0]. Returns the number of splits.
+static int loss_backward(pyci_mlp *m, i64 R, i64 n) {
     hipStream_t s = m->ctx->stream;
-    float *g = m->grads.p;
     forward(m, R, true);
-    k_y_loss<<<1, 1024, 0, s>>>(m->ypart.p, R, n, m->params.p, m->tgt.p, m->y.p, m->dy.p, m->red.p);
-    PE_LAUNCH_CHECK();
-    k_dz2<<<dim3((unsigned)(R / 64), HID / 64), 256, 0, s>>>(m->h2t.p, m->dy.p, m->params.p + OW3, R, m->dz2.p,
-                                                            m->dz2t.p);
+    k_dz2<<<dim3((unsigned)(R / 64), HID / 64), 256, 0, s>>>(m->h2t.p, m->ypart.p, m->tgt.p, m->params.p, R, n, m->dy.p,
+                                                            m->dz2.p, m->dz2t.p);
     PE_LAUNCH_CHECK();
     Epi eb;
     eb.ht = m->dz1t.p;
@@ -434,19 +526,15 @@ static void loss_backward(pyci_mlp *m, i64 R, i64 n) {
     const int nsplit = (int)((R + KCHUNK - 1) / KCHUNK);
     Epi ew;
     ew.out = m->wpart.p;
+    ew.a2 = m->xt.p;
+    ew.bt2 = m->dz1t.p;
+    ew.out2 = m->wpart.p + (i64)nsplit * HID * HID;
+    ew.m2 = FPAD;
     gemm<EPI_F32>(s, HID, HID, R, m->h1t.p, R, m->dz2t.p, R, KCHUNK, ew);
-    k_sum_splits<<<grid_for(HID * HID, 256), 256, 0, s>>>(m->wpart.p, nsplit, HID * HID, HID * HID, g + OW2);
+    k_sample_sums<<<3 * HID + 1, 256, 0, s>>>(m->dz1t.p, m->dz2t.p, m->h2t.p, m->dy.p, m->ypart.p, m->tgt.p,
+                                              m->params.p, R, n, m->grads.p, m->red.p);
     PE_LAUNCH_CHECK();
-    gemm<EPI_F32>(s, 128, HID, R, m->xt.p, R, m->dz1t.p, R, KCHUNK, ew);
-    k_sum_splits<<<grid_for(FPAD * HID, 256), 256, 0, s>>>(m->wpart.p, nsplit, 128 * HID, FPAD * HID, g + OW1);
-    PE_LAUNCH_CHECK();
-    k_rowsum<<<HID, 256, 0, s>>>(m->dz1t.p, R, R, nullptr, g + OB1);
-    PE_LAUNCH_CHECK();
-    k_rowsum<<<HID, 256, 0, s>>>(m->dz2t.p, R, R, nullptr, g + OB2);
-    PE_LAUNCH_CHECK();
-    k_rowsum<<<HID, 256, 0, s>>>(m->h2t.p, R, R, m->dy.p, g + OW3);
-    PE_LAUNCH_CHECK();
-    PE_HIP(hipMemcpyAsync(g + OB3, m->red.p + 1, sizeof(float), hipMemcpyDeviceToDevice, s));
+    return nsplit;
 }
 
 static void refresh(pyci_mlp *m) {
@@ -529,9 +617,8 @@ void mlp_predict_device(pyci_mlp *m, int kind, i64 nbasis, const u64 *d_dets, i6
         const i64 cnt = std::min(PRED_CHUNK, n - first), R = round128(cnt);
         featurise(m, kind, nbasis, nkey, d_dets, first, cnt, R, nullptr, 0, 0, nullptr);
         forward(m, R, false);
-        k_y_loss<<<1, 1024, 0, s>>>(m->ypart.p, R, cnt, m->params.p, nullptr, m->y.p, nullptr, nullptr);
+        k_y<<<grid_for(cnt, 256), 256, 0, s>>>(m->ypart.p, R, cnt, m->params.p, d_y + first);
         PE_LAUNCH_CHECK();
-        PE_HIP(hipMemcpyAsync(d_y + first, m->y.p, sizeof(float) * cnt, hipMemcpyDeviceToDevice, s));
     }
 }
 
@@ -559,7 +646,13 @@ float mlp_loss_grad(pyci_mlp *m, int kind, i64 nbasis, i64 n, const u64 *dets, c
     PE_HIP(hipMemsetAsync(m->tgt.p, 0, sizeof(float) * R, s));
     PE_HIP(hipMemcpyAsync(m->tgt.p, target, sizeof(float) * n, hipMemcpyHostToDevice, s));
     featurise(m, kind, nbasis, nkey, dd.p, 0, n, R, nullptr, 0, 0, nullptr);
-    loss_backward(m, R, n);
+    const int nsplit = loss_backward(m, R, n);
+    float *g = m->grads.p;
+    k_sum_splits<<<grid_for(HID * HID, 256), 256, 0, s>>>(m->wpart.p, nsplit, HID * HID, HID * HID, g + OW2);
+    PE_LAUNCH_CHECK();
+    k_sum_splits<<<grid_for(FPAD * HID, 256), 256, 0, s>>>(m->wpart.p + (i64)nsplit * HID * HID, nsplit, FPAD * HID,
+                                                          FPAD * HID, g + OW1);
+    PE_LAUNCH_CHECK();
     float loss = 0.0f;
     PE_HIP(hipMemcpyAsync(&loss, m->red.p, sizeof(float), hipMemcpyDeviceToHost, s));
     PE_HIP(hipMemcpyAsync(grad, m->grads.p, sizeof(float) * NPARAM, hipMemcpyDeviceToHost, s));
@@ -610,13 +703,13 @@ float mlp_train(pyci_mlp *m, const pyci_wfn *wfn, const double *coeffs, double c
     for (i64 t = 0; t < steps; ++t) {
         featurise(m, wfn->kind, wfn->nbasis, nkey, wfn->dets.p, 0, R, R, elig.p, nelig,
                   seed ^ (0xd1b54a32d192ed03ULL * (u64)(m->adam_t + 1)), tall.p);
-        loss_backward(m, R, R);
+        const int nsplit = loss_backward(m, R, R);
         m->adam_t += 1;
         const float bc1 = 1.0f - std::pow(b1, (float)m->adam_t), bc2 = 1.0f - std::pow(b2, (float)m->adam_t);
-        k_adam<<<grid_for(NPARAM, 256), 256, 0, s>>>(m->params.p, m->grads.p, m->adam_m.p, m->adam_v.p, NPARAM,
-                                                     (float)lr, b1, b2, 1e-8f, bc1, bc2);
+        k_update<<<grid_for(NPARAM, 256), 256, 0, s>>>(
+            m->params.p, m->grads.p, m->wpart.p + (i64)nsplit * HID * HID, m->wpart.p, nsplit, m->adam_m.p, m->adam_v.p,
+            (float)lr, b1, b2, 1e-8f, bc1, bc2, m->w1t.p, m->w2t.p, m->w2.p);
         PE_LAUNCH_CHECK();
-        refresh(m);
     }
     float loss = 0.0f;
     PE_HIP(hipMemcpyAsync(&loss, m->red.p, sizeof(float), hipMemcpyDeviceToHost, s));
