@@ -1114,6 +1114,11 @@ static bool pairs_pay(int kind, const pyci_wfn *wfn, const SetTraits &t, i64 nr,
     return ncol < 28 * exc;
 }
 
+bool pairs_serve(const pyci_wfn *wfn) {
+    if (wfn->kind == PYCI_WFN_DOCI || wfn->colex || wfn->ndet < 1) return false;
+    return pairs_pay(wfn->kind, wfn, set_traits(wfn, wfn->ctx->stream), wfn->ndet, wfn->ndet);
+}
+
 void build_rows(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn, i64 row0, i64 row1, i64 ncol,
                 DevBuf<i64> &rowptr_seg, DevBuf<int32_t> &cols, DevBuf<double> &vals, DevBuf<i64> &lowcnt_seg,
                 DevBuf<double> &diag_seg, i64 &nnz_seg, i64 &low_total) {

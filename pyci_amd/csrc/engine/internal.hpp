@@ -434,6 +434,8 @@ i64 exclusive_scan(pyci_ctx *ctx, i64 *d_data, i64 n);
 void build_rows(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn, i64 row0, i64 row1, i64 ncol,
                 DevBuf<i64> &rowptr_seg, DevBuf<int32_t> &cols, DevBuf<double> &vals, DevBuf<i64> &lowcnt_seg,
                 DevBuf<double> &diag_seg, i64 &nnz_seg, i64 &low_total);
+// whether testing pairs of determinants is the way to the connections of a hashed set
+bool pairs_serve(const pyci_wfn *wfn);
 // SpMM (sigma.hip): Y = A X, X ncol x nvec row-major, Y nrow x nvec row-major
 // sector = +1 / -1: the vectors lie in that parity sector of the alpha <-> beta
 // exchange (a hint the matrix-free operator uses; 0 = any vectors)

@@ -15,6 +15,7 @@
 #include <algorithm>
 
 #include "internal.hpp"
+#include "rdm.hpp"
 
 namespace pe {
 
@@ -496,8 +497,225 @@ void trdms_device(pyci_wfn *w1, pyci_wfn *w2, const double *c1_host, const doubl
     PE_HIP(hipStreamSynchronize(s));
 }
 
+// ---------------------------------------------------------------------------
+// Selected FullCI and GenCI sets: the connected pairs of determinants by testing every pair
+// (k_pair_rows of csr_build.hip has the same scan), each pair J > I once, into
+// the compact accumulators of rdm.hpp, whose images k_rf_expand forms. k_rdm hashes and
+// probes every excitation of every row, and adds each image of an element with an
+// atomic of its own.
+// ---------------------------------------------------------------------------
+constexpr int RP_ROWS = 8;
+constexpr int RP_COLS = 4096;
+
+template <int KIND>
+__global__ void __launch_bounds__(256) k_rdm_pairs(WfnView w, RfShape S, const double *__restrict__ c, i64 seglen,
+                                                   int R, double *__restrict__ acc) {
+    constexpr int NW = KIND == PYCI_WFN_FULLCI ? 2 : 1;
+    __shared__ u64 hits[4][RP_ROWS][64];
+    __shared__ int qcol[4][128];
+    __shared__ unsigned char qrow[4][128];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const i64 ngroup = (w.ndet + RP_ROWS - 1) / RP_ROWS, group = (i64)blockIdx.x * 4 + wave;
+    if (group >= ngroup) return;  // uniform per wavefront; no block barriers below
+    const int nrows = (int)((w.ndet - group + ngroup - 1) / ngroup), n = S.n, npd = S.npd;
+    const i64 cbeg = (i64)blockIdx.y * seglen, cend = min(w.ndet, cbeg + seglen);
+    double *base_acc = acc + (i64)((blockIdx.x + blockIdx.y) % R) * S.stride;
+    u64 ra[RP_ROWS], rb[RP_ROWS];
+#pragma unroll
+    for (int r = 0; r < RP_ROWS; ++r) {
+        const i64 row = min(group + r * ngroup, w.ndet - 1);
+        ra[r] = w.dets[NW * row];
+        rb[r] = NW == 2 ? w.dets[NW * row + NW - 1] : 0ULL;
+    }
+    auto pair = [](int p, int q) { return p < q ? q * (q - 1) / 2 + p : p * (p - 1) / 2 + q; };
+    auto emit = [&](int at) {
+        const i64 col = qcol[wave][at], row = group + (i64)qrow[wave][at] * ngroup;
+        const u64 up = w.dets[NW * row], dn = NW == 2 ? w.dets[NW * row + NW - 1] : 0ULL;
+        const u64 cu = w.dets[NW * col], cd = NW == 2 ? w.dets[NW * col + NW - 1] : 0ULL;
+        const u64 hu = up & ~cu, pu = cu & ~up, hd = dn & ~cd, pd = cd & ~dn;
+        const int nu = __popcll(hu), nd = __popcll(hd);
+        const double cc = c[row] * c[col];
+        if (nu == 1 && nd == 1) {
+            const int i = __builtin_ctzll(hu), a = __builtin_ctzll(pu), k = __builtin_ctzll(hd), l = __builtin_ctzll(pd);
+            const double v = cc * (double)(phase1(up, i, a) * phase1(dn, k, l));
+            // abab[i,k,a,l] = abab[a,l,i,k], held with the beta pair in order
+            const i64 pr = k < l ? (i64)(i * n + a) * S.npr + l * (l + 1) / 2 + k
+                                 : (i64)(a * n + i) * S.npr + k * (k + 1) / 2 + l;
+            aadd(&base_acc[S.oab + pr], v);
+            return;
+        }
+        const bool beta = nu == 0;
+        const u64 d = beta ? dn : up, h = beta ? hd : hu, p = beta ? pd : pu;
+        double *one = base_acc + (beta ? n * n : 0), *two = base_acc + (beta ? S.obb : S.oaa);
+        const int i = __builtin_ctzll(h), a = __builtin_ctzll(p);
+        const u64 h2 = h & (h - 1), p2 = p & (p - 1);
+        if (h2) {
+            const int k = __builtin_ctzll(h2), l = __builtin_ctzll(p2);
+            aadd(&two[(i64)pair(i, k) * npd + pair(a, l)], cc * phase2(d, i, k, a, l));
+            return;
+        }
+        const double v = cc * phase1(d, i, a);
+        aadd(&one[i * n + a], v);
+        for (u64 x = d; x; x &= x - 1) {
+            const int q = __builtin_ctzll(x);
+            if (q == i) continue;
+            aadd(&two[(i64)pair(i, q) * npd + pair(a, q)], (i < q) != (a < q) ? -v : v);
+        }
+        if constexpr (KIND == PYCI_WFN_FULLCI) {
+            if (beta) {
+                const int s = max(i, a), t = min(i, a);
+                for (u64 x = up; x; x &= x - 1) {
+                    const int q = __builtin_ctzll(x);
+                    aadd(&base_acc[S.oab + (i64)(q * n + q) * S.npr + s * (s + 1) / 2 + t], v);
+                }
+            } else {
+                for (u64 x = dn; x; x &= x - 1) {
+                    const int q = __builtin_ctzll(x), qq = q * (q + 1) / 2 + q;
+                    aadd(&base_acc[S.oab + (i64)(i * n + a) * S.npr + qq], v);
+                    aadd(&base_acc[S.oab + (i64)(a * n + i) * S.npr + qq], v);
+                }
+            }
+        }
+    };
+    auto settle = [] {
+        __builtin_amdgcn_wave_barrier();
+        asm volatile("" ::: "memory");
+    };
+    int qn = 0;
+    for (i64 base = cbeg; base < cend; base += RP_COLS) {
+        if (base + RP_COLS - 1 <= group) continue;  // no column beyond the first row
+        const int nch = (int)min((i64)(RP_COLS / 64), (cend - base + 63) / 64);
+        u64 mk[RP_ROWS] = {};
+        auto fetch = [&](int t, u64 &a, u64 &b) {
+            const i64 col = min(base + t * 64 + lane, cend - 1);
+            a = w.dets[NW * col];
+            b = NW == 2 ? w.dets[NW * col + NW - 1] : 0ULL;
+        };
+        u64 a, b, an, bn;
+        fetch(0, a, b);
+        for (int t = 0; t < nch; ++t) {
+            fetch(min(t + 1, nch - 1), an, bn);
+            const u64 valid = __ballot(base + t * 64 + lane < cend);
+#pragma unroll
+            for (int r = 0; r < RP_ROWS; ++r) {
+                int d = __popcll(a ^ ra[r]);
+                if (NW == 2) d += __popcll(b ^ rb[r]);
+                const u64 h = __ballot(d <= 4) & valid;
+                mk[r] = lane == t ? h : mk[r];
+            }
+            a = an, b = bn;
+        }
+#pragma unroll
+        for (int r = 0; r < RP_ROWS; ++r) hits[wave][r][lane] = mk[r];
+        settle();
+        for (int r = 0; r < nrows; ++r) {
+            u64 m = hits[wave][r][lane];
+            // columns beyond the row only
+            const i64 first = group + r * ngroup + 1 - (base + lane * 64);
+            if (first > 0) m = first >= 64 ? 0ULL : m & (~0ULL << first);
+            for (u64 act = __ballot(m != 0); act; act = __ballot(m != 0)) {
+                if (m) {
+                    const int slot = qn + __popcll(act & ((1ULL << lane) - 1ULL));
+                    qcol[wave][slot] = (int)base + lane * 64 + __builtin_ctzll(m);
+                    qrow[wave][slot] = (unsigned char)r;
+                    m &= m - 1;
+                }
+                qn += __popcll(act);
+                if (qn >= 64) {
+                    settle();
+                    qn -= 64;
+                    emit(qn + lane);
+                    settle();
+                }
+            }
+        }
+        settle();
+    }
+    if (lane < qn) emit(lane);
+}
+
+// The diagonal terms c_I^2 of the same accumulators: summed over a block's determinants in
+// LDS first, because every determinant adds to the elements of the common orbitals.
+template <int KIND>
+__global__ void __launch_bounds__(256) k_rdm_diagonal(WfnView w, RfShape S, const double *__restrict__ c, int R,
+                                                      double *__restrict__ acc) {
+    constexpr int NW = KIND == PYCI_WFN_FULLCI ? 2 : 1;
+    extern __shared__ double sums[];  // per string: n orbitals, npd pairs; FullCI: n x n mixed
+    const int n = S.n, per = n + S.npd, total = NW * per + (NW == 2 ? n * n : 0);
+    for (int t = threadIdx.x; t < total; t += 256) sums[t] = 0.0;
+    __syncthreads();
+    for (i64 row = (i64)blockIdx.x * 256 + threadIdx.x; row < w.ndet; row += (i64)gridDim.x * 256) {
+        const double v = c[row] * c[row];
+        for (int s = 0; s < NW; ++s) {
+            const u64 d = w.dets[NW * row + s];
+            for (u64 x = d; x; x &= x - 1) {
+                const int p = __builtin_ctzll(x);
+                atomicAdd(&sums[s * per + p], v);
+                for (u64 y = x & (x - 1); y; y &= y - 1) {
+                    const int q = __builtin_ctzll(y);
+                    atomicAdd(&sums[s * per + n + q * (q - 1) / 2 + p], v);
+                }
+                if (NW == 2 && s == 0)
+                    for (u64 y = w.dets[NW * row + 1]; y; y &= y - 1)
+                        atomicAdd(&sums[NW * per + p * n + __builtin_ctzll(y)], v);
+            }
+        }
+    }
+    __syncthreads();
+    double *base = acc + (i64)(blockIdx.x % R) * S.stride;
+    for (int t = threadIdx.x; t < total; t += 256) {
+        const double v = sums[t];
+        if (v == 0.0) continue;
+        const int s = t / per, u = t - s * per;
+        if (t >= NW * per) {
+            const int m = t - NW * per, p = m / n, q = m - p * n;
+            aadd(&base[S.oab + (i64)(p * n + p) * S.npr + q * (q + 1) / 2 + q], v);
+        } else if (u < n) {
+            aadd(&base[s * n * n + u * n + u], v);
+        } else {
+            aadd(&base[(s ? S.obb : S.oaa) + (i64)(u - n) * S.npd + (u - n)], v);
+        }
+    }
+}
+
+// Sums of up to 62 FullCI orbitals fit the 64 KB of k_rdm_diagonal.
+static bool rdms_pairs(pyci_wfn *wfn, const double *coeffs_host, double *rdm1, double *rdm2) {
+    if (wfn->kind == PYCI_WFN_DOCI || (wfn->kind == PYCI_WFN_FULLCI && wfn->nbasis > 60) || !pairs_serve(wfn))
+        return false;
+    hipStream_t s = wfn->ctx->stream;
+    const RfShape S = rf_shape(wfn);
+    const int R = rf_copies(S);
+    const i64 nd = wfn->ndet, nacc = R * S.stride;
+    DevBuf<double> buf((size_t)(nacc + nd));
+    double *acc = buf.p, *c = acc + nacc;
+    PE_HIP(hipMemsetAsync(acc, 0, sizeof(double) * nacc, s));
+    PE_HIP(hipMemcpyAsync(c, coeffs_host, sizeof(double) * nd, hipMemcpyHostToDevice, s));
+    const WfnView w = view_of(wfn);
+    const i64 groups = (nd + RP_ROWS - 1) / RP_ROWS;
+    // split as in build_rows_pairs
+    const i64 most = (nd + RP_COLS - 1) / RP_COLS, even = std::min<i64>(16, (nd + 8191) / 8192);
+    const i64 want = std::max<i64>(1, std::min(std::max((4096 + groups - 1) / groups, even), most));
+    const i64 seglen = ((nd + want - 1) / want + RP_COLS - 1) / RP_COLS * RP_COLS;
+    const dim3 grid((unsigned)((groups + 3) / 4), (unsigned)((nd + seglen - 1) / seglen));
+    const bool two = wfn->kind == PYCI_WFN_FULLCI;
+    const size_t lds = sizeof(double) * (size_t)((two ? 2 : 1) * (S.n + S.npd) + (two ? S.n * S.n : 0));
+    const unsigned dg = (unsigned)std::min<i64>(256, (nd + 255) / 256);
+    if (two) {
+        k_rdm_diagonal<PYCI_WFN_FULLCI><<<dg, 256, lds, s>>>(w, S, c, R, acc);
+        PE_LAUNCH_CHECK();
+        k_rdm_pairs<PYCI_WFN_FULLCI><<<grid, 256, 0, s>>>(w, S, c, seglen, R, acc);
+    } else {
+        k_rdm_diagonal<PYCI_WFN_GENCI><<<dg, 256, lds, s>>>(w, S, c, R, acc);
+        PE_LAUNCH_CHECK();
+        k_rdm_pairs<PYCI_WFN_GENCI><<<grid, 256, 0, s>>>(w, S, c, seglen, R, acc);
+    }
+    PE_LAUNCH_CHECK();
+    rf_result(wfn->ctx, S, R, acc, rdm1, rdm2);
+    return true;
+}
+
 void rdms_device(pyci_wfn *wfn, const double *coeffs_host, double *rdm1, double *rdm2) {
-    if (rdms_full_space(wfn, coeffs_host, rdm1, rdm2)) return;
+    if (rdms_full_space(wfn, coeffs_host, rdm1, rdm2) || rdms_pairs(wfn, coeffs_host, rdm1, rdm2)) return;
     hipStream_t s = wfn->ctx->stream;
     const i64 n = wfn->nbasis, n2 = n * n, n4 = n2 * n2;
     i64 s1, s2;

@@ -19,6 +19,7 @@
 #include <cmath>
 
 #include "internal.hpp"
+#include "rdm.hpp"
 
 namespace pe {
 
@@ -27,17 +28,6 @@ typedef double f64x4 __attribute__((ext_vector_type(4)));
 __device__ inline f64x4 mfma4(double a, double b, f64x4 c) {
     return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
-
-// Sizes and the layout of one accumulator copy: a1, b1 (n x n, single excitations one
-// way round), caa, cbb (pairs p < q by pairs r < s, each connected pair of strings
-// once), cab (n x n by pairs q <= s).
-struct RfShape {
-    int n, nup, ndn, na, nb;
-    int ldc, ldt;  // row strides of C and C^T: string counts rounded up to 16, padding zero
-    int npd, npr;  // pairs p < q, pairs q <= s
-    const i64 *binom;
-    i64 oaa, obb, oab, stride;
-};
 
 __device__ inline u64 rf_string(int r, int n, int k, const i64 *binom) {
     u64 s = 0;
@@ -299,19 +289,20 @@ __global__ void __launch_bounds__(256) k_rf_abab(RfShape S, const double *__rest
     }
 }
 
-// The reference's arrays (rdm1: aa, bb; rdm2: aaaa, bbbb, abab) from the accumulators.
+// The reference's arrays from the accumulators (FullCI: rdm1 aa, bb; rdm2 aaaa, bbbb, abab;
+// GenCI: rdm1, rdm2 of the one string).
 __global__ void k_rf_expand(RfShape S, int R, const double *__restrict__ acc, double *__restrict__ out) {
-    const i64 n = S.n, n2 = n * n, n4 = n2 * n2;
+    const i64 n = S.n, n2 = n * n, n4 = n2 * n2, none = (S.genci ? 1 : 2) * n2;
     const i64 t = (i64)blockIdx.x * 256 + threadIdx.x;
-    if (t >= 2 * n2 + 3 * n4) return;
+    if (t >= none + (S.genci ? 1 : 3) * n4) return;
     i64 at0, at1 = -1;
     double sign = 1.0;
-    if (t < 2 * n2) {
+    if (t < none) {
         const i64 x = t % n2, p = x / n, q = x - p * n;
         at0 = t;
         if (p != q) at1 = t - x + q * n + p;
     } else {
-        const i64 u = t - 2 * n2, blk = u / n4, x = u - blk * n4;
+        const i64 u = t - none, blk = u / n4, x = u - blk * n4;
         int p = (int)(x / (n2 * n)), q = (int)(x / n2 % n), r = (int)(x / n % n), s = (int)(x % n);
         if (blk < 2) {
             if (p == q || r == s) {
@@ -346,6 +337,50 @@ __global__ void k_rf_expand(RfShape S, int R, const double *__restrict__ acc, do
     out[t] = sign * v;
 }
 
+// Fills the sizes and the accumulator layout; C's strides are the full-space contractions' own.
+RfShape rf_shape(const pyci_wfn *w) {
+    RfShape S{};
+    S.n = (int)w->nbasis, S.nup = (int)w->nup, S.ndn = (int)w->ndn;
+    S.genci = w->kind == PYCI_WFN_GENCI;
+    S.npd = S.n * (S.n - 1) / 2, S.npr = S.n * (S.n + 1) / 2;
+    S.binom = w->ctx->binom.p;
+    const i64 n2 = (i64)S.n * S.n, npd2 = (i64)S.npd * S.npd;
+    S.oaa = S.genci ? n2 : 2 * n2, S.obb = S.oaa + npd2;
+    S.oab = S.genci ? S.obb : S.obb + npd2;
+    S.stride = S.genci ? S.obb : S.oab + n2 * S.npr;
+    return S;
+}
+
+int rf_copies(const RfShape &S) {
+    return (int)std::max<i64>(1, std::min<i64>(4, ((i64)256 << 20) / (S.stride * 8)));
+}
+
+// Expands the accumulators and brings the result to the caller: straight into page-locked memory
+// of the context (one synchronisation and no staged copies); beyond 16 MB (FullCI nbasis
+// 29, GenCI 38) through device memory.
+void rf_result(pyci_ctx *ctx, const RfShape &S, int R, const double *acc, double *rdm1, double *rdm2) {
+    hipStream_t s = ctx->stream;
+    const i64 n2 = (i64)S.n * S.n, s1 = (S.genci ? 1 : 2) * n2, nout = s1 + (S.genci ? 1 : 3) * n2 * n2;
+    const bool direct = nout <= (i64)2 << 20;
+    DevBuf<double> dout;
+    HostBuf<double> &host = ctx->rdm_out;
+    if (direct)
+        host.ensure((size_t)nout);
+    else
+        dout.alloc((size_t)nout);
+    k_rf_expand<<<grid_for(nout, 256), 256, 0, s>>>(S, R, acc, direct ? host.p : dout.p);
+    PE_LAUNCH_CHECK();
+    if (direct) {
+        PE_HIP(hipStreamSynchronize(s));
+        std::copy(host.p, host.p + s1, rdm1);
+        std::copy(host.p + s1, host.p + nout, rdm2);
+    } else {
+        PE_HIP(hipMemcpyAsync(rdm1, dout.p, sizeof(double) * s1, hipMemcpyDeviceToHost, s));
+        PE_HIP(hipMemcpyAsync(rdm2, dout.p + s1, sizeof(double) * (nout - s1), hipMemcpyDeviceToHost, s));
+        PE_HIP(hipStreamSynchronize(s));
+    }
+}
+
 template <int MT>
 static void launch_abab(int nt, dim3 grid, size_t lds, hipStream_t s, const RfShape &S, const double *C,
                         const uint16_t *tab, int nchunk, int R, double *acc) {
@@ -376,22 +411,17 @@ static bool full_rdm_applies(const pyci_wfn *w) {
 bool rdms_full_space(pyci_wfn *w, const double *coeffs_host, double *rdm1, double *rdm2) {
     if (!full_rdm_applies(w)) return false;
     hipStream_t s = w->ctx->stream;
-    RfShape S;
-    S.n = (int)w->nbasis, S.nup = (int)w->nup, S.ndn = (int)w->ndn;
+    RfShape S = rf_shape(w);
     S.na = (int)binom_host(S.n, S.nup), S.nb = (int)binom_host(S.n, S.ndn);
     S.ldc = (S.nb + 15) & ~15, S.ldt = (S.na + 15) & ~15;
-    S.npd = S.n * (S.n - 1) / 2, S.npr = S.n * (S.n + 1) / 2;
-    S.binom = w->ctx->binom.p;
-    const i64 n2 = (i64)S.n * S.n, n4 = n2 * n2, npd2 = (i64)S.npd * S.npd;
-    S.oaa = 2 * n2, S.obb = S.oaa + npd2, S.oab = S.obb + npd2, S.stride = S.oab + n2 * S.npr;
-    const int R = (int)std::max<i64>(1, std::min<i64>(4, ((i64)256 << 20) / (S.stride * 8)));
+    const int R = rf_copies(S);
     // the rows and pairs of k_rf_abab in equal chunks of at most 3 and 5 tiles
     const int mtiles = (S.nup * (S.n - S.nup + 1) + 15) / 16, ntiles = (S.npr + 15) / 16;
     const int mch = (mtiles + 2) / 3, nch = (ntiles + 4) / 5;
     const int MT = (mtiles + mch - 1) / mch, NT = (ntiles + nch - 1) / nch;
     const int trows = nch * NT * 16;
     const i64 nC = (i64)S.na * S.ldc, nCt = (i64)S.nb * S.ldt, nga = (i64)S.na * S.na, ngb = (i64)S.nb * S.nb;
-    const i64 nout = 2 * n2 + 3 * n4, ntab = ((i64)trows * S.ldc + 3) / 4;
+    const i64 ntab = ((i64)trows * S.ldc + 3) / 4;
     // one allocation: the vector, C and C^T, gamma of both spins, the table, the accumulators
     const i64 nacc = R * S.stride, even = (w->ndet + 1) & ~(i64)1;
     DevBuf<double> buf((size_t)(even + nC + nCt + nga + ngb + ntab + nacc));
@@ -417,26 +447,7 @@ bool rdms_full_space(pyci_wfn *w, const double *coeffs_host, double *rdm1, doubl
         launch_abab<2>(NT, grid, lds, s, S, C, tab, nch, R, acc);
     else
         launch_abab<3>(NT, grid, lds, s, S, C, tab, nch, R, acc);
-    // the result goes straight into page-locked memory of the context (one synchronisation
-    // and no staged copies); beyond 16 MB (nbasis 29) it is copied from device memory
-    const bool direct = nout <= (i64)2 << 20;
-    DevBuf<double> dout;
-    HostBuf<double> &host = w->ctx->rdm_out;
-    if (direct)
-        host.ensure((size_t)nout);
-    else
-        dout.alloc((size_t)nout);
-    k_rf_expand<<<grid_for(nout, 256), 256, 0, s>>>(S, R, acc, direct ? host.p : dout.p);
-    PE_LAUNCH_CHECK();
-    if (direct) {
-        PE_HIP(hipStreamSynchronize(s));
-        std::copy(host.p, host.p + 2 * n2, rdm1);
-        std::copy(host.p + 2 * n2, host.p + nout, rdm2);
-    } else {
-        PE_HIP(hipMemcpyAsync(rdm1, dout.p, sizeof(double) * 2 * n2, hipMemcpyDeviceToHost, s));
-        PE_HIP(hipMemcpyAsync(rdm2, dout.p + 2 * n2, sizeof(double) * 3 * n4, hipMemcpyDeviceToHost, s));
-        PE_HIP(hipStreamSynchronize(s));
-    }
+    rf_result(w->ctx, S, R, acc, rdm1, rdm2);
     double trace = 0.0;  // a sum of every squared coefficient
     for (i64 p = 0; p < S.n; ++p) trace += rdm1[p * (S.n + 1)];
     return std::isfinite(trace);
