@@ -72,7 +72,7 @@ struct BView {
     const i64 *row_first;    // row block -> first row
     const int *col_blk;      // sigma column block -> problem (256 columns)
     const i64 *col_first;
-    const int *tile_blk;     // product tile -> problem (128 columns)
+    const int *tile_blk;     // product tile -> problem (64 columns)
     const i64 *tile_first;
     const int2 *tab;
     const double *V64p;
@@ -93,26 +93,52 @@ struct BView {
 };
 
 // ---------------------------------------------------------------------------
-// Rayleigh-Ritz: cyclic Jacobi of G (m x m) in LDS, one 64-thread workgroup per
-// problem. Decides the restart (m + k > mmax) and the number of Ritz vectors kk.
+// Rayleigh-Ritz: cyclic Jacobi of G (m x m) in LDS, one workgroup per problem. Decides the
+// restart (m + k > mmax) and the number of Ritz vectors kk. A sweep goes in rounds of m / 2
+// disjoint pairs (the round-robin tournament), whose rotations are taken together: the chain
+// of divisions and square roots is walked once a round instead of once a pair. One wave for
+// m <= 16 (its barriers are free), four above. m = 10, one pair at a time -> in rounds:
+// 125 -> 35 us.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_bjac(BView b) {
+template <int BT>
+__global__ void __launch_bounds__(BT) k_bjac(BView b) {
     const int p = blockIdx.x, t = threadIdx.x;
     int *st = b.st + p * ST;
     if (!st[S_ACTIVE]) return;
     const int m = st[S_M], k = b.k, mmax = b.mmax;
     __shared__ double a[BM_MAX][BM_MAX + 1], v[BM_MAX][BM_MAX + 1];
+    __shared__ double rc[BM_MAX / 2], rs[BM_MAX / 2];
+    __shared__ int rp[BM_MAX / 2], rq[BM_MAX / 2];
     __shared__ int order[BM_MAX];
     const double *G = b.G + (i64)p * BM_MAX * BM_MAX;
-    for (int idx = t; idx < m * m; idx += 64) {
-        const int i = idx / m, j = idx % m;
-        a[i][j] = G[i * BM_MAX + j];
+    // an odd m is padded to 2 h by a row and a column of zeros, which take no rotation
+    const int h = (m + 1) / 2, n1 = 2 * h - 1;
+    for (int idx = t; idx < 4 * h * h; idx += BT) {
+        const int i = idx / (2 * h), j = idx % (2 * h);
+        a[i][j] = (i < m && j < m) ? G[i * BM_MAX + j] : 0.0;
         v[i][j] = (i == j) ? 1.0 : 0.0;
+    }
+    // what this thread rotates each round: the 2 x 2 blocks of a between two pairs, in which
+    // both sides' rotations meet, and the two entries of a row of v in a pair
+    constexpr int NA = (BT == 64) ? 1 : 3, NV = (BT == 64) ? 2 : 5;
+    int ai[NA], aj[NA], vi[NV], vj[NV];
+#pragma unroll
+    for (int u = 0; u < NA; ++u) {
+        const int idx = t + u * BT;
+        ai[u] = (idx < h * h) ? idx / h : -1;
+        aj[u] = idx % h;
+    }
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+        const int idx = t + u * BT;
+        vi[u] = (idx < m * h) ? idx / h : -1;
+        vj[u] = idx % h;
     }
     __syncthreads();
     for (int sweep = 0; sweep < 60; ++sweep) {
+        // every wave sums all of it, so that all take the same decision
         double off = 0.0, tot = 0.0;
-        for (int idx = t; idx < m * m; idx += 64) {
+        for (int idx = t & 63; idx < m * m; idx += 64) {
             const int i = idx / m, j = idx % m;
             const double x = a[i][j] * a[i][j];
             tot += x;
@@ -123,54 +149,70 @@ __global__ void __launch_bounds__(64) k_bjac(BView b) {
             tot += __shfl_xor(tot, o);
         }
         if (off <= 1e-30 * tot || off == 0.0) break;
-        for (int pp = 0; pp < m - 1; ++pp)
-            for (int qq = pp + 1; qq < m; ++qq) {
-                const double apq = a[pp][qq];
-                if (apq == 0.0) continue;
-                const double app = a[pp][pp], aqq = a[qq][qq];
-                const double tau = (aqq - app) / (2.0 * apq);
-                const double tt = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
-                const double c = 1.0 / sqrt(1.0 + tt * tt), s = tt * c;
-                __syncthreads();
-                if (t < m) {
-                    const double arp = a[t][pp], arq = a[t][qq];
-                    a[t][pp] = c * arp - s * arq;
-                    a[t][qq] = s * arp + c * arq;
+        for (int round = 0; round < n1; ++round) {
+            if (t < h) {
+                int x = round + t, y = round - t;
+                if (x >= n1) x -= n1;
+                if (y < 0) y += n1;
+                if (t == 0) x = n1;
+                const int pp = min(x, y), qq = max(x, y);
+                double c = 1.0, s = 0.0;
+                const double apq = a[pp][qq], app = a[pp][pp], aqq = a[qq][qq];
+                if (apq != 0.0) {
+                    const double tau = (aqq - app) / (2.0 * apq);
+                    const double tt = (tau >= 0 ? 1.0 : -1.0) / (fabs(tau) + sqrt(1.0 + tau * tau));
+                    c = rsqrt(1.0 + tt * tt);
+                    s = tt * c;
                 }
-                __syncthreads();
-                if (t < m) {
-                    const double apr = a[pp][t], aqr = a[qq][t];
-                    a[pp][t] = c * apr - s * aqr;
-                    a[qq][t] = s * apr + c * aqr;
-                    const double vrp = v[t][pp], vrq = v[t][qq];
-                    v[t][pp] = c * vrp - s * vrq;
-                    v[t][qq] = s * vrp + c * vrq;
+                rp[t] = pp;
+                rq[t] = qq;
+                rc[t] = c;
+                rs[t] = s;
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < NA; ++u)
+                if (ai[u] >= 0) {
+                    const int p1 = rp[ai[u]], q1 = rq[ai[u]], p2 = rp[aj[u]], q2 = rq[aj[u]];
+                    const double c1 = rc[ai[u]], s1 = rs[ai[u]], c2 = rc[aj[u]], s2 = rs[aj[u]];
+                    const double x = a[p1][p2], y = a[p1][q2], z = a[q1][p2], w = a[q1][q2];
+                    const double pl = c1 * x - s1 * z, pr = c1 * y - s1 * w;
+                    const double ql = s1 * x + c1 * z, qr = s1 * y + c1 * w;
+                    a[p1][p2] = c2 * pl - s2 * pr;
+                    a[p1][q2] = s2 * pl + c2 * pr;
+                    a[q1][p2] = c2 * ql - s2 * qr;
+                    a[q1][q2] = s2 * ql + c2 * qr;
                 }
-                __syncthreads();
-            }
-    }
-    if (t == 0) {
-        for (int i = 0; i < m; ++i) order[i] = i;
-        for (int i = 1; i < m; ++i) {  // stable insertion sort, ascending
-            const int x = order[i];
-            int j = i - 1;
-            while (j >= 0 && a[order[j]][order[j]] > a[x][x]) {
-                order[j + 1] = order[j];
-                --j;
-            }
-            order[j + 1] = x;
+#pragma unroll
+            for (int u = 0; u < NV; ++u)
+                if (vi[u] >= 0) {
+                    const int pp = rp[vj[u]], qq = rq[vj[u]];
+                    const double c = rc[vj[u]], s = rs[vj[u]], x = v[vi[u]][pp], y = v[vi[u]][qq];
+                    v[vi[u]][pp] = c * x - s * y;
+                    v[vi[u]][qq] = s * x + c * y;
+                }
+            __syncthreads();
         }
-        const int restart = (m + k > mmax) ? 1 : 0;
-        int kk = k;
-        if (restart) kk = max(k, min(m, min(2 * k, mmax - k)));
+    }
+    // ascending, equal values in their order; (an order that holds also where a value is NaN)
+    if (t < m) order[t] = t;
+    __syncthreads();
+    if (t < m) {
+        const double x = a[t][t];
+        int rank = 0;
+        for (int j = 0; j < m; ++j) rank += (a[j][j] < x || (a[j][j] == x && j < t)) ? 1 : 0;
+        order[rank] = t;
+    }
+    const int restart = (m + k > mmax) ? 1 : 0;
+    const int kk = restart ? max(k, min(m, min(2 * k, mmax - k))) : k;
+    if (t == 0) {
         st[S_RESTART] = restart;
         st[S_KK] = kk;
     }
     __syncthreads();
-    const int kk = st[S_KK];
     double *th = b.theta + (i64)p * BM_MAX, *Y = b.Y + (i64)p * BM_MAX * 2 * BK_MAX;
-    for (int j = t; j < m; j += 64) th[j] = a[order[j]][order[j]];
-    for (int idx = t; idx < m * kk; idx += 64) {
+    for (int j = t; j < m; j += BT) th[j] = a[order[j]][order[j]];
+    for (int idx = t; idx < m * kk; idx += BT) {
         const int i = idx / kk, j = idx % kk;
         Y[i * 2 * BK_MAX + j] = v[i][order[j]];
     }
@@ -178,8 +220,11 @@ __global__ void __launch_bounds__(64) k_bjac(BView b) {
 
 // ---------------------------------------------------------------------------
 // Ritz vectors X = V Y, WX = W Y (kk of them), corrections T = (WX - theta X) /
-// (theta - diag) and residual-norm partials for the k roots. Row-mapped.
+// (theta - diag) and residual-norm partials for the k roots. Row-mapped. At a few rows a
+// thread its time is the latency of the loads: four columns of V and W are in flight at
+// once (past the last one it is read again, with weight 0). KB = 2 k at least, 2 for one root.
 // ---------------------------------------------------------------------------
+template <int KB>
 __global__ void __launch_bounds__(256) k_britz(BView b) {
     const int p = b.row_blk[blockIdx.x];
     const int *st = b.st + p * ST;
@@ -190,32 +235,40 @@ __global__ void __launch_bounds__(256) k_britz(BView b) {
     const double *V = b.V + P.basis, *W = b.W + P.basis;
     double *X = b.X + P.ritz, *WX = b.WX + P.ritz, *T = b.T + P.corr;
     const i64 r0 = b.row_first[blockIdx.x], r1 = min(r0 + (i64)b.RB, P.nd);
-    double ss[BK_MAX];
+    double ss[KB / 2];
 #pragma unroll
-    for (int j = 0; j < BK_MAX; ++j) ss[j] = 0.0;
+    for (int j = 0; j < KB / 2; ++j) ss[j] = 0.0;
     for (i64 r = r0 + threadIdx.x; r < r1; r += 256) {
-        double x[2 * BK_MAX], w[2 * BK_MAX];
+        double x[KB], w[KB];
 #pragma unroll
-        for (int j = 0; j < 2 * BK_MAX; ++j) x[j] = w[j] = 0.0;
-        for (int i = 0; i < m; ++i) {
-            const double vv = V[(i64)i * P.nd + r], ww = W[(i64)i * P.nd + r];
+        for (int j = 0; j < KB; ++j) x[j] = w[j] = 0.0;
+        for (int i0 = 0; i0 < m; i0 += 4) {
+            double vv[4], ww[4];
 #pragma unroll
-            for (int j = 0; j < 2 * BK_MAX; ++j)
-                if (j < kk) {
-                    const double y = Y[i * 2 * BK_MAX + j];
-                    x[j] += vv * y;
-                    w[j] += ww * y;
-                }
+            for (int u = 0; u < 4; ++u) {
+                const i64 o = (i64)min(i0 + u, m - 1) * P.nd + r;
+                vv[u] = V[o];
+                ww[u] = W[o];
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int j = 0; j < KB; ++j)
+                    if (i0 + u < m && j < kk) {
+                        const double y = Y[(i0 + u) * 2 * BK_MAX + j];
+                        x[j] += vv[u] * y;
+                        w[j] += ww[u] * y;
+                    }
         }
         const double d = b.diag[P.vec + r];
 #pragma unroll
-        for (int j = 0; j < 2 * BK_MAX; ++j)
+        for (int j = 0; j < KB; ++j)
             if (j < kk) {
                 X[(i64)j * P.nd + r] = x[j];
                 WX[(i64)j * P.nd + r] = w[j];
             }
 #pragma unroll
-        for (int j = 0; j < BK_MAX; ++j)
+        for (int j = 0; j < KB / 2; ++j)
             if (j < k) {
                 const double res = w[j] - th[j] * x[j];
                 double den = th[j] - d;
@@ -224,10 +277,10 @@ __global__ void __launch_bounds__(256) k_britz(BView b) {
                 ss[j] += res * res;
             }
     }
-    __shared__ double red[4][BK_MAX];
+    __shared__ double red[4][KB / 2];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
 #pragma unroll
-    for (int j = 0; j < BK_MAX; ++j) {
+    for (int j = 0; j < KB / 2; ++j) {
         double v = ss[j];
         for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
         if (lane == 0) red[wave][j] = v;
@@ -314,6 +367,7 @@ __global__ void __launch_bounds__(256) k_bctl(BView b) {
     }
     if (done) {
         st[S_ACTIVE] = 0;
+        atomicAdd(b.nactive, -1);
         st[S_NADD] = 0;
         st[S_RESTART] = 0;
         for (int j = 0; j < k; ++j) b.energy[(i64)p * BK_MAX + j] = th[j] + P.ecore;
@@ -362,77 +416,92 @@ __global__ void __launch_bounds__(256) k_bmove(BView b) {
 }
 
 // ---------------------------------------------------------------------------
-// Tall-skinny products. mode 0: V[:, 0:c0]^T N; 1: N^T N; 2: V[:, 0:c0+nadd]^T W[:, c0:c0+nadd]
-// with N = V[:, c0:c0+nadd]. Partials per row block, 8 x 8 tile per blockIdx.y.
+// Tall-skinny products with N = V[:, c0:c0+nadd]. GR_VN: V[:, 0:c0]^T N; GR_NN: N^T N;
+// GR_VVN: V[:, 0:c0+nadd]^T N, both of them at once; GR_VW: V[:, 0:c0+nadd]^T W[:, c0:c0+nadd].
+// Partials per row block, 8 x NJ tile per blockIdx.y (NJ = 1 where a problem has one root).
+// As in the single-problem solver, every load is unconditional (columns past the tile repeat
+// its last one and are not stored) and the lanes are summed by halving. 16 problems of up to
+// 63,504 determinants, one root: 20 -> 12 us.
 // ---------------------------------------------------------------------------
+enum { GR_VN = 0, GR_NN, GR_VW, GR_VVN };
+
+template <int NJ>
 __global__ void __launch_bounds__(256) k_bgram(BView b, int mode) {
     const int p = b.row_blk[blockIdx.x];
     const int *st = b.st + p * ST;
     if (!st[S_ACTIVE]) return;
     const BProb P = b.prob[p];
     const int c0 = st[S_C0], nadd = st[S_NADD];
-    const int ma = (mode == 0) ? c0 : (mode == 1 ? nadd : c0 + nadd), mb = nadd;
+    const int ma = (mode == GR_VN) ? c0 : (mode == GR_NN ? nadd : c0 + nadd), mb = nadd;
     if (ma == 0 || mb == 0) return;
-    const int tj = (mb + 7) / 8;
-    const int i0 = (blockIdx.y / tj) * 8, j0 = (blockIdx.y % tj) * 8;
+    const int tj = (mb + NJ - 1) / NJ;
+    const int i0 = (blockIdx.y / tj) * 8, j0 = (blockIdx.y % tj) * NJ;
     if (i0 >= ma || j0 >= mb) return;
-    const int ni = min(8, ma - i0), nj = min(8, mb - j0);
-    const double *A = b.V + P.basis + (mode == 1 ? (i64)c0 * P.nd : 0);
-    const double *B = (mode == 2 ? b.W : b.V) + P.basis + (i64)c0 * P.nd;
+    const int ni = min(8, ma - i0), nj = min(NJ, mb - j0);
+    const double *A = b.V + P.basis + (mode == GR_NN ? (i64)c0 * P.nd : 0);
+    const double *B = (mode == GR_VW ? b.W : b.V) + P.basis + (i64)c0 * P.nd;
     const i64 r0 = b.row_first[blockIdx.x], r1 = min(r0 + (i64)b.RB, P.nd);
-    double acc[8][8];
+    double acc[8 * NJ];
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) acc[i][j] = 0.0;
+    for (int t = 0; t < 8 * NJ; ++t) acc[t] = 0.0;
     for (i64 r = r0 + threadIdx.x; r < r1; r += 256) {
-        double x[8], y[8];
+        double x[8], y[NJ];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) x[i] = (i < ni) ? A[(i64)(i0 + i) * P.nd + r] : 0.0;
+        for (int i = 0; i < 8; ++i) x[i] = A[(i64)(i0 + min(i, ni - 1)) * P.nd + r];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) y[j] = (j < nj) ? B[(i64)(j0 + j) * P.nd + r] : 0.0;
+        for (int j = 0; j < NJ; ++j) y[j] = B[(i64)(j0 + min(j, nj - 1)) * P.nd + r];
 #pragma unroll
         for (int i = 0; i < 8; ++i)
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[i][j] += x[i] * y[j];
+            for (int j = 0; j < NJ; ++j) acc[i * NJ + j] += x[i] * y[j];
     }
-    __shared__ double red[4][64];
+    __shared__ double red[4][8 * NJ];
+    constexpr int LV = 64 / (8 * NJ);  // lanes per value after the halving
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            double v = acc[i][j];
-            for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-            if (lane == 0) red[wave][i * 8 + j] = v;
-        }
+    const double sum = halving_sum<8 * NJ>(acc);
+    if (lane % LV == 0) red[wave][lane / LV] = sum;
     __syncthreads();
-    if (threadIdx.x < 64) {
-        const int i = threadIdx.x / 8, j = threadIdx.x % 8;
+    if (threadIdx.x < 8 * NJ) {
+        const int i = threadIdx.x / NJ, j = threadIdx.x % NJ;
         if (i < ni && j < nj)
             b.partial[(i64)blockIdx.x * b.S + (i0 + i) * mb + j0 + j] =
                 ((red[0][threadIdx.x] + red[1][threadIdx.x]) + red[2][threadIdx.x]) + red[3][threadIdx.x];
     }
 }
 
-// out[p][s] = sum over the problem's row blocks of partial[s]; a wave per slot.
+// out[p][s] = sum over the problem's row blocks of partial[s]; a wave per slot. What hangs on
+// one slot alone is done with it: the norms of the new columns before orthogonalisation
+// (GR_VVN), the Rayleigh matrix's new entries from its lower triangle, the basis size and the
+// count of sigma products (GR_VW).
 __global__ void __launch_bounds__(256) k_bred(BView b, int mode) {
     const int p = blockIdx.x;
-    const int *st = b.st + p * ST;
+    int *st = b.st + p * ST;
     if (!st[S_ACTIVE]) return;
     const BProb P = b.prob[p];
     const int c0 = st[S_C0], nadd = st[S_NADD];
-    const int ma = (mode == 0) ? c0 : (mode == 1 ? nadd : c0 + nadd);
+    const int ma = (mode == GR_VN) ? c0 : (mode == GR_NN ? nadd : c0 + nadd);
     const int cnt = ma * nadd;
     const int s = blockIdx.y * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (mode == GR_VW && s == 0 && lane == 0) {
+        st[S_M] = c0 + nadd;
+        st[S_NSIG] += nadd;
+    }
     if (s >= cnt) return;
     double v = 0.0;
     for (i64 q = lane; q < P.nrb; q += 64) v += b.partial[(P.rb0 + q) * b.S + s];
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    if (lane == 0) b.out[(i64)p * b.S + s] = v;
+    if (lane != 0) return;
+    const int i = s / nadd, a = s % nadd;
+    if (mode == GR_VW) {
+        double *G = b.G + (i64)p * BM_MAX * BM_MAX;
+        if (i >= c0 + a || i < c0) G[i * BM_MAX + c0 + a] = G[(c0 + a) * BM_MAX + i] = v;
+        return;
+    }
+    b.out[(i64)p * b.S + s] = v;
+    if (mode == GR_VVN && i == c0 + a) b.nrm0[(i64)p * NB2 + a] = sqrt(fmax(v, 0.0));
 }
 
-// N -= V[:, 0:c0] C (C = out, c0 x nadd). Row-mapped.
+// N -= V[:, 0:c0] C (C = out, c0 x nadd), eight columns of V in flight. Row-mapped.
 __global__ void __launch_bounds__(256) k_bupd(BView b) {
     const int p = b.row_blk[blockIdx.x];
     const int *st = b.st + p * ST;
@@ -445,27 +514,30 @@ __global__ void __launch_bounds__(256) k_bupd(BView b) {
     const i64 r0 = b.row_first[blockIdx.x], r1 = min(r0 + (i64)b.RB, P.nd);
     for (i64 r = r0 + threadIdx.x; r < r1; r += 256)
         for (int a = 0; a < nadd; ++a) {
+            const double x = V[(i64)(c0 + a) * P.nd + r];
             double acc = 0.0;
-            for (int i = 0; i < c0; ++i) acc += V[(i64)i * P.nd + r] * C[i * nadd + a];
-            V[(i64)(c0 + a) * P.nd + r] -= acc;
+            for (int i0 = 0; i0 < c0; i0 += 8) {
+                double vv[8];
+#pragma unroll
+                for (int u = 0; u < 8; ++u) vv[u] = V[(i64)min(i0 + u, c0 - 1) * P.nd + r];
+#pragma unroll
+                for (int u = 0; u < 8; ++u)
+                    if (i0 + u < c0) acc += vv[u] * C[(i0 + u) * nadd + a];
+            }
+            V[(i64)(c0 + a) * P.nd + r] = x - acc;
         }
 }
 
-// Per problem (one thread): save = 1 keeps the norms of the new columns before
-// orthogonalisation; save = 0 forms R^-1 of the Cholesky factor of N^T N, keeping
-// only columns whose norm did not collapse below 1e-10 of the saved one.
-__global__ void k_bchol(BView b, int save) {
+// Per problem (one thread): R^-1 of the Cholesky factor of N^T N, keeping only columns whose
+// norm did not collapse below 1e-10 of the one before orthogonalisation.
+__global__ void k_bchol(BView b) {
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= b.nprob) return;
     int *st = b.st + p * ST;
     if (!st[S_ACTIVE]) return;
     const int nadd = st[S_NADD];
     const double *M = b.out + (i64)p * b.S;
-    double *n0 = b.nrm0 + (i64)p * NB2;
-    if (save) {
-        for (int a = 0; a < nadd; ++a) n0[a] = sqrt(fmax(M[a * nadd + a], 0.0));
-        return;
-    }
+    const double *n0 = b.nrm0 + (i64)p * NB2;
     double R[NB2][NB2];
     int keep[NB2], nk = 0;
     for (int a = 0; a < nadd; ++a) {
@@ -506,7 +578,19 @@ __global__ void k_bchol(BView b, int save) {
     st[S_DONE] = nadd;  // columns present before the QR (read by k_bapplyR)
 }
 
-// N <- N R^-1 over the kept columns, row by row in place. Row-mapped.
+// ---------------------------------------------------------------------------
+// Batched matrix-free sigma of the new columns (see direct.hip for the passes).
+// Columns c = v * nd + J of the problem's new block; FP32 problems go through
+// FP32 copies of the columns. Problems of both precisions share each launch.
+// ---------------------------------------------------------------------------
+template <typename T>
+__device__ inline bool sigma_here(const int *st) {
+    return st[S_ACTIVE] && st[S_NADD] > 0 && (st[S_PHASE] == (sizeof(T) == 4 ? 1 : 0));
+}
+
+// N <- N R^-1 over the kept columns, row by row in place; a problem in its FP32 phase gets
+// the FP32 copy of the new columns with it. NB = 1 where a problem has one root. Row-mapped.
+template <int NB>
 __global__ void __launch_bounds__(256) k_bapplyR(BView b) {
     const int p = b.row_blk[blockIdx.x];
     const int *st = b.st + p * ST;
@@ -514,67 +598,29 @@ __global__ void __launch_bounds__(256) k_bapplyR(BView b) {
     const BProb P = b.prob[p];
     const int c0 = st[S_C0], nk = st[S_NADD], nold = st[S_DONE];
     if (nold == 0) return;
+    const bool copy = sigma_here<float>(st);
     const double *Rinv = b.Rinv + (i64)p * NB2 * NB2;
     double *V = b.V + P.basis + (i64)c0 * P.nd;
     const i64 r0 = b.row_first[blockIdx.x], r1 = min(r0 + (i64)b.RB, P.nd);
     for (i64 r = r0 + threadIdx.x; r < r1; r += 256) {
-        double x[NB2], y[NB2];
-        for (int a = 0; a < NB2; ++a) x[a] = (a < nold) ? V[(i64)a * P.nd + r] : 0.0;
-        for (int j = 0; j < NB2; ++j) {
+        double x[NB], y[NB];
+#pragma unroll
+        for (int a = 0; a < NB; ++a) x[a] = (a < nold) ? V[(i64)a * P.nd + r] : 0.0;
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
             double v = 0.0;
-            for (int a = 0; a < NB2; ++a)
+#pragma unroll
+            for (int a = 0; a < NB; ++a)
                 if (a < nold) v += x[a] * Rinv[a * NB2 + j];
             y[j] = v;
         }
-        for (int j = 0; j < NB2; ++j)
-            if (j < nk) V[(i64)j * P.nd + r] = y[j];
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+            if (j < nk) {
+                V[(i64)j * P.nd + r] = y[j];
+                if (copy) b.S32x[P.s32 + (i64)j * P.nd + r] = (float)y[j];
+            }
     }
-}
-
-// New Rayleigh-matrix entries (out: (c0+nadd) x nadd) and the basis size; counts
-// the sigma products. One thread per problem.
-__global__ void k_bgupd(BView b) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= b.nprob) return;
-    int *st = b.st + p * ST;
-    if (!st[S_ACTIVE]) return;
-    const int c0 = st[S_C0], nadd = st[S_NADD];
-    const double *h = b.out + (i64)p * b.S;
-    double *G = b.G + (i64)p * BM_MAX * BM_MAX;
-    for (int i = 0; i < c0 + nadd; ++i)
-        for (int a = 0; a < nadd; ++a) {
-            const double x = h[i * nadd + a];
-            G[i * BM_MAX + c0 + a] = x;
-            G[(c0 + a) * BM_MAX + i] = x;
-        }
-    for (int a = 0; a < nadd; ++a)
-        for (int c = a + 1; c < nadd; ++c) {
-            const double x = 0.5 * (G[(c0 + a) * BM_MAX + c0 + c] + G[(c0 + c) * BM_MAX + c0 + a]);
-            G[(c0 + a) * BM_MAX + c0 + c] = G[(c0 + c) * BM_MAX + c0 + a] = x;
-        }
-    st[S_M] = c0 + nadd;
-    st[S_NSIG] += nadd;
-}
-
-__global__ void k_bcount(BView b) {
-    __shared__ int c;
-    if (threadIdx.x == 0) c = 0;
-    __syncthreads();
-    int mine = 0;
-    for (int p = threadIdx.x; p < b.nprob; p += blockDim.x) mine += b.st[p * ST + S_ACTIVE];
-    atomicAdd(&c, mine);
-    __syncthreads();
-    if (threadIdx.x == 0) *b.nactive = c;
-}
-
-// ---------------------------------------------------------------------------
-// Batched matrix-free sigma of the new columns (see direct.hip for the passes).
-// Columns c = v * nd + J of the problem's new block; FP32 problems go through
-// FP32 copies of the columns.
-// ---------------------------------------------------------------------------
-template <typename T>
-__device__ inline bool sigma_here(const int *st) {
-    return st[S_ACTIVE] && st[S_NADD] > 0 && (st[S_PHASE] == (sizeof(T) == 4 ? 1 : 0));
 }
 
 template <typename T>
@@ -583,150 +629,158 @@ __device__ inline const T *xcols(const BView &b, const BProb &P, int c0) {
     else return b.S32x + P.s32;
 }
 template <typename T>
-__device__ inline T *ycols(const BView &b, const BProb &P, int c0) {
-    if constexpr (sizeof(T) == 8) return b.W + P.basis + (i64)c0 * P.nd;
-    else return b.S32y + P.s32;
-}
-template <typename T>
 __device__ inline T *wspace(const BView &b, const BProb &P) {
     if constexpr (sizeof(T) == 8) return b.work64 + P.work;
     else return b.work32 + P.work;
 }
 
-// to = 0: FP64 new columns -> FP32 scratch; to = 1: FP32 images -> W. Row-mapped.
-__global__ void __launch_bounds__(256) k_bcvt(BView b, int to) {
+// FP32 images of the fused pass's problems -> W. Row-mapped.
+__global__ void __launch_bounds__(256) k_bcvt(BView b) {
     const int p = b.row_blk[blockIdx.x];
     const int *st = b.st + p * ST;
     if (!sigma_here<float>(st)) return;
     const BProb P = b.prob[p];
+    if (!P.big) return;
     const int c0 = st[S_C0], nadd = st[S_NADD];
     const i64 r0 = b.row_first[blockIdx.x], r1 = min(r0 + (i64)b.RB, P.nd);
     for (i64 r = r0 + threadIdx.x; r < r1; r += 256)
         for (int a = 0; a < nadd; ++a) {
             const i64 o = (i64)a * P.nd + r;
-            if (to == 0) b.S32x[P.s32 + o] = (float)b.V[P.basis + (i64)c0 * P.nd + o];
-            else b.W[P.basis + (i64)c0 * P.nd + o] = (double)b.S32y[P.s32 + o];
+            b.W[P.basis + (i64)c0 * P.nd + o] = (double)b.S32y[P.s32 + o];
         }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) k_bmf_d(BView b) {
-    const int p = b.col_blk[blockIdx.x];
-    const int *st = b.st + p * ST;
-    if (!sigma_here<T>(st)) return;
-    const BProb P = b.prob[p];
-    const i64 c = b.col_first[blockIdx.x] + threadIdx.x;
-    const i64 ncol = (i64)st[S_NADD] * P.nd;
-    if (c >= ncol) return;
-    const int c0 = st[S_C0];
-    const i64 v = c / P.nd, J = c - v * P.nd;
-    const i64 Ja = J / P.NB, Jb = J - Ja * P.NB;
-    const T *X = xcols<T>(b, P, c0) + v * P.nd;
-    T *W = wspace<T>(b, P);
-    const int2 *pa = b.tab + P.tab_a + Ja * P.nea, *pb = b.tab + P.tab_b + Jb * P.neb;
-    int ia = 0, ib = 0;
-    int2 ea = pa[0], eb = pb[0];
-    for (int q = 0; q < P.npair; ++q) {
-        T acc = (T)0;
-        if (ia < P.nea && (ea.y & 0xffff) == q) {
-            acc += ((ea.y >> 16) ? (T)-1 : (T)1) * X[(i64)ea.x * P.NB + Jb];
-            if (++ia < P.nea) ea = pa[ia];
-        }
-        if (ib < P.neb && (eb.y & 0xffff) == q) {
-            acc += ((eb.y >> 16) ? (T)-1 : (T)1) * X[Ja * P.NB + eb.x];
-            if (++ib < P.neb) eb = pb[ib];
-        }
-        W[(i64)q * P.ldw + c] = acc;
-    }
 }
 
 typedef double bf64x4 __attribute__((ext_vector_type(4)));
 typedef float bf32x4 __attribute__((ext_vector_type(4)));
 
-// In-place product E = 1/2 V D + k x on the problem's workspace, 128 columns per
-// block (see k_mf_gemm); the row-tile count varies per problem (mt <= 8).
+constexpr int ETC = 64;  // columns of a product tile
+// Row length of D in LDS: the four rows that the lanes of a wave read together start in
+// different banks in both precisions.
+constexpr int ELD = ETC + 4;
+
+// Row tile m (16 pairs) of E = 1/2 V D + k x on all 64 columns of a tile, D in LDS, by one
+// wave, so that V is read once per tile. Lane group lk takes the contraction's indices 4 lk ..
+// 4 lk + 3 of each 16, so that V comes in vectors.
 template <typename T>
-__global__ void __launch_bounds__(256) k_bmf_gemm(BView b) {
-    const int p = b.tile_blk[blockIdx.x];
-    const int *st = b.st + p * ST;
-    if (!sigma_here<T>(st)) return;
-    const BProb P = b.prob[p];
-    const i64 ncol = (i64)st[S_NADD] * P.nd;
-    const i64 cb = b.tile_first[blockIdx.x];
-    if (cb >= ncol) return;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lr = lane & 15, lk = lane >> 4;
-    const i64 c0 = cb + wave * 32;
-    const int KP = P.kpad, MT = P.mt;
-    const T *V = (sizeof(T) == 8) ? (const T *)(b.V64p + P.vint) : (const T *)(b.V32p + P.vint);
-    const T *kv = (sizeof(T) == 8) ? (const T *)(b.k64p + P.kv) : (const T *)(b.k32p + P.kv);
-    const T *X = xcols<T>(b, P, b.st[p * ST + S_C0]);
-    T *W = wspace<T>(b, P);
-    typedef typename std::conditional<sizeof(T) == 8, bf64x4, bf32x4>::type acc_t;
-    acc_t acc[8][2];
+__device__ inline void e_product(const T *D, int KP, int m, const T *V, const T *kv, const T (&x)[4], T *W, i64 ldw) {
+    typedef typename std::conditional<sizeof(T) == 8, bf64x4, bf32x4>::type vec;
+    const int lane = threadIdx.x & 63, lr = lane & 15, lk = lane >> 4;
+    vec acc[4] = {vec{}, vec{}, vec{}, vec{}};
+    V += (16 * m + lr) * KP + 4 * lk;
+    D += 4 * lk * ELD + lr;
+    for (int k0 = 0; k0 < KP; k0 += 16) {
+        const vec a = *(const vec *)(V + k0);
+        T d[4][4];
 #pragma unroll
-    for (int m = 0; m < 8; ++m) {
-        acc[m][0] = acc_t{};
-        acc[m][1] = acc_t{};
-    }
-    const bool live0 = c0 + lr < ncol, live1 = c0 + 16 + lr < ncol;
-    for (int k0 = 0; k0 < KP; k0 += 4) {
-        const T b0 = live0 ? W[(i64)(k0 + lk) * P.ldw + c0 + lr] : (T)0;
-        const T b1 = live1 ? W[(i64)(k0 + lk) * P.ldw + c0 + 16 + lr] : (T)0;
+        for (int u = 0; u < 4; ++u)
 #pragma unroll
-        for (int m = 0; m < 8; ++m) {
-            if (m < MT) {
-                const T a = V[(16 * m + lr) * KP + k0 + lk];
-                if constexpr (sizeof(T) == 8) {
-                    acc[m][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b0, acc[m][0], 0, 0, 0);
-                    acc[m][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, b1, acc[m][1], 0, 0, 0);
-                } else {
-                    acc[m][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b0, acc[m][0], 0, 0, 0);
-                    acc[m][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a, b1, acc[m][1], 0, 0, 0);
-                }
+            for (int j = 0; j < 4; ++j) d[u][j] = D[(k0 + u) * ELD + 16 * j];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if constexpr (sizeof(T) == 8) acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[u], d[u][j], acc[j], 0, 0, 0);
+                else acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[u], d[u][j], acc[j], 0, 0, 0);
             }
-        }
     }
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const i64 c = c0 + 16 * t + lr;
-        const T x = (c < ncol) ? X[c] : (T)0;
+    for (int r = 0; r < 4; ++r) {
+        const int q = 16 * m + ((sizeof(T) == 8) ? lk + 4 * r : 4 * lk + r);
+        const T k = kv[q];
 #pragma unroll
-        for (int m = 0; m < 8; ++m)
-            if (m < MT)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const int q = (sizeof(T) == 8) ? 16 * m + lk + 4 * r : 16 * m + 4 * lk + r;
-                    W[(i64)q * P.ldw + c] = (T)0.5 * acc[m][t][r] + kv[q] * x;
-                }
+        for (int j = 0; j < 4; ++j) W[(i64)q * ldw + 16 * j] = (T)0.5 * acc[j][r] + k * x[j];
     }
 }
 
 template <typename T>
+__device__ inline void e_tile(const BView &b, const BProb &P, const int *st, unsigned cb, T *D) {
+    const unsigned ncol = (unsigned)(st[S_NADD] * P.nd), nd = (unsigned)P.nd, NB = (unsigned)P.NB;
+    if (cb >= ncol) return;
+    const int t = threadIdx.x, cl = t & 63, w = t >> 6;
+    const T *X = xcols<T>(b, P, st[S_C0]);
+    for (int i = t; i < P.kpad * ELD; i += 256) D[i] = (T)0;
+    const unsigned c = min(cb + cl, ncol - 1);
+    const unsigned v = c / nd, J = c - v * nd, Ja = J / NB, Jb = J - Ja * NB;
+    const T *Xv = X + (i64)v * nd;
+    const int2 *pa = b.tab + P.tab_a + (i64)Ja * P.nea, *pb = b.tab + P.tab_b + (i64)Jb * P.neb;
+    __syncthreads();
+    // a string reaches each pair once: the threads of a column write different rows
+#pragma unroll 4
+    for (int e = w; e < P.nea; e += 4) {
+        const int2 q = pa[e];
+        D[(q.y & 0xffff) * ELD + cl] = ((q.y >> 16) ? (T)-1 : (T)1) * Xv[(i64)q.x * NB + Jb];
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int e = w; e < P.neb; e += 4) {
+        const int2 q = pb[e];
+        D[(q.y & 0xffff) * ELD + cl] += ((q.y >> 16) ? (T)-1 : (T)1) * Xv[(i64)Ja * NB + q.x];
+    }
+    __syncthreads();
+    const T *V, *kv;
+    if constexpr (sizeof(T) == 8) {
+        V = b.V64p + P.vint;
+        kv = b.k64p + P.kv;
+    } else {
+        V = b.V32p + P.vint;
+        kv = b.k32p + P.kv;
+    }
+    const unsigned mine = cb + (t & 15);
+    T x[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) x[j] = (mine + 16 * j < ncol) ? X[mine + 16 * j] : (T)0;
+    T *W = wspace<T>(b, P) + mine;  // rows are padded to whole tiles
+    for (int m = w; m < P.mt; m += 4) e_product<T>(D, P.kpad, m, V, kv, x, W, P.ldw);
+}
+
+// D (the singly excited columns by pair, gathered from the string tables) built in LDS and
+// multiplied there, E = 1/2 V D + k x to the workspace: a tile of 64 columns per workgroup,
+// four threads a column in the gather, a wave per 16 pairs in the product. D never goes to
+// memory, which it did twice, and the gather's loads are independent (one thread per column
+// walked two sorted lists through a chain of up to 55 dependent steps). It is bound by the
+// write of E and its gathers. 16 problems of up to 63,504 determinants, one root: gather and
+// product of both precisions 183 -> 55 us an iteration, and four launches -> one.
+__global__ void __launch_bounds__(256, 4) k_bmf_e(BView b) {
+    extern __shared__ __align__(16) unsigned char bmf_lds[];
+    const int p = b.tile_blk[blockIdx.x];
+    const int *st = b.st + p * ST;
+    if (!st[S_ACTIVE] || st[S_NADD] <= 0) return;
+    const BProb P = b.prob[p];
+    const unsigned cb = (unsigned)b.tile_first[blockIdx.x];
+    if (st[S_PHASE] == 1) e_tile<float>(b, P, st, cb, (float *)bmf_lds);
+    else e_tile<double>(b, P, st, cb, (double *)bmf_lds);
+}
+
+template <typename T>
+__device__ inline void sigma_column(const BView &b, const BProb &P, const int *st, unsigned c) {
+    const unsigned nd = (unsigned)P.nd, NB = (unsigned)P.NB;
+    if (c >= (unsigned)(st[S_NADD] * P.nd)) return;
+    const unsigned v = c / nd, I = c - v * nd, Ia = I / NB, Ib = I - Ia * NB;
+    const T *E = wspace<T>(b, P) + (i64)v * nd;
+    T acc = (T)0;
+    const int2 *pa = b.tab + P.tab_a + (i64)Ia * P.nea;
+#pragma unroll 4
+    for (int t = 0; t < P.nea; ++t) {
+        const int2 e = pa[t];
+        acc += ((e.y >> 16) ? (T)-1 : (T)1) * E[(i64)(e.y & 0xffff) * P.ldw + (i64)e.x * NB + Ib];
+    }
+    const int2 *pb = b.tab + P.tab_b + (i64)Ib * P.neb;
+#pragma unroll 4
+    for (int t = 0; t < P.neb; ++t) {
+        const int2 e = pb[t];
+        acc += ((e.y >> 16) ? (T)-1 : (T)1) * E[(i64)(e.y & 0xffff) * P.ldw + (i64)Ia * NB + e.x];
+    }
+    b.W[P.basis + ((i64)st[S_C0] + v) * nd + I] = (double)acc;
+}
+
 __global__ void __launch_bounds__(256) k_bmf_sigma(BView b) {
     const int p = b.col_blk[blockIdx.x];
     const int *st = b.st + p * ST;
-    if (!sigma_here<T>(st)) return;
+    if (!st[S_ACTIVE] || st[S_NADD] <= 0) return;
     const BProb P = b.prob[p];
-    const i64 c = b.col_first[blockIdx.x] + threadIdx.x;
-    const i64 ncol = (i64)st[S_NADD] * P.nd;
-    if (c >= ncol) return;
-    const int c0 = st[S_C0];
-    const i64 v = c / P.nd, I = c - v * P.nd;
-    const i64 Ia = I / P.NB, Ib = I - Ia * P.NB;
-    const T *E = wspace<T>(b, P) + v * P.nd;
-    T acc = (T)0;
-    const int2 *pa = b.tab + P.tab_a + Ia * P.nea;
-    for (int t = 0; t < P.nea; ++t) {
-        const int2 e = pa[t];
-        acc += ((e.y >> 16) ? (T)-1 : (T)1) * E[(i64)(e.y & 0xffff) * P.ldw + (i64)e.x * P.NB + Ib];
-    }
-    const int2 *pb = b.tab + P.tab_b + Ib * P.neb;
-    for (int t = 0; t < P.neb; ++t) {
-        const int2 e = pb[t];
-        acc += ((e.y >> 16) ? (T)-1 : (T)1) * E[(i64)(e.y & 0xffff) * P.ldw + Ia * P.NB + e.x];
-    }
-    ycols<T>(b, P, c0)[v * P.nd + I] = acc;
+    const unsigned c = (unsigned)b.col_first[blockIdx.x] + threadIdx.x;
+    if (st[S_PHASE] == 1) sigma_column<float>(b, P, st, c);
+    else sigma_column<double>(b, P, st, c);
 }
 
 // Initial block (as the single-problem solver): unit vectors on the lowest
@@ -775,6 +829,7 @@ struct Batch {
     DevBuf<i64> row_first, col_first, tile_first;
     DevBuf<unsigned long long> tconv;
     i64 nrowblk = 0, ncolblk = 0, ntile = 0;
+    size_t e_lds = 0;  // LDS of the product tile of the largest pair dimension
     BView view{};
     // large sub-problems: the fused matrix-free pass (direct.hip), one launch pair per
     // sub-problem and precision in the captured iteration, gated by a device descriptor
@@ -840,47 +895,45 @@ static void launch_rows(Batch &B, void (*kern)(BView), hipStream_t s) {
     PE_LAUNCH_CHECK();
 }
 
+static void launch_gram(Batch &B, unsigned gy, int mode, hipStream_t s) {
+    if (B.kb0 == 1) k_bgram<1><<<dim3((unsigned)B.nrowblk, gy), 256, 0, s>>>(B.view, mode);
+    else k_bgram<8><<<dim3((unsigned)B.nrowblk, gy), 256, 0, s>>>(B.view, mode);
+    PE_LAUNCH_CHECK();
+}
+
+static void launch_ritz(Batch &B, hipStream_t s) { launch_rows(B, B.k == 1 ? k_britz<2> : k_britz<2 * BK_MAX>, s); }
+
 static void orthonormalize_and_apply(Batch &B, hipStream_t s) {
     const BView &v = B.view;
     const unsigned np = (unsigned)B.nprob;
     const unsigned gy_full = (unsigned)(((B.mmax + 7) / 8) * ((B.kb0 + 7) / 8));
     const unsigned gy_new = (unsigned)(((B.kb0 + 7) / 8) * ((B.kb0 + 7) / 8));
     const unsigned ry = (unsigned)((B.S + 3) / 4);
-    // norms of the new columns before orthogonalisation
-    k_bgram<<<dim3((unsigned)B.nrowblk, gy_new), 256, 0, s>>>(v, 1);
-    PE_LAUNCH_CHECK();
-    k_bred<<<dim3(np, ry), 256, 0, s>>>(v, 1);
-    PE_LAUNCH_CHECK();
-    k_bchol<<<(np + 63) / 64, 64, 0, s>>>(v, 1);
-    PE_LAUNCH_CHECK();
     for (int pass = 0; pass < 2; ++pass) {  // CGS2 against the basis
-        k_bgram<<<dim3((unsigned)B.nrowblk, gy_full), 256, 0, s>>>(v, 0);
-        PE_LAUNCH_CHECK();
-        k_bred<<<dim3(np, ry), 256, 0, s>>>(v, 0);
+        const int mode = pass ? GR_VN : GR_VVN;  // the first takes the new columns' norms with it
+        launch_gram(B, gy_full, mode, s);
+        k_bred<<<dim3(np, ry), 256, 0, s>>>(v, mode);
         PE_LAUNCH_CHECK();
         launch_rows(B, k_bupd, s);
     }
     // Cholesky-QR of the new block, dropping dependent columns
-    k_bgram<<<dim3((unsigned)B.nrowblk, gy_new), 256, 0, s>>>(v, 1);
+    launch_gram(B, gy_new, GR_NN, s);
+    k_bred<<<dim3(np, ry), 256, 0, s>>>(v, GR_NN);
     PE_LAUNCH_CHECK();
-    k_bred<<<dim3(np, ry), 256, 0, s>>>(v, 1);
+    k_bchol<<<(np + 63) / 64, 64, 0, s>>>(v);
     PE_LAUNCH_CHECK();
-    k_bchol<<<(np + 63) / 64, 64, 0, s>>>(v, 0);
-    PE_LAUNCH_CHECK();
-    launch_rows(B, k_bapplyR, s);
-    // sigma of the new columns: FP64 problems, then FP32 ones; small sub-problems in
-    // the batched kernels (one launch each for all), large ones by the fused pass
+    launch_rows(B, B.kb0 == 1 ? k_bapplyR<1> : k_bapplyR<NB2>, s);
+    // sigma of the new columns: small sub-problems in the batched kernels (one launch each
+    // for all), large ones by the fused pass, FP64 problems, then FP32 ones
     const int nbig = (int)B.bigp.size();
     if (nbig) {
         k_btask<<<(unsigned)((nbig + 63) / 64), 64, 0, s>>>(v, B.bigp_d.p, nbig, B.dyn.p);
         PE_LAUNCH_CHECK();
     }
     if (B.ncolblk) {
-        k_bmf_d<double><<<(unsigned)B.ncolblk, 256, 0, s>>>(v);
+        k_bmf_e<<<(unsigned)B.ntile, 256, B.e_lds, s>>>(v);
         PE_LAUNCH_CHECK();
-        k_bmf_gemm<double><<<(unsigned)B.ntile, 256, 0, s>>>(v);
-        PE_LAUNCH_CHECK();
-        k_bmf_sigma<double><<<(unsigned)B.ncolblk, 256, 0, s>>>(v);
+        k_bmf_sigma<<<(unsigned)B.ncolblk, 256, 0, s>>>(v);
         PE_LAUNCH_CHECK();
     }
     for (int i = 0; i < nbig; ++i) {
@@ -888,43 +941,28 @@ static void orthonormalize_and_apply(Batch &B, hipStream_t s) {
         mf_sigma_batched<double>(B.bigv[(size_t)i], P.nd, B.kb0, B.V.p, B.W.p, (double *)B.fws.p, B.V64p.p + P.vint,
                                  B.k64p.p + P.kv, B.dyn.p + 6 * i, P.sector, s);
     }
-    k_bcvt<<<(unsigned)B.nrowblk, 256, 0, s>>>(v, 0);
-    PE_LAUNCH_CHECK();
-    if (B.ncolblk) {
-        k_bmf_d<float><<<(unsigned)B.ncolblk, 256, 0, s>>>(v);
-        PE_LAUNCH_CHECK();
-        k_bmf_gemm<float><<<(unsigned)B.ntile, 256, 0, s>>>(v);
-        PE_LAUNCH_CHECK();
-        k_bmf_sigma<float><<<(unsigned)B.ncolblk, 256, 0, s>>>(v);
-        PE_LAUNCH_CHECK();
-    }
     for (int i = 0; i < nbig; ++i) {
         const BProb &P = B.hp[(size_t)B.bigp[(size_t)i]];
         mf_sigma_batched<float>(B.bigv[(size_t)i], P.nd, B.kb0, B.S32x.p, B.S32y.p, (float *)B.fws.p,
                                 B.V32p.p + P.vint, B.k32p.p + P.kv, B.dyn.p + 6 * i + 3, P.sector, s);
     }
-    k_bcvt<<<(unsigned)B.nrowblk, 256, 0, s>>>(v, 1);
-    PE_LAUNCH_CHECK();
+    if (nbig) launch_rows(B, k_bcvt, s);
     // Rayleigh-matrix entries of the new columns
-    k_bgram<<<dim3((unsigned)B.nrowblk, gy_full), 256, 0, s>>>(v, 2);
-    PE_LAUNCH_CHECK();
-    k_bred<<<dim3(np, ry), 256, 0, s>>>(v, 2);
-    PE_LAUNCH_CHECK();
-    k_bgupd<<<(np + 63) / 64, 64, 0, s>>>(v);
+    launch_gram(B, gy_full, GR_VW, s);
+    k_bred<<<dim3(np, ry), 256, 0, s>>>(v, GR_VW);
     PE_LAUNCH_CHECK();
 }
 
 static void iteration(Batch &B, hipStream_t s) {
     const BView &v = B.view;
-    k_bjac<<<(unsigned)B.nprob, 64, 0, s>>>(v);
+    if (B.mmax <= 16) k_bjac<64><<<(unsigned)B.nprob, 64, 0, s>>>(v);
+    else k_bjac<256><<<(unsigned)B.nprob, 256, 0, s>>>(v);
     PE_LAUNCH_CHECK();
-    launch_rows(B, k_britz, s);
+    launch_ritz(B, s);
     k_bctl<<<(unsigned)B.nprob, 256, 0, s>>>(v);
     PE_LAUNCH_CHECK();
     launch_rows(B, k_bmove, s);
     orthonormalize_and_apply(B, s);
-    k_bcount<<<1, 256, 0, s>>>(v);
-    PE_LAUNCH_CHECK();
 }
 
 // The replayed-graph path over all given problems, on stream s.
@@ -1030,14 +1068,15 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
                 P.work = 0;
                 B.bigp.push_back(sp);
             } else {
-                P.ldw = (cols + 127) / 128 * 128;
+                P.ldw = (cols + ETC - 1) / ETC * ETC;
                 P.work = work;
                 work += (i64)P.kpad * P.ldw;
+                B.e_lds = std::max(B.e_lds, sizeof(double) * (size_t)P.kpad * ELD);
                 for (i64 c = 0; c < cols; c += 256) {
                     col_blk.push_back(sp);
                     col_first.push_back(c);
                 }
-                for (i64 c = 0; c < cols; c += 128) {
+                for (i64 c = 0; c < cols; c += ETC) {
                     tile_blk.push_back(sp);
                     tile_first.push_back(c);
                 }
@@ -1104,10 +1143,8 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
     B.S32x.alloc((size_t)s32);
     B.S32y.alloc((size_t)s32);
     B.work64.alloc((size_t)work);
-    PE_HIP(hipMemsetAsync(B.work64.p, 0, sizeof(double) * work, s));
     if (precision == PYCI_PREC_MIXED) {
         B.work32.alloc((size_t)work);
-        PE_HIP(hipMemsetAsync(B.work32.p, 0, sizeof(float) * work, s));
     } else {
         B.work32.alloc(1);
     }
@@ -1213,17 +1250,26 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
         // sa, sb, ca, cb leave scope here: the copies from them may still be pending
         PE_HIP(hipStreamSynchronize(s));
     }
+    std::vector<int> st_start((size_t)nsub * ST, 0);
     {
-        std::vector<int> st0((size_t)nsub * ST, 0);
         std::vector<double> best0((size_t)nsub * BK_MAX, 1e300);
         for (int q = 0; q < nsub; ++q) {
-            int *w = &st0[(size_t)q * ST];
+            int *w = &st_start[(size_t)q * ST];
             w[S_NADD] = nstart[(size_t)q];
             w[S_ACTIVE] = 1;
             w[S_PHASE] = (precision == PYCI_PREC_MIXED) ? 1 : 0;
         }
+        // for the timing below: a basis that is half full
+        std::vector<int> st0 = st_start;
+        for (int q = 0; q < nsub; ++q) {
+            int *w = &st0[(size_t)q * ST];
+            w[S_M] = w[S_C0] = B.mmax / 2;
+            w[S_NADD] = B.k;
+            w[S_KK] = B.k;
+        }
         PE_HIP(hipMemcpyAsync(B.st.p, st0.data(), sizeof(int) * st0.size(), hipMemcpyHostToDevice, s));
         PE_HIP(hipMemcpyAsync(B.best.p, best0.data(), sizeof(double) * best0.size(), hipMemcpyHostToDevice, s));
+        PE_HIP(hipMemcpyAsync(B.nactive.p, &nsub, sizeof(int), hipMemcpyHostToDevice, s));
         PE_HIP(hipStreamSynchronize(s));
     }
     // device view
@@ -1270,7 +1316,9 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
     v.tconv = B.tconv.p;
     v.nactive = B.nactive.p;
     // autotune the rows per block of the row-mapped kernels: time the Rayleigh-matrix
-    // product and the Ritz pass (their outputs are rewritten before use) per candidate
+    // product and the Ritz pass (their outputs are rewritten before use) per candidate, on a
+    // half-full basis (an empty one hides the Ritz pass's loads and took 1024 rows for 16
+    // problems of up to 63,504 determinants, where 256 is 11 % faster over the solve)
     int best_rb = 1024;
     {
         build_row_map(B, 1024);
@@ -1290,14 +1338,12 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
         for (int rb : {256, 1024, 4096}) {
             build_row_map(B, rb);
             const unsigned gy_full = (unsigned)(((B.mmax + 7) / 8) * ((B.kb0 + 7) / 8));
-            k_bgram<<<dim3((unsigned)B.nrowblk, gy_full), 256, 0, s>>>(B.view, 2);  // warm-up
-            PE_LAUNCH_CHECK();
+            launch_gram(B, gy_full, GR_VW, s);  // warm-up
+            launch_ritz(B, s);
             PE_HIP(hipEventRecord(e0, s));
             for (int r = 0; r < 3; ++r) {
-                k_bgram<<<dim3((unsigned)B.nrowblk, gy_full), 256, 0, s>>>(B.view, 2);
-                PE_LAUNCH_CHECK();
-                k_britz<<<(unsigned)B.nrowblk, 256, 0, s>>>(B.view);
-                PE_LAUNCH_CHECK();
+                launch_gram(B, gy_full, GR_VW, s);
+                launch_ritz(B, s);
             }
             PE_HIP(hipEventRecord(e1, s));
             PE_HIP(hipEventSynchronize(e1));
@@ -1309,6 +1355,8 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
             }
         }
         build_row_map(B, best_rb);
+        PE_HIP(hipMemcpyAsync(B.st.p, st_start.data(), sizeof(int) * st_start.size(), hipMemcpyHostToDevice, s));
+        PE_HIP(hipStreamSynchronize(s));
     }
     // prologue: orthonormalise the initial block and take its sigma
     unsigned long long t0 = 0;
@@ -1322,6 +1370,9 @@ static void batch_graph(pyci_ctx *ctx, hipStream_t s, i64 nprob, const i64 *nbas
     }
     k_binit<<<(unsigned)B.nrowblk, 256, 0, s>>>(B.view, dsa.p, dsb.p, dca.p, dcb.p);
     PE_LAUNCH_CHECK();
+    if (B.ncolblk)
+        PE_HIP(hipFuncSetAttribute((const void *)k_bmf_e, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   (int)(sizeof(double) * 128 * ELD)));  // any batch's, for callers on other threads
     orthonormalize_and_apply(B, s);
     // the iteration as a captured graph, replayed until no sub-problem is active
     hipGraph_t graph = nullptr;

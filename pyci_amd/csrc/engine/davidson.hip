@@ -111,30 +111,6 @@ __device__ void block_sums_to(double (&acc)[M], double *out) {
     }
 }
 
-// Sums over the 64 lanes of N values (32 or 64) by recursive halving: at each step a lane
-// passes on half of the values it holds and adds the partner's share of the other half, so
-// that N values take N - 1 exchanges (+ 1) instead of 6 N. Every value is added up in the
-// order of the shuffle tree xor 32, 16, .., 1. Lane l ends with value l (N = 64) or l / 2.
-template <int N, int O, int L>
-__device__ inline void halve(double (&v)[L]) {
-    if constexpr (N > 1) {
-        const bool up = threadIdx.x & O;
-#pragma unroll
-        for (int t = 0; t < N / 2; ++t) {
-            const double keep = up ? v[t + N / 2] : v[t], pass = up ? v[t] : v[t + N / 2];
-            v[t] = keep + __shfl_xor(pass, O);
-        }
-        halve<N / 2, O / 2, L>(v);
-    }
-}
-
-template <int N>
-__device__ double halving_sum(double (&v)[N]) {
-    halve<N, 32, N>(v);
-    if (N == 32) v[0] += __shfl_xor(v[0], 1);
-    return v[0];
-}
-
 // partial[b][ma][mb] = sum over rows of block b of A[:, i] * B[:, j] (8 x NJ tile per
 // blockIdx.y). At one or two rows a thread its time is the loads' latency and the
 // tile's reduction over the lanes: every load is unconditional (columns past the tile

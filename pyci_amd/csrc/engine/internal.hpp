@@ -421,6 +421,32 @@ __device__ inline XT lanes_sum(XT v) {
     return v;
 }
 
+// Sums over the 64 lanes of N values (a power of two) by recursive halving: at each step a
+// lane passes on half of the values it holds and adds the partner's share of the other half,
+// so that N values take N - 1 exchanges (and one for each step left) instead of 6 N. Every
+// value is added up in the order of the shuffle tree xor 32, 16, .., 1. Lane l ends with
+// value l / (64 / N).
+template <int N, int O, int L>
+__device__ inline void halve(double (&v)[L]) {
+    if constexpr (N > 1) {
+        const bool up = threadIdx.x & O;
+#pragma unroll
+        for (int t = 0; t < N / 2; ++t) {
+            const double keep = up ? v[t + N / 2] : v[t], pass = up ? v[t] : v[t + N / 2];
+            v[t] = keep + __shfl_xor(pass, O);
+        }
+        halve<N / 2, O / 2, L>(v);
+    }
+}
+
+template <int N>
+__device__ double halving_sum(double (&v)[N]) {
+    halve<N, 32, N>(v);
+#pragma unroll
+    for (int o = 32 / N; o > 0; o >>= 1) v[0] += __shfl_xor(v[0], o);
+    return v[0];
+}
+
 // ---------------------------------------------------------------------------
 // Host helpers
 // ---------------------------------------------------------------------------
