@@ -97,7 +97,7 @@ struct BView {
 // restart (m + k > mmax) and the number of Ritz vectors kk. A sweep goes in rounds of m / 2
 // disjoint pairs (the round-robin tournament), whose rotations are taken together: the chain
 // of divisions and square roots is walked once a round instead of once a pair. One wave for
-// m <= 16 (its barriers are free), four above. m = 10, one pair at a time -> in rounds:
+// m <= 16 (its barriers are free), four above. m = 10..12, one pair at a time -> in rounds:
 // 125 -> 35 us.
 // ---------------------------------------------------------------------------
 template <int BT>
@@ -222,7 +222,7 @@ __global__ void __launch_bounds__(BT) k_bjac(BView b) {
 // Ritz vectors X = V Y, WX = W Y (kk of them), corrections T = (WX - theta X) /
 // (theta - diag) and residual-norm partials for the k roots. Row-mapped. At a few rows a
 // thread its time is the latency of the loads: four columns of V and W are in flight at
-// once (past the last one it is read again, with weight 0). KB = 2 k at least, 2 for one root.
+// once (past the last one it is read again, with weight 0). KB = 2 k at least: 2 for one root, 4 for two.
 // ---------------------------------------------------------------------------
 template <int KB>
 __global__ void __launch_bounds__(256) k_britz(BView b) {
@@ -418,10 +418,10 @@ __global__ void __launch_bounds__(256) k_bmove(BView b) {
 // ---------------------------------------------------------------------------
 // Tall-skinny products with N = V[:, c0:c0+nadd]. GR_VN: V[:, 0:c0]^T N; GR_NN: N^T N;
 // GR_VVN: V[:, 0:c0+nadd]^T N, both of them at once; GR_VW: V[:, 0:c0+nadd]^T W[:, c0:c0+nadd].
-// Partials per row block, 8 x NJ tile per blockIdx.y (NJ = 1 where a problem has one root).
+// Partials per row block, 8 x NJ tile per blockIdx.y (NJ = 1 where a problem has one root, 4 for two).
 // As in the single-problem solver, every load is unconditional (columns past the tile repeat
 // its last one and are not stored) and the lanes are summed by halving. 16 problems of up to
-// 63,504 determinants, one root: 20 -> 12 us.
+// 63,504 determinants, two roots: 20 -> 7 us.
 // ---------------------------------------------------------------------------
 enum { GR_VN = 0, GR_NN, GR_VW, GR_VVN };
 
@@ -589,7 +589,7 @@ __device__ inline bool sigma_here(const int *st) {
 }
 
 // N <- N R^-1 over the kept columns, row by row in place; a problem in its FP32 phase gets
-// the FP32 copy of the new columns with it. NB = 1 where a problem has one root. Row-mapped.
+// the FP32 copy of the new columns with it. NB = 1 where a problem has one root, 4 for two. Row-mapped.
 template <int NB>
 __global__ void __launch_bounds__(256) k_bapplyR(BView b) {
     const int p = b.row_blk[blockIdx.x];
@@ -738,7 +738,7 @@ __device__ inline void e_tile(const BView &b, const BProb &P, const int *st, uns
 // four threads a column in the gather, a wave per 16 pairs in the product. D never goes to
 // memory, which it did twice, and the gather's loads are independent (one thread per column
 // walked two sorted lists through a chain of up to 55 dependent steps). It is bound by the
-// write of E and its gathers. 16 problems of up to 63,504 determinants, one root: gather and
+// write of E and its gathers. 16 problems of up to 63,504 determinants, two roots: gather and
 // product of both precisions 183 -> 55 us an iteration, and four launches -> one.
 __global__ void __launch_bounds__(256, 4) k_bmf_e(BView b) {
     extern __shared__ __align__(16) unsigned char bmf_lds[];
@@ -897,11 +897,12 @@ static void launch_rows(Batch &B, void (*kern)(BView), hipStream_t s) {
 
 static void launch_gram(Batch &B, unsigned gy, int mode, hipStream_t s) {
     if (B.kb0 == 1) k_bgram<1><<<dim3((unsigned)B.nrowblk, gy), 256, 0, s>>>(B.view, mode);
+    else if (B.kb0 <= 4) k_bgram<4><<<dim3((unsigned)B.nrowblk, gy), 256, 0, s>>>(B.view, mode);
     else k_bgram<8><<<dim3((unsigned)B.nrowblk, gy), 256, 0, s>>>(B.view, mode);
     PE_LAUNCH_CHECK();
 }
 
-static void launch_ritz(Batch &B, hipStream_t s) { launch_rows(B, B.k == 1 ? k_britz<2> : k_britz<2 * BK_MAX>, s); }
+static void launch_ritz(Batch &B, hipStream_t s) { launch_rows(B, B.k == 1 ? k_britz<2> : B.k == 2 ? k_britz<4> : k_britz<2 * BK_MAX>, s); }
 
 static void orthonormalize_and_apply(Batch &B, hipStream_t s) {
     const BView &v = B.view;
@@ -922,7 +923,7 @@ static void orthonormalize_and_apply(Batch &B, hipStream_t s) {
     PE_LAUNCH_CHECK();
     k_bchol<<<(np + 63) / 64, 64, 0, s>>>(v);
     PE_LAUNCH_CHECK();
-    launch_rows(B, B.kb0 == 1 ? k_bapplyR<1> : k_bapplyR<NB2>, s);
+    launch_rows(B, B.kb0 == 1 ? k_bapplyR<1> : B.kb0 <= 4 ? k_bapplyR<4> : k_bapplyR<NB2>, s);
     // sigma of the new columns: small sub-problems in the batched kernels (one launch each
     // for all), large ones by the fused pass, FP64 problems, then FP32 ones
     const int nbig = (int)B.bigp.size();
