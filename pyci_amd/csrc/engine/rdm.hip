@@ -1,14 +1,16 @@
 // One- and two-particle reduced density matrices on the GPU.
 //
 // Reference: compute_rdms for DOCIWfn (rdm.cpp:20-65) and FullCIWfn
-// (rdm.cpp:269-530; full FullCI spaces are contracted in rdm_full.hip): a loop over determinants I that visits every excitation
-// J of I present in the wave function with J > I and scatters c_I c_J times the
-// phase into the symmetric index permutations, plus the diagonal c_I^2 terms.
+// (rdm.cpp:269-530; full FullCI spaces are contracted in rdm_full.hip): a loop over
+// determinants I that visits every excitation J of I present in the wave function with
+// J > I and scatters c_I c_J times the phase into the symmetric index permutations, plus
+// the diagonal c_I^2 terms. Selected FullCI and GenCI sets find the connected pairs by
+// testing pairs of determinants (k_rdm_pairs); the rest enumerate.
 // GenCIWfn is computed from the operator algebra (every ordered pair I, J); the
 // reference's GenCI routine (rdm.cpp:532-632) has index errors and is not
 // reproduced.
 //
-// One wavefront per determinant; lanes take excitations from the same flat
+// Enumeration: one wavefront per determinant; lanes take excitations from the same flat
 // candidate index as the CSR builder. Accumulation uses hardware FP64 atomics
 // into R replicated copies of the RDM arrays (block b uses copy b % R) to spread
 // contention on hot elements, followed by a reduction over the copies.
