@@ -142,9 +142,10 @@ k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
     vals += beg;
     XT acc = (XT)0;
     for (i64 p0 = 0; p0 < len; p0 += U * 64) {
+        const bool whole = p0 + U * 64 <= len;
         int c[U];
         VT v[U];
-        if (p0 + U * 64 <= len) {
+        if (whole) {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 c[u] = __builtin_nontemporal_load(&cols[p0 + lane + u * 64]);
@@ -162,6 +163,11 @@ k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
         XT x[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) x[u] = X[c[u]];
+        if (!whole) {  // an infinity or a NaN times the 0 beyond the row would be a NaN
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (p0 + lane + u * 64 >= len) x[u] = (XT)0;
+        }
 #pragma unroll
         for (int u = 0; u < U; ++u) acc += (XT)v[u] * x[u];
     }
@@ -176,7 +182,9 @@ k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
 // of LDS. Longer rows are taken by the whole block afterwards. For sets whose columns follow
 // no order the gathers then cost LDS cycles instead of a 128-byte line of L2 each: 60,000
 // GenCI determinants (32 M entries, 3 panels) 286 -> 119 us (3.3 TB/s), 100,000 FullCI ones
-// (5 panels) 580 -> 221 us, 17,317 (one panel) 51 -> 22.5 us.
+// (5 panels) 580 -> 221 us, 17,317 (one panel) 51 -> 22.5 us. Lanes beyond a row's entries
+// multiply 0 by the 0 behind the panel: X may hold infinities and NaNs, which belong to the
+// rows of their columns alone.
 constexpr int SPMV_PANEL = 20000;
 constexpr int SPMV_LDS_WAVES = 16;
 
@@ -196,7 +204,7 @@ k_spmv_lds(i64 ncol, int npanel, const i64 *__restrict__ rowptr, const int32_t *
         const i64 pb = (i64)p * SPMV_PANEL;
         const int width = (int)min((i64)SPMV_PANEL, ncol - pb);
         __syncthreads();
-        if (threadIdx.x == 0) nlong = 0;
+        if (threadIdx.x == 0) nlong = 0, xs[SPMV_PANEL] = (XT)0;
         for (int t = threadIdx.x; t < width; t += NT) xs[t] = X[pb + t];
         __syncthreads();
         // entries [beg, beg + len) of a row in this panel
@@ -214,7 +222,7 @@ k_spmv_lds(i64 ncol, int npanel, const i64 *__restrict__ rowptr, const int32_t *
 #pragma unroll
             for (int u = 0; u < U; ++u) {
                 const int e = at + l + u * LANES;
-                c[u] = (int)pb;
+                c[u] = (int)((unsigned)pb + SPMV_PANEL);
                 v[u] = (VT)0;
                 if (e < len) {
                     c[u] = __builtin_nontemporal_load(&cp[e]);
@@ -225,7 +233,7 @@ k_spmv_lds(i64 ncol, int npanel, const i64 *__restrict__ rowptr, const int32_t *
         auto dot = [&](const int (&c)[U], const VT (&v)[U]) {
             XT s = (XT)0;
 #pragma unroll
-            for (int u = 0; u < U; ++u) s += (XT)v[u] * xs[c[u] - (int)pb];
+            for (int u = 0; u < U; ++u) s += (XT)v[u] * xs[(unsigned)c[u] - (unsigned)pb];
             return s;
         };
         int row = r0 + sub;
@@ -382,7 +390,7 @@ void spmv_plan(pyci_op *op, bool column_ordered_space) {
 
 template <int LANES, typename VT, typename XT>
 static void launch_lds(const pyci_op *op, const VT *vals, const XT *X, XT *Y, hipStream_t s) {
-    const size_t lds = sizeof(XT) * SPMV_PANEL;
+    const size_t lds = sizeof(XT) * (SPMV_PANEL + 1);
     static const bool attr = [&] {
         PE_HIP(hipFuncSetAttribute((const void *)k_spmv_lds<LANES, VT, XT>,
                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));

@@ -63,3 +63,41 @@ def test_rows_of_full_spaces():
         w = cls(nb, nu, nd)
         w.add_all_dets()
         _check(pyci.sparse_op(pyci.hamiltonian(0.0, one, two), w, storage="csr"), True)
+
+
+# one and several panels with a wave and with 16 lanes a row, ordered rows of a full space, one
+# or two chunks a row (DOCI), rows of a small set and of a large one that the panels leave out
+@pytest.mark.parametrize("kind,nb,nu,nd,ndet", [("fullci", 16, 3, 3, 19999), ("fullci", 18, 3, 3, 45000),
+                                                ("fullci", 10, 5, 4, 0), ("doci", 12, 5, 5, 0), ("fullci", 9, 4, 3, 3000),
+                                                ("genci", 44, 6, 0, 100000)])
+def test_non_finite_elements_stay_in_their_rows(kind, nb, nu, nd, ndet):
+    """An infinity or a NaN in x reaches the rows that hold its column and no other, and as
+    itself (an infinity of a row that has no other stays one)."""
+    rng = np.random.default_rng(ndet)
+    cls = {"fullci": pyci.fullci_wfn, "genci": pyci.genci_wfn, "doci": pyci.doci_wfn}[kind]
+    _, one, two = seeded_integrals(nb if kind != "genci" else nb // 2, 4, 63)
+    if kind == "genci":
+        one, two = spin_orbital(one, two)
+        dets = np.unique(np.sort(rng.random((2 * ndet, nb)).argpartition(nu, axis=1)[:, :nu], axis=1), axis=0)
+        dets = np.bitwise_or.reduce(np.uint64(1) << dets.astype(np.uint64), axis=1)
+        w = cls(nb, nu, nd, rng.permutation(dets)[:ndet].reshape(-1, 1))
+    else:
+        w = cls(nb, nu, nd)
+        w.add_all_dets()
+        if ndet:
+            w = cls(nb, nu, nd, rng.permutation(w.to_det_array())[:ndet])
+    op = pyci.sparse_op(pyci.hamiltonian(0.0, one, two), w, storage="csr")
+    data, indices, indptr = op.export()
+    row = np.repeat(np.arange(len(indptr) - 1), np.diff(indptr))
+    off = row != indices  # entries of value 0 are kept: they turn an infinity into a NaN
+    a = sp.coo_matrix((np.append(data, data[off]), (np.append(row, indices[off]), np.append(indices, row[off]))),
+                      shape=op.shape).tocsr()
+    n = op.shape[1]
+    for col in sorted({0, min(20000, n - 1), min(40000, n - 1), int(a.indices[a.indptr[7] - 1]), n - 1}):
+        for value in (np.inf, np.nan):
+            x = rng.normal(size=n)
+            x[col] = value
+            y, expect = op(x), a @ x
+            npt.assert_array_equal(np.isnan(y), np.isnan(expect))
+            npt.assert_array_equal(np.isinf(y), np.isinf(expect))
+            assert np.isfinite(y).sum() > 0
