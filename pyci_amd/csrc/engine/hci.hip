@@ -220,191 +220,194 @@ __global__ void __launch_bounds__(256) k_hb_most(const double *v, int n, double 
 // row's lists: the reference determinant's row alone holds a large part of all passing
 // candidates and one wave would still walk it when the others are done. Counters leave a
 // block in one atomic (one per wave and chunk on the same address took over half of the
-// ENPT2 pass).
+// ENPT2 pass). A launch holds fewer than 2^32 threads, 16.7 million such blocks: beyond a
+// million blocks a block takes several rows.
 constexpr int HCI_WAVES = 4;
+constexpr i64 HCI_BLOCKS = (i64)1 << 20;
 
 template <int KIND, int PASS>
 __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, const double *coeffs, double eps, double eps_plain,
                                              i64 rows_stride, NewSet S, unsigned long long *count, HbLists L) {
     __shared__ unsigned long long sums[HCI_WAVES];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const i64 row = blockIdx.x;
     const int n = H.n;
     const double *one = H.one, *two = H.two;
     const u64 m = full_mask(n);
-    const u64 up = w.dets[(i64)w.nkey * row];
-    const u64 dn = (KIND == PYCI_WFN_FULLCI) ? w.dets[2 * row + 1] : 0ULL;
-    const int nou = __popcll(up), nvu = n - nou, nod = __popcll(dn), nvd = n - nod;
-    const double cabs = fabs(coeffs[row]);
-    const double eps_i = eps / cabs, eps_plain_i = eps_plain / cabs;
-    // a row of the tail, whose threshold no element reaches
-    if (KIND != PYCI_WFN_DOCI && *L.most * (1.0 + 1e-12) <= eps_i) return;  // uniform per block
-    // lane q holds the q-th occupied / virtual orbital of each string
-    auto nth = [](u64 x, int t) {
-        for (int s = 0; s < t && x; ++s) x &= x - 1;
-        return x ? __builtin_ctzll(x) : 0;
-    };
-    const int packed = nth(up, lane) | (nth(~up & m, lane) << 8) | (nth(dn, lane) << 16) | (nth(~dn & m, lane) << 24);
     u64 local = 0;   // PASS 1: passing candidates of the wave
     int claims = 0;  // slots this lane has claimed
+    for (i64 row = blockIdx.x; row < w.ndet; row += gridDim.x) {
+        const u64 up = w.dets[(i64)w.nkey * row];
+        const u64 dn = (KIND == PYCI_WFN_FULLCI) ? w.dets[2 * row + 1] : 0ULL;
+        const int nou = __popcll(up), nvu = n - nou, nod = __popcll(dn), nvd = n - nod;
+        const double cabs = fabs(coeffs[row]);
+        const double eps_i = eps / cabs, eps_plain_i = eps_plain / cabs;
+        // a row of the tail, whose threshold no element reaches
+        if (KIND != PYCI_WFN_DOCI && *L.most * (1.0 + 1e-12) <= eps_i) continue;  // uniform per block
+        // lane q holds the q-th occupied / virtual orbital of each string
+        auto nth = [](u64 x, int t) {
+            for (int s = 0; s < t && x; ++s) x &= x - 1;
+            return x ? __builtin_ctzll(x) : 0;
+        };
+        const int packed = nth(up, lane) | (nth(~up & m, lane) << 8) | (nth(dn, lane) << 16) | (nth(~dn & m, lane) << 24);
 
-    // Evaluates one candidate; returns true when it passes and is new.
-    auto consider = [&](bool valid, u64 nu, u64 nd, double val, u64 pos, int sg) {
-        bool pass = false;
-        u64 key = 0;
-        if (valid && fabs(val) > eps_i) {
-            if (wfn_lookup(w, nu, nd) < 0) {
-                pass = true;
-                key = set_key(w, nu, nd);
-            }
-        }
-        if (PASS == 1) {
-            local += __popcll(__ballot(pass));
-        } else if (PASS == 5) {
-            // the reference multiplies the element by (phase * c_i) (enpt2.cpp:122-205)
-            if (pass) {
-                const u64 slot = set_insert(S, key, claims);
-                if (slot != ~0ULL)
-                    atomicAdd(reinterpret_cast<double *>(&S.slot[2 * slot + 1]), val * ((double)sg * coeffs[row]));
-            }
-        } else if (PASS == 2) {
-            if (pass) {
-                const u64 slot = set_insert(S, key, claims);
-                if (slot != ~0ULL)
-                    atomicMin((unsigned long long *)&S.slot[2 * slot + 1], (unsigned long long)pos);
-                if (S.score != nullptr && slot != ~0ULL) {
-                    atomicMax((unsigned long long *)&S.score[slot],
-                              (unsigned long long)__double_as_longlong(fabs(val) * cabs));
-                    if (fabs(val) > eps_plain_i) atomicOr(&S.plain[slot], 1);
+        // Evaluates one candidate; returns true when it passes and is new.
+        auto consider = [&](bool valid, u64 nu, u64 nd, double val, u64 pos, int sg) {
+            bool pass = false;
+            u64 key = 0;
+            if (valid && fabs(val) > eps_i) {
+                if (wfn_lookup(w, nu, nd) < 0) {
+                    pass = true;
+                    key = set_key(w, nu, nd);
                 }
             }
-        }
-    };
-
-    const u64 rbase = (u64)row * (u64)rows_stride;
-    if constexpr (KIND == PYCI_WFN_DOCI) {
-        const int total = nou * nvu;
-        for (int e0 = wave * 64; e0 < total; e0 += HCI_WAVES * 64) {
-            const int e = e0 + lane;
-            const bool valid = e < total;
-            const int i = valid ? e / nvu : 0, j = valid ? e - (e / nvu) * nvu : 0;
-            const int pi = __shfl(packed, i), pj = __shfl(packed, j);
-            const int k = pi & 255, l = (pj >> 8) & 255;
-            double val = valid ? two[GIX(k, k, l, l)] : 0.0;
-            consider(valid, up ^ (1ULL << k) ^ (1ULL << l), 0ULL, val, rbase + (u64)e, 1);
-        }
-    } else {
-        // Position of a candidate in the reference's row order (alpha: for i, for j: single
-        // (i, j), FullCI the doubles with a beta single (k, l), then the doubles (k > i,
-        // l > j); beta after alpha, without the second kind): the single (i, j) at off(i, j).
-        const i64 mixed = KIND == PYCI_WFN_FULLCI ? (i64)nod * nvd : 0;
-        auto off = [](int no, int nv, i64 mid, int i, int j) -> i64 {
-            const i64 hv = (i64)nv * (nv - 1) / 2;
-            return ((i64)i * nv + j) * (1 + mid) + hv * ((i64)i * (no - 1) - (i64)i * (i - 1) / 2) +
-                   (i64)(no - 1 - i) * ((i64)j * (nv - 1) - (i64)j * (j - 1) / 2);
-        };
-        const i64 beta0 = KIND == PYCI_WFN_FULLCI ? off(nou, nvu, mixed, nou, 0) : 0;
-        // index of orbital r among the empty orbitals of string d
-        auto hole = [](u64 d, int r) { return r - __popcll(d & ((1ULL << r) - 1ULL)); };
-        int turn = 0;  // lists seen: the waves take them in turn
-        // the entries of a list above the threshold, in chunks of 64 lanes
-        auto walk = [&](const double *lv, const unsigned short *lrs, int len, auto &&take) {
-            for (int t0 = 0; t0 < len; t0 += 64) {
-                const int t = t0 + lane;
-                const double V = t < len ? lv[t] : 0.0;
-                const bool above = t < len && fabs(V) > eps_i;
-                if (__ballot(above) == 0) break;  // the list is sorted: nothing further passes
-                const unsigned rs = above ? lrs[t] : 0u;
-                take(above, V, (int)(rs & 255u), (int)(rs >> 8));
+            if (PASS == 1) {
+                local += __popcll(__ballot(pass));
+            } else if (PASS == 5) {
+                // the reference multiplies the element by (phase * c_i) (enpt2.cpp:122-205)
+                if (pass) {
+                    const u64 slot = set_insert(S, key, claims);
+                    if (slot != ~0ULL)
+                        atomicAdd(reinterpret_cast<double *>(&S.slot[2 * slot + 1]), val * ((double)sg * coeffs[row]));
+                }
+            } else if (PASS == 2) {
+                if (pass) {
+                    const u64 slot = set_insert(S, key, claims);
+                    if (slot != ~0ULL)
+                        atomicMin((unsigned long long *)&S.slot[2 * slot + 1], (unsigned long long)pos);
+                    if (S.score != nullptr && slot != ~0ULL) {
+                        atomicMax((unsigned long long *)&S.score[slot],
+                                  (unsigned long long)__double_as_longlong(fabs(val) * cabs));
+                        if (fabs(val) > eps_plain_i) atomicOr(&S.plain[slot], 1);
+                    }
+                }
             }
         };
-        // singles and same-spin doubles of one spin
-        auto spin = [&](bool beta) {
-            const u64 d = beta ? dn : up;
-            const int no = beta ? nod : nou, nv = beta ? nvd : nvu, so = beta ? 16 : 0;
-            const i64 mid = beta ? 0 : mixed;
-            const u64 at0 = rbase + (u64)(beta ? beta0 : 0);
-            // singles, where the bound reaches the threshold
-            for (int e0 = wave * 64; e0 < no * nv; e0 += HCI_WAVES * 64) {
+
+        const u64 rbase = (u64)row * (u64)rows_stride;
+        if constexpr (KIND == PYCI_WFN_DOCI) {
+            const int total = nou * nvu;
+            for (int e0 = wave * 64; e0 < total; e0 += HCI_WAVES * 64) {
                 const int e = e0 + lane;
-                const bool in = e < no * nv;
-                const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
-                const int ii = (__shfl(packed, i) >> so) & 255, jj = (__shfl(packed, j) >> (so + 8)) & 255;
-                const bool live = in && L.sb[ii * n + jj] * (1.0 + 1e-12) > eps_i;
-                double val = 0.0;
-                int sg = 1;
-                if (live) {
-                    double v = one[ii * n + jj];
-                    for (u64 x = up; x; x &= x - 1) {
-                        const int q = __builtin_ctzll(x);
-                        if (beta)
-                            v += two[GIX(ii, q, jj, q)];
-                        else
-                            v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                    }
-                    if (KIND == PYCI_WFN_FULLCI)
-                        for (u64 x = dn; x; x &= x - 1) {
+                const bool valid = e < total;
+                const int i = valid ? e / nvu : 0, j = valid ? e - (e / nvu) * nvu : 0;
+                const int pi = __shfl(packed, i), pj = __shfl(packed, j);
+                const int k = pi & 255, l = (pj >> 8) & 255;
+                double val = valid ? two[GIX(k, k, l, l)] : 0.0;
+                consider(valid, up ^ (1ULL << k) ^ (1ULL << l), 0ULL, val, rbase + (u64)e, 1);
+            }
+        } else {
+            // Position of a candidate in the reference's row order (alpha: for i, for j: single
+            // (i, j), FullCI the doubles with a beta single (k, l), then the doubles (k > i,
+            // l > j); beta after alpha, without the second kind): the single (i, j) at off(i, j).
+            const i64 mixed = KIND == PYCI_WFN_FULLCI ? (i64)nod * nvd : 0;
+            auto off = [](int no, int nv, i64 mid, int i, int j) -> i64 {
+                const i64 hv = (i64)nv * (nv - 1) / 2;
+                return ((i64)i * nv + j) * (1 + mid) + hv * ((i64)i * (no - 1) - (i64)i * (i - 1) / 2) +
+                       (i64)(no - 1 - i) * ((i64)j * (nv - 1) - (i64)j * (j - 1) / 2);
+            };
+            const i64 beta0 = KIND == PYCI_WFN_FULLCI ? off(nou, nvu, mixed, nou, 0) : 0;
+            // index of orbital r among the empty orbitals of string d
+            auto hole = [](u64 d, int r) { return r - __popcll(d & ((1ULL << r) - 1ULL)); };
+            int turn = 0;  // lists seen: the waves take them in turn
+            // the entries of a list above the threshold, in chunks of 64 lanes
+            auto walk = [&](const double *lv, const unsigned short *lrs, int len, auto &&take) {
+                for (int t0 = 0; t0 < len; t0 += 64) {
+                    const int t = t0 + lane;
+                    const double V = t < len ? lv[t] : 0.0;
+                    const bool above = t < len && fabs(V) > eps_i;
+                    if (__ballot(above) == 0) break;  // the list is sorted: nothing further passes
+                    const unsigned rs = above ? lrs[t] : 0u;
+                    take(above, V, (int)(rs & 255u), (int)(rs >> 8));
+                }
+            };
+            // singles and same-spin doubles of one spin
+            auto spin = [&](bool beta) {
+                const u64 d = beta ? dn : up;
+                const int no = beta ? nod : nou, nv = beta ? nvd : nvu, so = beta ? 16 : 0;
+                const i64 mid = beta ? 0 : mixed;
+                const u64 at0 = rbase + (u64)(beta ? beta0 : 0);
+                // singles, where the bound reaches the threshold
+                for (int e0 = wave * 64; e0 < no * nv; e0 += HCI_WAVES * 64) {
+                    const int e = e0 + lane;
+                    const bool in = e < no * nv;
+                    const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
+                    const int ii = (__shfl(packed, i) >> so) & 255, jj = (__shfl(packed, j) >> (so + 8)) & 255;
+                    const bool live = in && L.sb[ii * n + jj] * (1.0 + 1e-12) > eps_i;
+                    double val = 0.0;
+                    int sg = 1;
+                    if (live) {
+                        double v = one[ii * n + jj];
+                        for (u64 x = up; x; x &= x - 1) {
                             const int q = __builtin_ctzll(x);
                             if (beta)
-                                v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
-                            else
                                 v += two[GIX(ii, q, jj, q)];
+                            else
+                                v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
                         }
-                    val = v;
-                    if (PASS == 5) sg = phase1(d, ii, jj);
+                        if (KIND == PYCI_WFN_FULLCI)
+                            for (u64 x = dn; x; x &= x - 1) {
+                                const int q = __builtin_ctzll(x);
+                                if (beta)
+                                    v += two[GIX(ii, q, jj, q)] - two[GIX(ii, q, q, jj)];
+                                else
+                                    v += two[GIX(ii, q, jj, q)];
+                            }
+                        val = v;
+                        if (PASS == 5) sg = phase1(d, ii, jj);
+                    }
+                    const u64 x = d ^ (1ULL << ii) ^ (1ULL << jj);
+                    consider(live, beta ? up : x, beta ? x : dn, val, at0 + (u64)off(no, nv, mid, i, j), sg);
                 }
-                const u64 x = d ^ (1ULL << ii) ^ (1ULL << jj);
-                consider(live, beta ? up : x, beta ? x : dn, val, at0 + (u64)off(no, nv, mid, i, j), sg);
-            }
-            // doubles: the occupied pairs whose list begins above the threshold, a lane each
-            const int np = no * (no - 1) / 2;
-            for (int p0 = 0; p0 < np; p0 += 64) {
-                int i = 0, k = 0;
-                if (p0 + lane < np) tri_decode(p0 + lane, i, k);
-                const int ii0 = (__shfl(packed, i) >> so) & 255, kk0 = (__shfl(packed, k) >> so) & 255;
-                u64 todo = __ballot(p0 + lane < np && L.top[kk0 * (kk0 - 1) / 2 + ii0] > eps_i);
-                for (; todo; todo &= todo - 1) {
-                    if (turn++ % HCI_WAVES != wave) continue;
-                    const int from = __builtin_ctzll(todo);
-                    const int pi = __shfl(i, from), pk = __shfl(k, from);
-                    const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
-                    const i64 lb = (i64)(kk * (kk - 1) / 2 + ii) * L.npair;
-                    walk(L.v + lb, L.rs + lb, L.npair, [&](bool above, double V, int r, int s2) {
-                        const bool free = above && !((d >> r) & 1ULL) && !((d >> s2) & 1ULL);
-                        const int j = hole(d, r), l = hole(d, s2);
-                        int sg = 1;
-                        if (PASS == 5 && free) sg = phase2(d, ii, kk, r, s2);
-                        const i64 o = off(no, nv, mid, pi, j) + 1 + mid + (i64)(pk - pi - 1) * (nv - 1 - j) + (l - j - 1);
-                        const u64 x = d ^ (1ULL << ii) ^ (1ULL << kk) ^ (1ULL << r) ^ (1ULL << s2);
-                        consider(free, beta ? up : x, beta ? x : dn, V, at0 + (u64)o, sg);
-                    });
+                // doubles: the occupied pairs whose list begins above the threshold, a lane each
+                const int np = no * (no - 1) / 2;
+                for (int p0 = 0; p0 < np; p0 += 64) {
+                    int i = 0, k = 0;
+                    if (p0 + lane < np) tri_decode(p0 + lane, i, k);
+                    const int ii0 = (__shfl(packed, i) >> so) & 255, kk0 = (__shfl(packed, k) >> so) & 255;
+                    u64 todo = __ballot(p0 + lane < np && L.top[kk0 * (kk0 - 1) / 2 + ii0] > eps_i);
+                    for (; todo; todo &= todo - 1) {
+                        if (turn++ % HCI_WAVES != wave) continue;
+                        const int from = __builtin_ctzll(todo);
+                        const int pi = __shfl(i, from), pk = __shfl(k, from);
+                        const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
+                        const i64 lb = (i64)(kk * (kk - 1) / 2 + ii) * L.npair;
+                        walk(L.v + lb, L.rs + lb, L.npair, [&](bool above, double V, int r, int s2) {
+                            const bool free = above && !((d >> r) & 1ULL) && !((d >> s2) & 1ULL);
+                            const int j = hole(d, r), l = hole(d, s2);
+                            int sg = 1;
+                            if (PASS == 5 && free) sg = phase2(d, ii, kk, r, s2);
+                            const i64 o = off(no, nv, mid, pi, j) + 1 + mid + (i64)(pk - pi - 1) * (nv - 1 - j) + (l - j - 1);
+                            const u64 x = d ^ (1ULL << ii) ^ (1ULL << kk) ^ (1ULL << r) ^ (1ULL << s2);
+                            consider(free, beta ? up : x, beta ? x : dn, V, at0 + (u64)o, sg);
+                        });
+                    }
                 }
-            }
-        };
-        spin(false);
-        if constexpr (KIND == PYCI_WFN_FULLCI) {
-            // doubles of both spins
-            for (int p0 = 0; p0 < nou * nod; p0 += 64) {
-                const int e = p0 + lane < nou * nod ? p0 + lane : 0, i = e / nod, k = e - i * nod;
-                const int ii0 = __shfl(packed, i) & 255, kk0 = (__shfl(packed, k) >> 16) & 255;
-                u64 todo = __ballot(p0 + lane < nou * nod && L.topo[ii0 * n + kk0] > eps_i);
-                for (; todo; todo &= todo - 1) {
-                    if (turn++ % HCI_WAVES != wave) continue;
-                    const int from = __builtin_ctzll(todo);
-                    const int pi = __shfl(i, from), pk = __shfl(k, from);
-                    const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
-                    const i64 lb = (i64)(ii * n + kk) * n * n;
-                    walk(L.vo + lb, L.rso + lb, n * n, [&](bool above, double V, int r, int s2) {
-                        const bool free = above && !((up >> r) & 1ULL) && !((dn >> s2) & 1ULL);
-                        int sg = 1;
-                        if (PASS == 5 && free) sg = phase1(up, ii, r) * phase1(dn, kk, s2);
-                        const i64 o = off(nou, nvu, mixed, pi, hole(up, r)) + 1 + (i64)pk * nvd + hole(dn, s2);
-                        consider(free, up ^ (1ULL << ii) ^ (1ULL << r), dn ^ (1ULL << kk) ^ (1ULL << s2), V,
-                                 rbase + (u64)o, sg);
-                    });
+            };
+            spin(false);
+            if constexpr (KIND == PYCI_WFN_FULLCI) {
+                // doubles of both spins
+                for (int p0 = 0; p0 < nou * nod; p0 += 64) {
+                    const int e = p0 + lane < nou * nod ? p0 + lane : 0, i = e / nod, k = e - i * nod;
+                    const int ii0 = __shfl(packed, i) & 255, kk0 = (__shfl(packed, k) >> 16) & 255;
+                    u64 todo = __ballot(p0 + lane < nou * nod && L.topo[ii0 * n + kk0] > eps_i);
+                    for (; todo; todo &= todo - 1) {
+                        if (turn++ % HCI_WAVES != wave) continue;
+                        const int from = __builtin_ctzll(todo);
+                        const int pi = __shfl(i, from), pk = __shfl(k, from);
+                        const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
+                        const i64 lb = (i64)(ii * n + kk) * n * n;
+                        walk(L.vo + lb, L.rso + lb, n * n, [&](bool above, double V, int r, int s2) {
+                            const bool free = above && !((up >> r) & 1ULL) && !((dn >> s2) & 1ULL);
+                            int sg = 1;
+                            if (PASS == 5 && free) sg = phase1(up, ii, r) * phase1(dn, kk, s2);
+                            const i64 o = off(nou, nvu, mixed, pi, hole(up, r)) + 1 + (i64)pk * nvd + hole(dn, s2);
+                            consider(free, up ^ (1ULL << ii) ^ (1ULL << r), dn ^ (1ULL << kk) ^ (1ULL << s2), V,
+                                     rbase + (u64)o, sg);
+                        });
+                    }
                 }
+                spin(true);
             }
-            spin(true);
         }
     }
     if (PASS != 1) {
@@ -463,7 +466,7 @@ struct HbTables {
 template <int PASS>
 static void launch_hci(int kind, const WfnView &w, const HamView &H, const double *c, double eps, double eps_plain,
                        i64 stride, const NewSet &S, unsigned long long *count, hipStream_t s, const HbLists &L) {
-    const unsigned g = (unsigned)w.ndet, t = HCI_WAVES * 64;
+    const unsigned g = (unsigned)std::min(w.ndet, HCI_BLOCKS), t = HCI_WAVES * 64;
     if (kind == PYCI_WFN_DOCI)
         k_hci<PYCI_WFN_DOCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     else if (kind == PYCI_WFN_FULLCI)

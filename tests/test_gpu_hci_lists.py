@@ -1,10 +1,13 @@
 """FullCI selection and ENPT2 through sorted integral lists against the CPU oracle, which
 evaluates every excitation: same determinants in the same order, same energy."""
+import math
+
 import numpy as np
 import numpy.testing as npt
 import pytest
 
 import pyci_amd as pyci
+from pyci_amd.synthetic import seeded_integrals, spin_orbital
 
 pytestmark = pytest.mark.gpu
 
@@ -28,3 +31,26 @@ def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
         npt.assert_allclose(e, ref, rtol=1e-11)
         assert pyci.add_hci(ham, w, c, eps=eps) == len(expect)
         npt.assert_array_equal(w.to_det_array().reshape(-1, 2)[len(dets):], expect)
+
+
+def test_rows_past_two_to_the_24():
+    """Additions from the last of 17,000,000 determinants (the first of 28 spin orbitals and 11
+    electrons in colex order), which are those of that determinant alone outside the set."""
+    nb, nocc, ndet = 28, 11, 17_000_000
+    _, one, two = seeded_integrals(nb // 2, 6, 77)
+    one, two = spin_orbital(one, two)
+    ham = pyci.hamiltonian(0.0, one, two)
+    full = pyci.genci_wfn(nb, nocc, 0)
+    full.add_all_dets()
+    dets = full.to_det_array()[:ndet]
+    last = pyci.genci_wfn(nb, nocc, 0, dets[-1:])
+    pyci.add_hci(ham, last, np.ones(1), eps=1e-3)
+    expect = last.to_det_array()[1:].ravel()
+    expect = expect[[sum(math.comb(p, k + 1) for k, p in enumerate(p for p in range(nb) if int(d) >> p & 1)) >= ndet
+                     for d in expect]]
+    c = np.zeros(ndet)
+    c[-1] = 1.0
+    w = pyci.genci_wfn(nb, nocc, 0, dets)
+    assert len(expect) > 0
+    assert pyci.add_hci(ham, w, c, eps=1e-3) == len(expect)
+    npt.assert_array_equal(w.to_det_array()[ndet:].ravel(), expect)
