@@ -326,13 +326,13 @@ __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, co
                 const int no = beta ? nod : nou, nv = beta ? nvd : nvu, so = beta ? 16 : 0;
                 const i64 mid = beta ? 0 : mixed;
                 const u64 at0 = rbase + (u64)(beta ? beta0 : 0);
-                // singles, where the bound reaches the threshold
+                // singles, unless the bound stays below the threshold (one that is NaN tells nothing)
                 for (int e0 = wave * 64; e0 < no * nv; e0 += HCI_WAVES * 64) {
                     const int e = e0 + lane;
                     const bool in = e < no * nv;
                     const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
                     const int ii = (__shfl(packed, i) >> so) & 255, jj = (__shfl(packed, j) >> (so + 8)) & 255;
-                    const bool live = in && L.sb[ii * n + jj] * (1.0 + 1e-12) > eps_i;
+                    const bool live = in && !(L.sb[ii * n + jj] * (1.0 + 1e-12) <= eps_i);
                     double val = 0.0;
                     int sg = 1;
                     if (live) {

@@ -33,6 +33,27 @@ def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
         npt.assert_array_equal(w.to_det_array().reshape(-1, 2)[len(dets):], expect)
 
 
+@pytest.mark.parametrize("kind,nb,nu,nd", [("fullci", 8, 3, 2), ("genci", 12, 4, 0)])
+@pytest.mark.parametrize("value", [np.nan, np.inf])
+def test_non_finite_integrals_match_oracle(oracle, kind, nb, nu, nd, value):
+    """A NaN or an infinity among the integrals decides about the excitations whose element it
+    enters, and about no others."""
+    rng = np.random.default_rng(nb)
+    one = rng.normal(size=(nb, nb))
+    two = rng.normal(size=(nb,) * 4)
+    two[0, 5, 4, 5] = two[1, 2, 6, 3] = value
+    strings = [[sum(1 << int(p) for p in rng.permutation(nb)[:k]) for _ in range(12)] for k in (nu, nd)]
+    dets = np.unique(np.array(strings[:2 if kind == "fullci" else 1], dtype=np.uint64).T, axis=0)
+    c = rng.normal(size=len(dets))
+    cls = {"fullci": pyci.fullci_wfn, "genci": pyci.genci_wfn}[kind]
+    ham = pyci.hamiltonian(0.0, one, two)
+    for eps in (0.0, 0.1, 2.0):
+        w = cls(nb, nu, nd, dets.reshape((-1, 2, 1) if kind == "fullci" else (-1, 1)))
+        expect = oracle.add_hci(kind, nb, nu, nd, dets, one, two, c, eps).reshape(-1, dets.shape[1])
+        assert pyci.add_hci(ham, w, c, eps=eps) == len(expect)
+        npt.assert_array_equal(w.to_det_array().reshape(-1, dets.shape[1])[len(dets):], expect)
+
+
 def test_rows_past_two_to_the_24():
     """Additions from the last of 17,000,000 determinants (the first of 28 spin orbitals and 11
     electrons in colex order), which are those of that determinant alone outside the set."""
