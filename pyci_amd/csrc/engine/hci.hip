@@ -868,8 +868,10 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
     }
     DevBuf<double> part(PT2_BLOCKS);
     const size_t lds = sizeof(double) * (size_t)(H.n + H.n * H.n * (w.nkey == 2 ? 2 : 1));
-    if (lds > 60000)  // 63 and 64 orbitals of two spins: above 64 KB with the reduction's
-        PE_HIP(hipFuncSetAttribute((const void *)k_pt2_terms, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    // tables of two spins from 59 orbitals on, with the kernel's own 10 KB, are more than the
+    // 64 KB that need no attribute: set for the largest, for callers on other threads
+    PE_HIP(hipFuncSetAttribute((const void *)k_pt2_terms, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)(sizeof(double) * (64 + 2 * 64 * 64))));
     k_pt2_terms<<<PT2_BLOCKS, 256, lds, s>>>(w, S, cap, H, e, part.p);
     PE_LAUNCH_CHECK();
     std::vector<double> hp(PT2_BLOCKS);

@@ -13,8 +13,10 @@ pytestmark = pytest.mark.gpu
 
 
 # no electrons or no holes of a spin, no same-spin pairs, the longest strings that are
-# their own key and the first that are ranked, a list of 2,048 and the longest lists
-@pytest.mark.parametrize("nb,nu,nd", [(7, 3, 0), (6, 6, 3), (20, 1, 1), (32, 2, 2), (33, 2, 1), (46, 2, 1), (64, 1, 1)])
+# their own key and the first that are ranked, a list of 2,048 and the longest lists, the
+# sizes around which the terms' tables need more than 64 KB of LDS
+@pytest.mark.parametrize("nb,nu,nd", [(7, 3, 0), (6, 6, 3), (20, 1, 1), (32, 2, 2), (33, 2, 1), (46, 2, 1),
+                                      (58, 1, 1), (59, 1, 1), (60, 1, 1), (61, 1, 1), (64, 1, 1)])
 def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
     rng = np.random.default_rng(nb)
     one = rng.normal(size=(nb, nb))
