@@ -117,18 +117,22 @@ k_spmm(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
 }
 
 // Single vector, a row per wave: every lane issues the column and value loads of U entries
-// (non-temporal: the CSR is streamed once per sigma and must not evict X), also in a row's
-// last chunk, then their U gathers of X. The gathers bound it: an 8-byte element costs a
-// 128-byte line from L2 unless L1 still holds it.
+// (non-temporal: the CSR is streamed once per sigma and must not evict X), then their U
+// gathers of X. A row's last chunk takes part with the lanes that have an entry: loads beyond
+// the row cost requests, and an element of X that belongs to no entry may be an infinity or a
+// NaN. The gathers bound it: an 8-byte element costs a 128-byte line from L2 unless L1 still
+// holds it.
 //   WAVES 16, U 1   rows of a full space, sorted in column order: 16 neighbouring rows (most
 //                   with the same alpha string) walk the same lines of X in step, so L1 serves
 //                   them; a wider window per lane spreads the waves over more lines than L1
 //                   holds. nbasis 12 (18.6 GB): 4.11 ms (4.5 TB/s) against 5.18-6.4 with U
-//                   2..16 and 4 waves; nbasis 10: 160 us against 164-224.
-//   WAVES 4, U 16   other large sets: nothing to share, most loads in flight (100,000 FullCI
-//                   determinants of 24 orbitals: 527 us, 572-643 with U 2..12).
-//   WAVES 4, U 2, 4 sets below a few thousand rows, one or two chunks a row: 3,000 GenCI
-//                   determinants 4.7 us (7.4 with U 16), DOCI of 11,628 rows of 71 5.8 (7.8).
+//                   2..16 and 4 waves; nbasis 10: 147 us against 156-200. And sets of short
+//                   rows, two chunks at most (400,000 FullCI determinants of 32 entries a row
+//                   114 us, 172 with 4 waves and U 3; DOCI of 74,613 rows of 97 33 us, 40).
+//   WAVES 4, U 3    other sets, whose entries are too few or too thin for panels of X in LDS
+//                   (100,000 GenCI determinants of 154 entries a row 90 us, 99 with 16 waves,
+//                   94 with U 6; full spaces of 15,876 rows of 561 26.6 us, 27-28 with U 2..8,
+//                   36 with U 1).
 template <int U, int WAVES, typename VT, typename XT>
 __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(1, WAVES == 4 ? 4 : 8)))
 k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__restrict__ cols,
@@ -137,37 +141,41 @@ k_spmv(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
     const i64 blk = xcd_row_block(blockIdx.x, nblocks);
     const i64 row = blk * WAVES + (threadIdx.x >> 6);
     if (blk >= nblocks || row >= nrow) return;
-    const i64 beg = rowptr[row], len = rowptr[row + 1] - beg;
+    const i64 beg = rowptr[row];
+    const int len = (int)(rowptr[row + 1] - beg);
     cols += beg;
     vals += beg;
     XT acc = (XT)0;
-    for (i64 p0 = 0; p0 < len; p0 += U * 64) {
-        const bool whole = p0 + U * 64 <= len;
+    int p = lane;
+    for (; p - lane + U * 64 <= len; p += U * 64) {
         int c[U];
         VT v[U];
-        if (whole) {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                c[u] = __builtin_nontemporal_load(&cols[p0 + lane + u * 64]);
-                v[u] = __builtin_nontemporal_load(&vals[p0 + lane + u * 64]);
-            }
-        } else {
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const i64 p = p0 + lane + u * 64, q = p < len ? p : len - 1;
-                c[u] = __builtin_nontemporal_load(&cols[q]);
-                const VT t = __builtin_nontemporal_load(&vals[q]);
-                v[u] = p < len ? t : (VT)0;
-            }
-        }
         XT x[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) x[u] = X[c[u]];
-        if (!whole) {  // an infinity or a NaN times the 0 beyond the row would be a NaN
-#pragma unroll
-            for (int u = 0; u < U; ++u)
-                if (p0 + lane + u * 64 >= len) x[u] = (XT)0;
+        for (int u = 0; u < U; ++u) {
+            c[u] = __builtin_nontemporal_load(&cols[p + u * 64]);
+            v[u] = __builtin_nontemporal_load(&vals[p + u * 64]);
         }
+#pragma unroll
+        for (int u = 0; u < U; ++u) x[u] = X[c[u]];
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc += (XT)v[u] * x[u];
+    }
+    if (p - lane < len) {
+        int c[U];
+        VT v[U];
+        XT x[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            c[u] = 0, v[u] = (VT)0, x[u] = (XT)0;
+            if (p + u * 64 < len) {
+                c[u] = __builtin_nontemporal_load(&cols[p + u * 64]);
+                v[u] = __builtin_nontemporal_load(&vals[p + u * 64]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (p + u * 64 < len) x[u] = X[c[u]];
 #pragma unroll
         for (int u = 0; u < U; ++u) acc += (XT)v[u] * x[u];
     }
@@ -413,9 +421,12 @@ static void spmv(const pyci_op *op, const VT *vals, const XT *X, XT *Y, hipStrea
     const SpmvPlan &P = op->spmv;
     if (P.npanel > 0) {
         // 16 lanes a row take 64 rows at a time with a quarter of the instructions per entry
-        // (60,000 GenCI determinants 119 us, 160 with a wave a row); with few rows a block the
-        // last of its rounds is mostly empty (17,317 FullCI determinants 31 us, 22.5)
-        if (nrow >= (i64)P.nblk * 160)
+        // (60,000 GenCI determinants 119 us, 160 with a wave a row). With few rows a block the
+        // last of its rounds is mostly empty, and a wave a row is the better one where a row's
+        // entries of a panel keep it busy (17,317 FullCI determinants 31 us, 22.5; 10,000
+        // GenCI ones of 426 entries 14.6, 13.0), not where they leave most of it idle (30,000
+        // FullCI ones of 2 x 41 entries 16.3, 29.4; the two meet near 200)
+        if (nrow >= (i64)P.nblk * 160 || op->nnz < nrow * P.npanel * 200)
             launch_lds<16, VT, XT>(op, vals, X, Y, s);
         else
             launch_lds<64, VT, XT>(op, vals, X, Y, s);
@@ -426,14 +437,11 @@ static void spmv(const pyci_op *op, const VT *vals, const XT *X, XT *Y, hipStrea
         kern<<<(unsigned)grid, waves * 64, 0, s>>>(nrow, nblocks, rp, c, vals, X, Y);
         PE_LAUNCH_CHECK();
     };
-    if (P.ordered && nrow >= 32768)
+    // below 4,096 rows blocks of 16 would not reach every CU
+    if ((P.ordered && nrow >= 32768) || (mean <= 100 && nrow >= 4096))
         launch(k_spmv<1, 16, VT, XT>, 16);
-    else if (mean <= 128)
-        launch(k_spmv<2, 4, VT, XT>, 4);
-    else if (op->nnz < SPMV_LDS_MIN_NNZ)
-        launch(k_spmv<4, 4, VT, XT>, 4);
     else
-        launch(k_spmv<16, 4, VT, XT>, 4);
+        launch(k_spmv<3, 4, VT, XT>, 4);
 }
 
 template <typename VT, typename XT>
