@@ -370,6 +370,12 @@ __global__ void __launch_bounds__(256) k_spmm_any(i64 nrow, i64 nblocks, int nv,
     }
 }
 
+template <int LANES, typename XT>
+static void allow_lds() {
+    PE_HIP(hipFuncSetAttribute((const void *)k_spmv_lds<LANES, XT, XT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)(sizeof(XT) * (SPMV_PANEL + 1))));
+}
+
 // Which single-vector product serves an operator's rows, and the plan of the one that
 // needs one. Called when the rows are final (the operator's build).
 void spmv_plan(pyci_op *op, bool column_ordered_space) {
@@ -383,6 +389,11 @@ void spmv_plan(pyci_op *op, bool column_ordered_space) {
     hipStream_t s = op->ctx->stream;
     int cus = 0;
     PE_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, op->ctx->device));
+    // a kernel's attribute belongs to a device: set for the operator's with every plan
+    allow_lds<16, double>();
+    allow_lds<64, double>();
+    allow_lds<16, float>();
+    allow_lds<64, float>();
     P.npanel = (int)npanel;
     P.nblk = cus;
     P.bounds.alloc((size_t)(cus + 1));
@@ -399,12 +410,6 @@ void spmv_plan(pyci_op *op, bool column_ordered_space) {
 template <int LANES, typename VT, typename XT>
 static void launch_lds(const pyci_op *op, const VT *vals, const XT *X, XT *Y, hipStream_t s) {
     const size_t lds = sizeof(XT) * (SPMV_PANEL + 1);
-    static const bool attr = [&] {
-        PE_HIP(hipFuncSetAttribute((const void *)k_spmv_lds<LANES, VT, XT>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-        return true;
-    }();
-    (void)attr;
     const SpmvPlan &P = op->spmv;
     // at most 25 rows of a block are longer than a 24th of its share
     const i64 long_len = std::max<i64>(1024, op->nnz / ((i64)P.nblk * 24));
