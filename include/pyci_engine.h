@@ -7,8 +7,9 @@
  * one of the PYCI_E* codes below; pyci_last_error() then holds a message for the
  * calling thread. Host pointers are never retained after a call returns; device
  * memory belongs to the handle that allocated it and is freed by its *_destroy.
- * Calls on one context are serialised on that context's HIP stream and are not
- * re-entrant; different contexts may be used from different threads.
+ * The GPU work of a context is ordered on its HIP stream; its calls are not
+ * re-entrant, except pyci_compute_rdms, pyci_add_hci and pyci_compute_enpt2 on
+ * different wave functions. Different contexts may be used from different threads.
  *
  * Determinant layout (as the reference's `dets` vectors, one 64-bit word per
  * spin string): DOCI and GenCI dets are one uint64 each; FullCI dets are two

@@ -538,25 +538,23 @@ static i64 set_capacity(unsigned long long upper) {
     return std::max<i64>(1024, (want + want / 2 + 255) / 256 * 256);
 }
 
-// The table's memory: the context's, kept between calls up to 4 GB (allocating and freeing
-// it on each call took longer than filling it), else the caller's own.
-static u64 *set_table(pyci_ctx *ctx, DevBuf<u64> &own, i64 cap) {
-    DevBuf<u64> &buf = 2 * cap <= (i64)1 << 29 ? ctx->hci_table : own;
-    buf.ensure((size_t)(2 * cap));
-    return buf.p;
-}
+// The table's memory comes from the context, which keeps up to 4 GB between calls
+// (allocating and freeing it on each call took longer than filling it).
+using SetTable = Lease<DevBuf<u64>>;
 
 // Passes 1-2 of the selection: the set of new candidates (|H_ji| > eps/|c_i|,
 // not in the wave function) with their first-occurrence positions; then its
 // claimed slots ordered by that position (a radix sort), which is the order of
 // first occurrence in the serial enumeration: slots[0 .. nnew).
 struct HciRun {
-    DevBuf<u64> table, score, slots;
+    SetTable table;
+    DevBuf<u64> score, slots;
     DevBuf<int> plain, ovf;
     DevBuf<unsigned long long> cnt;
     NewSet S{};
     i64 stride = 0, nnew = 0;
     unsigned long long S_unique_host = 0;  // claimed slots after pass 2
+    explicit HciRun(pyci_ctx *ctx) : table(ctx->hci_table) {}
 };
 
 static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double eps, double eps_plain, bool pool,
@@ -590,7 +588,8 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
     if (upper == 0) return;
     i64 cap = set_capacity(upper);
     for (;;) {
-        u64 *table = set_table(ctx, R.table, cap);
+        R.table.buf.ensure((size_t)(2 * cap));
+        u64 *table = R.table.buf.p;
         if (pool) {
             R.score.alloc((size_t)cap);
             R.plain.alloc((size_t)cap);
@@ -649,7 +648,7 @@ i64 add_hci_device(pyci_ham *ham, pyci_wfn *wfn, const double *coeffs_host, doub
     if (nd == 0) return 0;
     DevBuf<double> dc((size_t)nd);
     PE_HIP(hipMemcpyAsync(dc.p, coeffs_host, sizeof(double) * nd, hipMemcpyHostToDevice, s));
-    HciRun R;
+    HciRun R(ctx);
     hci_collect(ham, wfn, dc.p, eps, eps, false, R);
     const i64 nnew = R.nnew;
     if (nnew == 0) return 0;
@@ -691,7 +690,7 @@ void hci_pool_device(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double eps,
     P.n = 0;
     P.nplain = 0;
     if (wfn->ndet == 0) return;
-    HciRun R;
+    HciRun R(wfn->ctx);
     hci_collect(ham, wfn, dc, eps_pool, eps, true, R);
     if (R.nnew == 0) return;
     P.n = R.nnew;
@@ -848,10 +847,11 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
     PE_HIP(hipStreamSynchronize(s));
     if (upper == 0) return 0.0;
     i64 cap = set_capacity(upper);
-    DevBuf<u64> own;
+    SetTable kept(ctx->hci_table);
     unsigned long long uniq = 0;
     for (;;) {
-        u64 *table = set_table(ctx, own, cap);
+        kept.buf.ensure((size_t)(2 * cap));
+        u64 *table = kept.buf.p;
         k_set_clear<<<4096, 256, 0, s>>>(table, 0ULL, nullptr, nullptr, cap);
         PE_LAUNCH_CHECK();
         PE_HIP(hipMemsetAsync(cnt.p + 1, 0, sizeof(unsigned long long), s));

@@ -5,8 +5,10 @@
 
 #include <cstdint>
 #include <memory>
+#include <mutex>
 #include <stdexcept>
 #include <string>
+#include <utility>
 #include <vector>
 
 #include "pyci_engine.h"
@@ -103,6 +105,15 @@ struct HostBuf {
     HostBuf() = default;
     HostBuf(const HostBuf &) = delete;
     HostBuf &operator=(const HostBuf &) = delete;
+    HostBuf(HostBuf &&o) noexcept : p(o.p), n(o.n) { o.p = nullptr, o.n = 0; }
+    HostBuf &operator=(HostBuf &&o) noexcept {
+        if (this != &o) {
+            release();
+            p = o.p, n = o.n;
+            o.p = nullptr, o.n = 0;
+        }
+        return *this;
+    }
     ~HostBuf() { release(); }
     void ensure(size_t count) {
         if (!p || n < count) alloc(count);
@@ -129,6 +140,35 @@ struct HostBuf {
 }  // namespace pe
 
 namespace pe {
+// A working buffer of up to `most` elements that the context keeps between calls. A call takes
+// it out for as long as it runs (Lease): the Python layer has one context for all threads and
+// calls without the interpreter's lock, so a second caller finds none and allocates its own.
+// The larger of what comes back is kept.
+template <class Buf>
+struct Kept {
+    const size_t most;
+    std::mutex lock;
+    Buf idle;
+    explicit Kept(size_t most_) : most(most_) {}
+};
+
+template <class Buf>
+struct Lease {
+    Kept<Buf> &home;
+    Buf buf;
+    explicit Lease(Kept<Buf> &h) : home(h) {
+        std::lock_guard<std::mutex> g(home.lock);
+        std::swap(buf, home.idle);
+    }
+    Lease(const Lease &) = delete;
+    Lease &operator=(const Lease &) = delete;
+    // work still queued on it is on the context's stream, ahead of the next holder's
+    ~Lease() {
+        std::lock_guard<std::mutex> g(home.lock);
+        if (buf.n <= home.most && buf.n > home.idle.n) std::swap(buf, home.idle);
+    }
+};
+
 // Working memory of one Davidson run (davidson.hip). The context keeps one set per
 // parity-sector stream between solves, so that a solve allocates nothing once the
 // sizes have been seen; the sets are released with the context.
@@ -153,8 +193,8 @@ struct pyci_ctx {
     hipStream_t stream2 = nullptr;
     pe::DevBuf<unsigned char> mf_ws2;
     std::unique_ptr<pe::DavBufs> dav[2];  // solver working memory per sector stream
-    pe::DevBuf<pe::u64> hci_table;    // hash set of the selection and ENPT2 passes (at most 4 GB)
-    pe::HostBuf<double> rdm_out;      // page-locked result of the full-space density matrices (at most 16 MB)
+    pe::Kept<pe::DevBuf<pe::u64>> hci_table{(size_t)1 << 29};  // hash set of the selection and ENPT2 passes (4 GB)
+    pe::Kept<pe::HostBuf<double>> rdm_out{(size_t)2 << 20};    // page-locked density matrices (16 MB)
     double *noalloc_ws = nullptr;     // the fixed workspace of the allocation-free product on this device
 };
 

@@ -363,7 +363,8 @@ void rf_result(pyci_ctx *ctx, const RfShape &S, int R, const double *acc, double
     const i64 n2 = (i64)S.n * S.n, s1 = (S.genci ? 1 : 2) * n2, nout = s1 + (S.genci ? 1 : 3) * n2 * n2;
     const bool direct = nout <= (i64)2 << 20;
     DevBuf<double> dout;
-    HostBuf<double> &host = ctx->rdm_out;
+    Lease<HostBuf<double>> out(ctx->rdm_out);
+    HostBuf<double> &host = out.buf;
     if (direct)
         host.ensure((size_t)nout);
     else
