@@ -742,51 +742,56 @@ __global__ void k_sorted_meta(i64 row0, i64 nr, i64 rowlen, i64 nsd, SortedRows 
 }
 
 // lo[0] = min, lo[1] = max over the determinants of the occupied orbitals below h;
-// lo[2] is set where a determinant has other electron counts than nu and nd
-__global__ void k_low_range(const u64 *dets, i64 ndet, int nkey, int h, int nu, int nd, int *lo) {
-    int mn = 64, mx = 0, bad = 0;
-    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < ndet; i += (i64)gridDim.x * blockDim.x) {
-        const u64 d = dets[i * nkey];
+// with `strict` lo[2] is set where a determinant has other electron counts than the wave
+// function's or an orbital beyond its basis, or is in the set twice (the index finds one place)
+__global__ void k_low_range(WfnView w, int h, bool strict, int *lo) {
+    int mn = 64, mx = 0;
+    bool bad = false;
+    for (i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x; i < w.ndet; i += (i64)gridDim.x * blockDim.x) {
+        const u64 d = w.dets[i * w.nkey], e = w.nkey == 2 ? w.dets[i * 2 + 1] : 0ULL;
         const int c = __popcll(d & full_mask(h));
         mn = min(mn, c);
         mx = max(mx, c);
-        bad |= __popcll(d) != nu || (nkey == 2 && __popcll(dets[i * 2 + 1]) != nd);
+        if (strict && !bad)
+            bad = __popcll(d) != w.nup || (w.nkey == 2 && __popcll(e) != w.ndn) || ((d | e) & ~full_mask(w.nb)) != 0 ||
+                  wfn_lookup(w, d, e) != i;
     }
     for (int o = 32; o > 0; o >>= 1) {
         mn = min(mn, __shfl_xor(mn, o));
         mx = max(mx, __shfl_xor(mx, o));
-        bad |= __shfl_xor(bad, o);
     }
+    const bool any = __ballot(bad) != 0;
     if ((threadIdx.x & 63) == 0) {
         atomicMin(lo, mn);
         atomicMax(lo + 1, mx);
-        if (bad) atomicMax(lo + 2, 1);
+        if (any) atomicMax(lo + 2, 1);
     }
 }
 
 // What the row kernels may take for granted of a set. szh: GenCI, nbasis / 2 if every
 // determinant has the same number of occupied spin orbitals in the lower half (a set of one
 // Sz in the alpha-then-beta ordering), else 0: an excitation that changes that number then
-// cannot find a column. occ: every determinant has the wave function's electron counts.
+// cannot find a column. sound (looked at with `strict`): every determinant has the wave
+// function's electron counts, lies within its basis and is there once.
 struct SetTraits {
     int szh;
-    bool occ;
+    bool sound;
 };
 
-static SetTraits set_traits(const pyci_wfn *wfn, hipStream_t s) {
+static SetTraits set_traits(const pyci_wfn *wfn, bool strict, hipStream_t s) {
     const int n = (int)wfn->nbasis;
-    if (wfn->ndet < 1) return {0, true};
+    if (wfn->ndet < 1) return {0, strict};
     DevBuf<int> lo(3);
     const int init[3] = {64, 0, 0};
     PE_HIP(hipMemcpyAsync(lo.p, init, sizeof(init), hipMemcpyHostToDevice, s));
-    k_low_range<<<(unsigned)std::min<i64>(1024, (wfn->ndet + 255) / 256), 256, 0, s>>>(
-        wfn->dets.p, wfn->ndet, (int)wfn->nkey, n / 2, (int)wfn->nup, (int)wfn->ndn, lo.p);
+    k_low_range<<<(unsigned)std::min<i64>(1024, (wfn->ndet + 255) / 256), 256, 0, s>>>(view_of(wfn), n / 2, strict,
+                                                                                     lo.p);
     PE_LAUNCH_CHECK();
     int h[3] = {0, 1, 1};
     PE_HIP(hipMemcpyAsync(h, lo.p, sizeof(h), hipMemcpyDeviceToHost, s));
     PE_HIP(hipStreamSynchronize(s));
     const bool half = wfn->kind == PYCI_WFN_GENCI && n >= 2 && n % 2 == 0 && h[0] == h[1];
-    return {half ? n / 2 : 0, h[2] == 0};
+    return {half ? n / 2 : 0, strict && h[2] == 0};
 }
 
 template <int KIND>
@@ -1100,26 +1105,34 @@ static void build_rows_pairs(pyci_op *op, const WfnView &w, const HamView &H, i6
 // determinants 1.25 / 0.18, 20,000 6.5 / 0.94, 60,000 20.4 / 3.0, 200,000 75 / 19.8, 500,000
 // 224 / 108, of one spin projection (16,500) 300,000 69 / 41; FullCI of 24 orbitals, 5 + 5
 // electrons (12,600) 17,317 3.5 / 0.83, 200,000 46 / 30, 400,000 107 / 106; of 14 orbitals,
-// 4 + 4 (2,220) 100,000 9.7 / 8.8: both sides meet near 30 columns per excitation. Needs
-// every determinant to have the wave function's electron counts (the test sees only which
-// orbitals differ) and a row's split to stay below 2^28 entries.
-static bool pairs_pay(int kind, const pyci_wfn *wfn, const SetTraits &t, i64 nr, i64 ncol) {
-    if (kind == PYCI_WFN_DOCI || wfn->colex || !t.occ || nr < 1 || ncol < 1 || ncol >= ((i64)1 << 28)) return false;
+// 4 + 4 (2,220) 100,000 9.7 / 8.8: both sides meet near 30 columns per excitation. A row's
+// split has to stay below 2^28 entries.
+static bool pairs_pay(int kind, const pyci_wfn *wfn, int szh, i64 nr, i64 ncol) {
+    if (kind == PYCI_WFN_DOCI || wfn->colex || nr < 1 || ncol < 1 || ncol >= ((i64)1 << 28)) return false;
     const i64 n = wfn->nbasis, nu = wfn->nup, vu = n - nu;
     const auto c2 = [](i64 x) { return x * (x - 1) / 2; };
     i64 exc = nu * vu + c2(nu) * c2(vu);
     if (kind == PYCI_WFN_FULLCI) {
         const i64 nd = wfn->ndn, vd = n - nd;
         exc += nu * vu * nd * vd + nd * vd + c2(nd) * c2(vd);
-    } else if (t.szh) {
+    } else if (szh) {
         exc = exc * 2 / 5;  // k_rows leaves out what changes the projection
     }
     return ncol < 28 * exc;
 }
 
+// The traits of a set, and whether its rows are built by testing pairs. The test sees only which
+// orbitals differ: a determinant of another electron count would pass it where no excitation
+// leads, and two places of the same one would meet as a pair without any difference. Sets
+// that hold such determinants, which no call refuses, are enumerated.
+static bool by_pairs(int kind, const pyci_wfn *wfn, i64 nr, i64 ncol, SetTraits &t) {
+    t = set_traits(wfn, pairs_pay(kind, wfn, 0, nr, ncol), wfn->ctx->stream);
+    return t.sound && pairs_pay(kind, wfn, t.szh, nr, ncol);
+}
+
 bool pairs_serve(const pyci_wfn *wfn) {
-    if (wfn->kind == PYCI_WFN_DOCI || wfn->colex || wfn->ndet < 1) return false;
-    return pairs_pay(wfn->kind, wfn, set_traits(wfn, wfn->ctx->stream), wfn->ndet, wfn->ndet);
+    SetTraits t;
+    return pairs_pay(wfn->kind, wfn, 0, wfn->ndet, wfn->ndet) && by_pairs(wfn->kind, wfn, wfn->ndet, wfn->ndet, t);
 }
 
 void build_rows(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn, i64 row0, i64 row1, i64 ncol,
@@ -1133,12 +1146,13 @@ void build_rows(pyci_op *op, const pyci_ham *ham, const pyci_wfn *wfn, i64 row0,
     if (build_rows_sorted(op, wfn, w, H, row0, row1, ncol, rowptr_seg, cols, vals, lowcnt_seg, diag_seg, nnz_seg,
                           low_total))
         return;
-    const SetTraits traits = op->kind == PYCI_WFN_DOCI ? SetTraits{0, true} : set_traits(wfn, s);
+    SetTraits traits{0, false};
+    const bool pairs = op->kind != PYCI_WFN_DOCI && by_pairs(op->kind, wfn, nr, ncol, traits);
     w.szh = traits.szh;
     rowptr_seg.alloc((size_t)(nr + 1));
     lowcnt_seg.alloc((size_t)(nr + 1));
     diag_seg.alloc((size_t)(nr > 0 ? nr : 1));
-    if (pairs_pay(op->kind, wfn, traits, nr, ncol)) {
+    if (pairs) {
         if (op->kind == PYCI_WFN_FULLCI)
             build_rows_pairs<PYCI_WFN_FULLCI>(op, w, H, row0, row1, ncol, rowptr_seg, cols, vals, lowcnt_seg, diag_seg,
                                               nnz_seg, low_total);

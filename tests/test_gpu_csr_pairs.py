@@ -1,6 +1,6 @@
 """CSR rows of selected sets built by testing pairs of determinants: bit for bit the
 oracle's, and those of the enumerating build, which a set with one determinant of another
-electron count takes."""
+electron count takes, and one that holds a determinant twice."""
 import numpy as np
 import numpy.testing as npt
 import pytest
@@ -60,3 +60,25 @@ def test_pair_rows_match_enumerated_rows(kind):
     b = pyci.sparse_op(ham, _wfn(kind, np.concatenate([dets, other])), 3000, 3000, symmetric=False)
     for x, y in ((a.indptr(), b.indptr()), (a.indices(), b.indices()), (a.data(), b.data())):
         npt.assert_array_equal(x, y)
+
+
+@pytest.mark.parametrize("kind", ["fullci", "genci"])
+def test_rows_of_a_set_with_a_determinant_twice(kind):
+    """The rows of a set whose last determinant is there twice: each of the two has its own
+    diagonal and none of the other, the rest find one of them."""
+    dets, one, two = _set(kind, 700)
+    ham = pyci.hamiltonian(0.0, one, two)
+    n = len(dets) - 1
+    rows = []
+    for d in (dets, np.concatenate([dets, dets[-1:]])):
+        data, indices, indptr = pyci.sparse_op(ham, _wfn(kind, d), symmetric=False).export()
+        rows.append([dict(zip(indices[a:b], data[a:b])) for a, b in zip(indptr, indptr[1:])])
+        assert [len(r) for r in rows[-1]] == np.diff(indptr).tolist()
+    once, twice = rows
+    for r in range(n):
+        expect = dict(once[r])
+        if n in expect and n not in twice[r]:
+            expect[n + 1] = expect.pop(n)
+        assert twice[r] == expect
+    last = {c: v for c, v in once[n].items() if c != n}
+    assert twice[n] == {**last, n: once[n][n]} and twice[n + 1] == {**last, n + 1: once[n][n]}

@@ -44,3 +44,26 @@ def test_pair_rdms_match_enumerated_ones(kind):
     b = pyci.compute_rdms(_wfn(kind, np.concatenate([dets, other])), c)
     for x, y in zip(a, b):
         npt.assert_array_equal(np.isnan(x), np.isnan(y))
+
+
+@pytest.mark.parametrize("kind", ["fullci", "genci"])
+def test_rdms_of_a_set_with_a_determinant_twice(kind):
+    """The same elements as by enumeration of the set (which one more determinant, of another
+    electron count and without weight, takes as well)."""
+    dets, _, _ = _set(kind, 700)
+    dets = np.concatenate([dets, dets[-1:]])
+    c = np.random.default_rng(2).normal(size=len(dets) + 1)
+    c[-2], c[-1] = c[-3], 0.0
+    c /= np.linalg.norm(c)
+    other = dets[:1].copy()
+    other[0, 0] |= ~other[0, 0] & (other[0, 0] + np.uint64(1))
+    a = pyci.compute_rdms(_wfn(kind, dets), c[:-1])
+    b = pyci.compute_rdms(_wfn(kind, np.concatenate([dets, other])), c)
+    once = pyci.compute_rdms(_wfn(kind, dets[:-1]), c[:-2])
+    for x, y in zip(a, b):
+        npt.assert_allclose(x, y, rtol=0, atol=2 * EPS * 700)
+    # its diagonal elements count twice
+    d1 = a[0][0] if kind == "fullci" else a[0]
+    o1 = once[0][0] if kind == "fullci" else once[0]
+    occ = np.array([int(dets[-1, 0]) >> p & 1 for p in range(SPACE[kind][0])])
+    npt.assert_allclose(np.diag(d1), np.diag(o1) + c[-2] ** 2 * occ, rtol=0, atol=2 * EPS * 700)
