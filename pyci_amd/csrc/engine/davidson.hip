@@ -1340,17 +1340,21 @@ struct Davidson {
     // Thick restart on the lowest kk Ritz vectors: they are orthonormal and G
     // becomes diag(w).
     void restart(int kk, const std::vector<double> &w, const std::vector<double> &y) {
-        RV.ensure((size_t)(nd * 2 * k));
-        RW.ensure((size_t)(nd * 2 * k));
+        // X and WX hold k columns; only a restart on more needs memory of its own
+        if (kk > k) {
+            RV.ensure((size_t)(nd * 2 * k));
+            RW.ensure((size_t)(nd * 2 * k));
+        }
+        double *rv = kk > k ? RV.p : X.p, *rw = kk > k ? RW.p : WX.p;
         for (int j = 0; j < kk; ++j)
             for (int i = 0; i < m; ++i) hb.p[oYK + (size_t)j * m + i] = y[(size_t)i * m + j];
         PE_HIP(hipMemcpyAsync(dv.p + oYK, hb.p + oYK, sizeof(double) * (size_t)m * kk, hipMemcpyHostToDevice, s));
-        k_gemm_set<<<g1(), 256, 0, s>>>(nd, V.p, nd, m, dv.p + oYK, kk, RV.p, nd);
+        k_gemm_set<<<g1(), 256, 0, s>>>(nd, V.p, nd, m, dv.p + oYK, kk, rv, nd);
         PE_LAUNCH_CHECK();
-        k_gemm_set<<<g1(), 256, 0, s>>>(nd, W.p, nd, m, dv.p + oYK, kk, RW.p, nd);
+        k_gemm_set<<<g1(), 256, 0, s>>>(nd, W.p, nd, m, dv.p + oYK, kk, rw, nd);
         PE_LAUNCH_CHECK();
-        put_basis(RV.p, kk);
-        PE_HIP(hipMemcpyAsync(W.p, RW.p, sizeof(double) * nd * kk, hipMemcpyDeviceToDevice, s));
+        put_basis(rv, kk);
+        PE_HIP(hipMemcpyAsync(W.p, rw, sizeof(double) * nd * kk, hipMemcpyDeviceToDevice, s));
         std::fill(G.begin(), G.end(), 0.0);
         for (int j = 0; j < kk; ++j) G[(size_t)j * mmax + j] = w[(size_t)j];
         m = kk;

@@ -357,18 +357,23 @@ int rf_copies(const RfShape &S) {
 
 // Expands the accumulators and brings the result to the caller: straight into page-locked memory
 // of the context (one synchronisation and no staged copies); beyond 16 MB (FullCI nbasis
-// 29, GenCI 38) through device memory.
+// 29, GenCI 38), or where there is none to be had, through device memory.
 void rf_result(pyci_ctx *ctx, const RfShape &S, int R, const double *acc, double *rdm1, double *rdm2) {
     hipStream_t s = ctx->stream;
     const i64 n2 = (i64)S.n * S.n, s1 = (S.genci ? 1 : 2) * n2, nout = s1 + (S.genci ? 1 : 3) * n2 * n2;
-    const bool direct = nout <= (i64)2 << 20;
+    bool direct = nout <= (i64)2 << 20;
     DevBuf<double> dout;
     Lease<HostBuf<double>> out(ctx->rdm_out);
     HostBuf<double> &host = out.buf;
-    if (direct)
-        host.ensure((size_t)nout);
-    else
-        dout.alloc((size_t)nout);
+    if (direct) {
+        try {
+            host.ensure((size_t)nout);
+        } catch (const EngineError &) {
+            (void)hipGetLastError();
+            direct = false;
+        }
+    }
+    if (!direct) dout.alloc((size_t)nout);
     k_rf_expand<<<grid_for(nout, 256), 256, 0, s>>>(S, R, acc, direct ? host.p : dout.p);
     PE_LAUNCH_CHECK();
     if (direct) {
@@ -406,7 +411,8 @@ static bool full_rdm_applies(const pyci_wfn *w) {
     return na <= 8000 && nb <= 8000;
 }
 
-// compute_rdms of a full FullCI space; false where it does not apply. A vector with
+// compute_rdms of a full FullCI space; false where it does not apply or its scratch memory (three
+// copies of the vector and the string matrices) is not to be had. A vector with
 // infinities or NaNs is left to the scatter kernel as well: in a contraction they would
 // reach elements that no connected pair of determinants carries them to.
 bool rdms_full_space(pyci_wfn *w, const double *coeffs_host, double *rdm1, double *rdm2) {
@@ -425,7 +431,14 @@ bool rdms_full_space(pyci_wfn *w, const double *coeffs_host, double *rdm1, doubl
     const i64 ntab = ((i64)trows * S.ldc + 3) / 4;
     // one allocation: the vector, C and C^T, gamma of both spins, the table, the accumulators
     const i64 nacc = R * S.stride, even = (w->ndet + 1) & ~(i64)1;
-    DevBuf<double> buf((size_t)(even + nC + nCt + nga + ngb + ntab + nacc));
+    DevBuf<double> buf;
+    try {
+        buf.alloc((size_t)(even + nC + nCt + nga + ngb + ntab + nacc));
+    } catch (const EngineError &e) {
+        if (e.code != PYCI_ENOMEM) throw;
+        (void)hipGetLastError();  // not to be reported against a later launch
+        return false;             // the scatter kernel needs the vector and its accumulators only
+    }
     double *c = buf.p, *C = c + even, *Ct = C + nC, *ga = Ct + nCt, *gb = ga + nga;
     double *acc = gb + ngb;
     uint16_t *tab = reinterpret_cast<uint16_t *>(acc + nacc);

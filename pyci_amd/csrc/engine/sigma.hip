@@ -394,10 +394,17 @@ void spmv_plan(pyci_op *op, bool column_ordered_space) {
     allow_lds<64, double>();
     allow_lds<16, float>();
     allow_lds<64, float>();
+    try {
+        P.bounds.alloc((size_t)(cus + 1));
+        P.split.alloc((size_t)(nrow * (npanel - 1)));  // up to 1 % of the entries' bytes
+    } catch (const EngineError &e) {
+        if (e.code != PYCI_ENOMEM) throw;
+        (void)hipGetLastError();
+        P = SpmvPlan();  // the product without panels serves any operator
+        return;
+    }
     P.npanel = (int)npanel;
     P.nblk = cus;
-    P.bounds.alloc((size_t)(cus + 1));
-    P.split.alloc((size_t)(nrow * (npanel - 1)));
     k_spmv_bounds<<<grid_for(cus + 1, 64), 64, 0, s>>>(nrow, op->nnz, cus, op->rowptr.p, P.bounds.p);
     PE_LAUNCH_CHECK();
     if (npanel > 1) {
