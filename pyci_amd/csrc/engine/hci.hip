@@ -107,7 +107,8 @@ __device__ inline u64 set_insert(const NewSet &S, u64 key, int &claims) {
 // single-excitation element: |h_ia| + sum over all q of
 // |two_mo[i][q][a][q] - two_mo[i][q][q][a]| (FullCI: + |two_mo[i][q][a][q]|). A row then
 // visits, per occupied pair, only the list prefix above eps / |c_i|, and computes a single's
-// element only where the bound reaches it, instead of evaluating every excitation.
+// element only where the bound reaches it, instead of evaluating every excitation. FullCI sets
+// too small to pay for the lists (lists_pay) go without them (v = nullptr).
 struct HbLists {
     const double *v = nullptr;         // [P][npair]
     const double *vo = nullptr;        // [p * n + q][n * n] (FullCI)
@@ -115,7 +116,6 @@ struct HbLists {
     const double *top = nullptr, *topo = nullptr;  // |V| of each list's first entry
     const double *most = nullptr;      // the largest of sb, top and topo
     const unsigned short *rs = nullptr, *rso = nullptr;  // r | s << 8 of each entry
-    int npair = 0;
 };
 constexpr int HB_CAP = 2048;      // n (n - 1) / 2 <= 2016 for n <= 64
 constexpr int HB_CAP_OPP = 4096;  // n n
@@ -225,7 +225,8 @@ __global__ void __launch_bounds__(256) k_hb_most(const double *v, int n, double 
 constexpr int HCI_WAVES = 4;
 constexpr i64 HCI_BLOCKS = (i64)1 << 20;
 
-template <int KIND, int PASS>
+// LISTS: there are lists (DOCI has none).
+template <int KIND, int PASS, bool LISTS>
 __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, const double *coeffs, double eps, double eps_plain,
                                              i64 rows_stride, NewSet S, unsigned long long *count, HbLists L) {
     __shared__ unsigned long long sums[HCI_WAVES];
@@ -242,7 +243,7 @@ __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, co
         const double cabs = fabs(coeffs[row]);
         const double eps_i = eps / cabs, eps_plain_i = eps_plain / cabs;
         // a row of the tail, whose threshold no element reaches
-        if (KIND != PYCI_WFN_DOCI && *L.most * (1.0 + 1e-12) <= eps_i) continue;  // uniform per block
+        if (LISTS && *L.most * (1.0 + 1e-12) <= eps_i) continue;  // uniform per block
         // lane q holds the q-th occupied / virtual orbital of each string
         auto nth = [](u64 x, int t) {
             for (int s = 0; s < t && x; ++s) x &= x - 1;
@@ -309,15 +310,37 @@ __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, co
             // index of orbital r among the empty orbitals of string d
             auto hole = [](u64 d, int r) { return r - __popcll(d & ((1ULL << r) - 1ULL)); };
             int turn = 0;  // lists seen: the waves take them in turn
-            // the entries of a list above the threshold, in chunks of 64 lanes
-            auto walk = [&](const double *lv, const unsigned short *lrs, int len, auto &&take) {
+            // the pairs (r, s) of p and q whose element is above the threshold, in chunks of 64
+            // lanes: the beginning of their list, or all elements where there are no lists
+            auto walk = [&](auto same, int p, int q, auto &&take) {
+                constexpr bool SAME = decltype(same)::value;
+                const int len = SAME ? n * (n - 1) / 2 : n * n;
+                const i64 at = (SAME ? (i64)(q * (q - 1) / 2 + p) : (i64)(p * n + q)) * len;
                 for (int t0 = 0; t0 < len; t0 += 64) {
                     const int t = t0 + lane;
-                    const double V = t < len ? lv[t] : 0.0;
+                    int r = 0, s2 = 0;
+                    double V = 0.0;
+                    if (LISTS) {
+                        if (t < len) V = (SAME ? L.v : L.vo)[at + t];
+                    } else if (t < len) {
+                        if (SAME) {
+                            tri_decode(t, r, s2);
+                            V = two[GIX(p, q, r, s2)] - two[GIX(p, q, s2, r)];
+                        } else {
+                            r = t / n, s2 = t - r * n;
+                            V = two[at + t];
+                        }
+                    }
                     const bool above = t < len && fabs(V) > eps_i;
-                    if (__ballot(above) == 0) break;  // the list is sorted: nothing further passes
-                    const unsigned rs = above ? lrs[t] : 0u;
-                    take(above, V, (int)(rs & 255u), (int)(rs >> 8));
+                    if (__ballot(above) == 0) {
+                        if (LISTS) break;  // sorted: nothing further passes
+                        continue;
+                    }
+                    if (LISTS) {
+                        const unsigned rs = above ? (SAME ? L.rs : L.rso)[at + t] : 0u;
+                        r = (int)(rs & 255u), s2 = (int)(rs >> 8);
+                    }
+                    take(above, V, r, s2);
                 }
             };
             // singles and same-spin doubles of one spin
@@ -332,7 +355,7 @@ __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, co
                     const bool in = e < no * nv;
                     const int ec = in ? e : 0, i = ec / nv, j = ec - i * nv;
                     const int ii = (__shfl(packed, i) >> so) & 255, jj = (__shfl(packed, j) >> (so + 8)) & 255;
-                    const bool live = in && !(L.sb[ii * n + jj] * (1.0 + 1e-12) <= eps_i);
+                    const bool live = in && !(LISTS && L.sb[ii * n + jj] * (1.0 + 1e-12) <= eps_i);
                     double val = 0.0;
                     int sg = 1;
                     if (live) {
@@ -364,14 +387,13 @@ __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, co
                     int i = 0, k = 0;
                     if (p0 + lane < np) tri_decode(p0 + lane, i, k);
                     const int ii0 = (__shfl(packed, i) >> so) & 255, kk0 = (__shfl(packed, k) >> so) & 255;
-                    u64 todo = __ballot(p0 + lane < np && L.top[kk0 * (kk0 - 1) / 2 + ii0] > eps_i);
+                    u64 todo = __ballot(p0 + lane < np && !(LISTS && !(L.top[kk0 * (kk0 - 1) / 2 + ii0] > eps_i)));
                     for (; todo; todo &= todo - 1) {
                         if (turn++ % HCI_WAVES != wave) continue;
                         const int from = __builtin_ctzll(todo);
                         const int pi = __shfl(i, from), pk = __shfl(k, from);
                         const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
-                        const i64 lb = (i64)(kk * (kk - 1) / 2 + ii) * L.npair;
-                        walk(L.v + lb, L.rs + lb, L.npair, [&](bool above, double V, int r, int s2) {
+                        walk(std::true_type{}, ii, kk, [&](bool above, double V, int r, int s2) {
                             const bool free = above && !((d >> r) & 1ULL) && !((d >> s2) & 1ULL);
                             const int j = hole(d, r), l = hole(d, s2);
                             int sg = 1;
@@ -389,14 +411,13 @@ __global__ void __launch_bounds__(HCI_WAVES * 64) k_hci(WfnView w, HamView H, co
                 for (int p0 = 0; p0 < nou * nod; p0 += 64) {
                     const int e = p0 + lane < nou * nod ? p0 + lane : 0, i = e / nod, k = e - i * nod;
                     const int ii0 = __shfl(packed, i) & 255, kk0 = (__shfl(packed, k) >> 16) & 255;
-                    u64 todo = __ballot(p0 + lane < nou * nod && L.topo[ii0 * n + kk0] > eps_i);
+                    u64 todo = __ballot(p0 + lane < nou * nod && !(LISTS && !(L.topo[ii0 * n + kk0] > eps_i)));
                     for (; todo; todo &= todo - 1) {
                         if (turn++ % HCI_WAVES != wave) continue;
                         const int from = __builtin_ctzll(todo);
                         const int pi = __shfl(i, from), pk = __shfl(k, from);
                         const int ii = __shfl(ii0, from), kk = __shfl(kk0, from);
-                        const i64 lb = (i64)(ii * n + kk) * n * n;
-                        walk(L.vo + lb, L.rso + lb, n * n, [&](bool above, double V, int r, int s2) {
+                        walk(std::false_type{}, ii, kk, [&](bool above, double V, int r, int s2) {
                             const bool free = above && !((up >> r) & 1ULL) && !((dn >> s2) & 1ULL);
                             int sg = 1;
                             if (PASS == 5 && free) sg = phase1(up, ii, r) * phase1(dn, kk, s2);
@@ -434,6 +455,20 @@ __global__ void k_set_clear(u64 *slot, u64 second, u64 *score, int *plain, i64 n
     }
 }
 
+// Whether a FullCI set is large enough for sorting the lists, which takes 1.1 ms at 64 orbitals
+// and hardly less than 40 us at any size: the elements that a pass over the set would look at
+// without them against those of the lists. ENPT2 without / with lists, us: 64 orbitals, 1 + 1
+// electrons, one determinant 51 / 1,170, 882 determinants 434 / 1,670; 2 + 2 electrons, 500
+// determinants 1,010 / 2,010 (walk : sort 0.5); 5 + 5 electrons, 100 determinants (0.7) 4,970 / 3,560;
+// 48 orbitals, 5 + 5 electrons, 50 determinants (0.6) 2,500 / 1,870; 12 orbitals, 6 + 6 electrons, 100
+// determinants 266 / 284 (700,000 elements); 24 orbitals, 5 + 5 electrons, 300 determinants 760 / 666,
+// 3,000 determinants 1,070 / 710.
+static bool lists_pay(const WfnView &w) {
+    const double n2 = (double)w.nb * w.nb, np = (n2 - w.nb) / 2, nu = w.nup, nd = w.ndn;
+    const double walk = (double)w.ndet * (nu * nd * n2 + (nu * (nu - 1) + nd * (nd - 1)) / 2 * np);
+    return walk > 1 << 20 && 2 * walk > n2 * n2 + np * np;
+}
+
 // The heat-bath lists of a selection (HbLists), built for one call.
 struct HbTables {
     DevBuf<double> v;
@@ -459,7 +494,7 @@ struct HbTables {
         PE_LAUNCH_CHECK();
         k_hb_most<<<1, 256, 0, s>>>(sb, (int)(n2 + npair + nto), most);
         PE_LAUNCH_CHECK();
-        L = HbLists{v.p, vo, sb, top, topo, most, rs.p, rs.p + np2, npair};
+        L = HbLists{v.p, vo, sb, top, topo, most, rs.p, rs.p + np2};
     }
 };
 
@@ -468,11 +503,13 @@ static void launch_hci(int kind, const WfnView &w, const HamView &H, const doubl
                        i64 stride, const NewSet &S, unsigned long long *count, hipStream_t s, const HbLists &L) {
     const unsigned g = (unsigned)std::min(w.ndet, HCI_BLOCKS), t = HCI_WAVES * 64;
     if (kind == PYCI_WFN_DOCI)
-        k_hci<PYCI_WFN_DOCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+        k_hci<PYCI_WFN_DOCI, PASS, false><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+    else if (kind == PYCI_WFN_FULLCI && L.v)
+        k_hci<PYCI_WFN_FULLCI, PASS, true><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     else if (kind == PYCI_WFN_FULLCI)
-        k_hci<PYCI_WFN_FULLCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+        k_hci<PYCI_WFN_FULLCI, PASS, false><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     else
-        k_hci<PYCI_WFN_GENCI, PASS><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
+        k_hci<PYCI_WFN_GENCI, PASS, true><<<g, t, 0, s>>>(w, H, c, eps, eps_plain, stride, S, count, L);
     PE_LAUNCH_CHECK();
 }
 
@@ -579,7 +616,8 @@ static void hci_collect(pyci_ham *ham, pyci_wfn *wfn, const double *dc, double e
     PE_HIP(hipMemsetAsync(R.cnt.p, 0, sizeof(unsigned long long) * 2, s));
     R.S = NewSet{nullptr, 0, R.cnt.p + 1, R.ovf.p};
     HbTables hb;
-    if (wfn->kind != PYCI_WFN_DOCI) hb.build(H, wfn->kind == PYCI_WFN_FULLCI, s);
+    if (wfn->kind == PYCI_WFN_GENCI || (wfn->kind == PYCI_WFN_FULLCI && lists_pay(w)))
+        hb.build(H, wfn->kind == PYCI_WFN_FULLCI, s);
     launch_hci<1>(wfn->kind, w, H, dc, eps, eps_plain, R.stride, R.S, R.cnt.p, s, hb.L);
     unsigned long long upper = 0;
     PE_HIP(hipMemcpyAsync(&upper, R.cnt.p, sizeof(upper), hipMemcpyDeviceToHost, s));
@@ -840,7 +878,7 @@ double enpt2_device(pyci_ham *ham, pyci_wfn *wfn_in, const double *coeffs_host, 
     NewSet S{nullptr, 0, cnt.p + 1, ovf.p};
     // pass 1: passing external candidates (with repeats) bound the set size
     HbTables hb;
-    hb.build(H, wfn->kind == PYCI_WFN_FULLCI, s);
+    if (wfn->kind == PYCI_WFN_GENCI || lists_pay(w)) hb.build(H, wfn->kind == PYCI_WFN_FULLCI, s);
     launch_hci<1>(wfn->kind, w, H, dc.p, eps, eps, 0, S, cnt.p, s, hb.L);
     unsigned long long upper = 0;
     PE_HIP(hipMemcpyAsync(&upper, cnt.p, sizeof(upper), hipMemcpyDeviceToHost, s));

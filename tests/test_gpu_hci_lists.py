@@ -12,20 +12,15 @@ from pyci_amd.synthetic import seeded_integrals, spin_orbital
 pytestmark = pytest.mark.gpu
 
 
-# no electrons or no holes of a spin, no same-spin pairs, the longest strings that are
-# their own key and the first that are ranked, a list of 2,048 and the longest lists, the
-# sizes around which the terms' tables need more than 64 KB of LDS
-@pytest.mark.parametrize("nb,nu,nd", [(7, 3, 0), (6, 6, 3), (20, 1, 1), (32, 2, 2), (33, 2, 1), (46, 2, 1),
-                                      (58, 1, 1), (59, 1, 1), (60, 1, 1), (61, 1, 1), (64, 1, 1)])
-def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
+def _check(oracle, nb, nu, nd, count, eps_all):
     rng = np.random.default_rng(nb)
     one = rng.normal(size=(nb, nb))
     two = rng.normal(size=(nb,) * 4) * 10.0 ** rng.uniform(-4, 0, size=(nb,) * 4)  # no symmetry assumed
-    strings = [[sum(1 << int(p) for p in rng.permutation(nb)[:k]) for _ in range(25)] for k in (nu, nd)]
+    strings = [[sum(1 << int(p) for p in rng.permutation(nb)[:k]) for _ in range(count)] for k in (nu, nd)]
     dets = np.unique(np.array(strings, dtype=np.uint64).T, axis=0)
     c = rng.normal(size=len(dets)) * 10.0 ** rng.uniform(-3, 0, size=len(dets))
     ham = pyci.hamiltonian(0.0, one, two)
-    for eps in (0.0, 3e-3, 0.3, 1e9):
+    for eps in eps_all:
         w = pyci.fullci_wfn(nb, nu, nd, dets.reshape(-1, 2, 1))
         expect = oracle.add_hci("fullci", nb, nu, nd, dets, one, two, c, eps).reshape(-1, 2)
         e = pyci.compute_enpt2(ham, w, c, -1e3, eps=eps)
@@ -33,6 +28,27 @@ def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
         npt.assert_allclose(e, ref, rtol=1e-11)
         assert pyci.add_hci(ham, w, c, eps=eps) == len(expect)
         npt.assert_array_equal(w.to_det_array().reshape(-1, 2)[len(dets):], expect)
+    return len(dets)
+
+
+# no electrons or no holes of a spin, no same-spin pairs, the longest strings that are
+# their own key and the first that are ranked, a list of 2,048 and the longest lists, the
+# sizes around which the terms' tables need more than 64 KB of LDS
+@pytest.mark.parametrize("nb,nu,nd", [(7, 3, 0), (6, 6, 3), (20, 1, 1), (32, 2, 2), (33, 2, 1), (46, 2, 1),
+                                      (58, 1, 1), (59, 1, 1), (60, 1, 1), (61, 1, 1), (64, 1, 1)])
+def test_fullci_lists_match_oracle(oracle, nb, nu, nd):
+    _check(oracle, nb, nu, nd, 25, (0.0, 3e-3, 0.3, 1e9))
+
+
+# sets large enough for sorted lists: both key forms, lists of one and two chunks, of 2,048 and
+# the longest; the last set of a size that goes without and the first that sorts
+@pytest.mark.parametrize("nb,nu,nd,count", [(9, 4, 3, 3000), (12, 6, 6, 300), (32, 2, 2, 400), (33, 2, 1, 600),
+                                            (46, 2, 1, 700), (64, 1, 1, 5000), (16, 8, 8, 45), (16, 8, 8, 46)])
+def test_sorted_lists_match_oracle(oracle, nb, nu, nd, count):
+    ndet = _check(oracle, nb, nu, nd, count, (3e-3, 0.3, 1e9))
+    n2, pairs = nb * nb, nb * (nb - 1) // 2
+    walk = ndet * (nu * nd * n2 + (nu * (nu - 1) + nd * (nd - 1)) // 2 * pairs)
+    assert (walk > 1 << 20 and 2 * walk > n2 * n2 + pairs * pairs) == (count != 45)
 
 
 @pytest.mark.parametrize("kind,nb,nu,nd", [("fullci", 8, 3, 2), ("genci", 12, 4, 0)])
