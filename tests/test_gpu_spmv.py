@@ -43,6 +43,7 @@ def test_lds_panels(kind, nb, nu, nd, ndet):
     dets = dets[np.sort(at)[:ndet]]
     op = pyci.sparse_op(pyci.hamiltonian(0.0, one, two), cls(nb, nu, nd, dets))
     assert op.size > 1 << 19
+    assert 2 * op.size - ndet > 32 * ndet * -(-ndet // 20000)  # dense enough for panels
     _check(op, True)
 
 
@@ -101,3 +102,24 @@ def test_non_finite_elements_stay_in_their_rows(kind, nb, nu, nd, ndet):
             npt.assert_array_equal(np.isnan(y), np.isnan(expect))
             npt.assert_array_equal(np.isinf(y), np.isinf(expect))
             assert np.isfinite(y).sum() > 0
+
+
+@pytest.mark.parametrize("symmetric", [True, False])
+def test_panels_after_an_update(symmetric):
+    """Products after update: rows and columns appended past a panel, and a small operator
+    that grows into panels."""
+    _, one, two = seeded_integrals(18, 4, 64)
+    ham = pyci.hamiltonian(0.0, one, two)
+    full = pyci.fullci_wfn(18, 3, 3)
+    full.add_all_dets()
+    dets = full.to_det_array()[np.random.default_rng(3).permutation(len(full))[:61000]]
+    for sizes in ((39000, 41000, 61000), (900, 30000)):
+        w = pyci.fullci_wfn(18, 3, 3, dets[:sizes[0]])
+        op = pyci.sparse_op(ham, w, symmetric=symmetric)
+        _check(op, symmetric)
+        for a, b in zip(sizes, sizes[1:]):
+            more = pyci.fullci_wfn(18, 3, 3, dets[a:b])
+            w.add_dets_from_wfn(more)
+            op.update(ham, w)
+            assert op.shape == (b, b)
+            _check(op, symmetric)
