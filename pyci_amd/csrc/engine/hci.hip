@@ -82,7 +82,11 @@ __device__ inline void key_det(const WfnView &w, u64 key, u64 &a, u64 &b) {
     }
 }
 
-// Finds or claims the slot of key (counted in claims); returns it, or ~0 on overflow.
+// Finds or claims the slot of key (counted in claims); returns it, or ~0 on overflow. A table
+// that has become too small is found out by the first lane that walks it to its end or, long
+// before, by one that meets 4,096 other keys (at the intended load of 2/3 chains have some
+// hundreds at most); the others see the flag and leave it too, so that a pass over a
+// full table ends.
 __device__ inline u64 set_insert(const NewSet &S, u64 key, int &claims) {
     u64 h = __umul64hi(mix64(key), S.cap);
     for (u64 step = 0; step < S.cap; ++step) {
@@ -91,6 +95,9 @@ __device__ inline u64 set_insert(const NewSet &S, u64 key, int &claims) {
         if (old == EMPTY_KEY) ++claims;
         if (old == EMPTY_KEY || old == key) return h;
         h = h + 1 < S.cap ? h + 1 : 0;
+        if ((step & 63) == 63 &&
+            (step >= 4095 || __hip_atomic_load(S.overflow, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)))
+            break;
     }
     atomicOr(S.overflow, 1);
     return ~0ULL;
