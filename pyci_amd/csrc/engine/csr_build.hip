@@ -1099,7 +1099,7 @@ static void build_rows_pairs(pyci_op *op, const WfnView &w, const HamView &H, i6
 }
 
 // Whether testing pairs is the shorter way to the rows of a hashed set: its time grows
-// with the columns (0.35 ps a pair in both passes together), that of k_rows with a row's
+// with the columns (0.35-0.6 ps a pair in both passes together), that of k_rows with a row's
 // excitations (5 ps each, and its rows are sorted afterwards). Builds by excitations / by
 // pairs, ms: GenCI of 48 spin orbitals and 12 electrons (42,012 excitations) 500
 // determinants 1.25 / 0.18, 20,000 6.5 / 0.94, 60,000 20.4 / 3.0, 200,000 75 / 19.8, 500,000

@@ -680,7 +680,7 @@ __global__ void __launch_bounds__(256) k_rdm_diagonal(WfnView w, RfShape S, cons
     }
 }
 
-// Sums of up to 62 FullCI orbitals fit the 64 KB of k_rdm_diagonal.
+// FullCI up to 60 orbitals: the sums of k_rdm_diagonal take 58 KB of the 64 KB of LDS there.
 static bool rdms_pairs(pyci_wfn *wfn, const double *coeffs_host, double *rdm1, double *rdm2) {
     if (wfn->kind == PYCI_WFN_DOCI || (wfn->kind == PYCI_WFN_FULLCI && wfn->nbasis > 60) || !pairs_serve(wfn))
         return false;

@@ -125,7 +125,7 @@ k_spmm(i64 nrow, i64 nblocks, const i64 *__restrict__ rowptr, const int32_t *__r
 //   WAVES 16, U 1   rows of a full space, sorted in column order: 16 neighbouring rows (most
 //                   with the same alpha string) walk the same lines of X in step, so L1 serves
 //                   them; a wider window per lane spreads the waves over more lines than L1
-//                   holds. nbasis 12 (18.6 GB): 4.11 ms (4.5 TB/s) against 5.18-6.4 with U
+//                   holds. nbasis 12 (18.6 GB): 3.99 ms (4.7 TB/s) against 5.18-6.4 with U
 //                   2..16 and 4 waves; nbasis 10: 147 us against 156-200. And sets of short
 //                   rows, two chunks at most (400,000 FullCI determinants of 32 entries a row
 //                   114 us, 172 with 4 waves and U 3; DOCI of 74,613 rows of 97 33 us, 40).
